@@ -906,14 +906,69 @@ __device__ __forceinline__ void mfmaHalf(const float4 *aSrc, const float4 *bSrc,
   }
 }
 
+// ---- fp32 products on the bf16 matrix pipe ------------------------------------------------------
+// A float is the exact sum of three bf16 values h + m + l (8 significant bits each, every remainder exact), and the
+// product of two bf16 values is exact in fp32. x * w is computed as the six products hh + hm + mh + mm + hl + lh; the
+// three left out (ml, lm, ll) are below 2^-26 of x * w, a quarter of what rounding the product to fp32 would cost. The
+// large products (hh) and the five small ones are summed in accumulators of their own, so a k-step of 16 rounds the
+// large sum once where the fp32 instruction rounds it 16 times: against a 64-bit sum the error over K = 128 / 2304 /
+// 8192 normally distributed terms is 6.4e-8 / 2.9e-7 / 5.8e-7 of the result's norm, with v_mfma_f32_32x32x2_f32
+// 2.0e-7 / 8.6e-7 / 1.6e-6 (one-signed, badly scaled and 1e-30-sized terms: the same ratio or better).
+// The matrix pipe runs bf16 at 16 times its fp32 rate, so six products cost 6/16 of the fp32 instruction's time
+// (measured on registers alone: 300 TFLOP/s of fp32 products, held back by power, against 138 - 150).
+// An operand that is not finite (or rounds up to infinity as bf16) makes the result NaN or infinite; the kernels then
+// compute that block again with the fp32 instruction, so infinities, NaNs and overflows come out as they did.
+// (Splitting a float into bf16 parts: Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial intelligence
+// datatype for higher-precision computations", ARITH 2019.)
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// two neighbouring k -> the packed pairs of their three parts
+__device__ __forceinline__ void splitPair(unsigned x0, unsigned x1, unsigned &h, unsigned &m, unsigned &l) {
+  f32x2 r = {__uint_as_float(x0), __uint_as_float(x1)};
+  h = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+  r = f32x2{r.x - __uint_as_float(h << 16), r.y - __uint_as_float(h & 0xffff0000u)};
+  m = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+  r = f32x2{r.x - __uint_as_float(m << 16), r.y - __uint_as_float(m & 0xffff0000u)};
+  l = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+}
+
+__device__ __forceinline__ bf16x8 asBf16(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
+
+// One k-step of 16 of one wave: TI x 2 blocks of 32 x 32. a[s][i], b[s][j]: part s (h, m, l) of the lane's 8
+// consecutive k (k-group lane / 32) of row / column lane % 32 of a block.
+template <int TI>
+__device__ __forceinline__ void mfmaSplit(const u32x4 (&a)[3][TI], const u32x4 (&b)[3][2], float16v (&hi)[TI][2],
+                                          float16v (&lo)[TI][2]) {
+  auto all = [&](int sa, int sb, float16v (&acc)[TI][2]) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(asBf16(a[sa][i]), asBf16(b[sb][j]), acc[i][j], 0, 0, 0);
+  };
+  all(0, 0, hi);
+  all(0, 1, lo);
+  all(1, 0, lo);
+  all(1, 1, lo);
+  all(0, 2, lo);
+  all(2, 0, lo);
+}
+
 // Forward kernel for images that carry their zero border in memory (padH = padW = 0 in g,
-// K % BK == 0, 16-byte loadable weight rows). On this part every ordinary vector-ALU
-// instruction takes issue time away from the MFMA pipe, so the main loop has none:
+// K % BK == 0, 16-byte loadable weight rows), on split operands (see above). Tiles come from memory as fp32 and are
+// split by the lane that fetched them, on the way into LDS:
 //  * a lane's output position is a fixed byte offset in a VGPR, the tap (c, kh, kw) of each k
 //    is a byte offset read from a table with scalar loads and handed to the buffer load as its
 //    scalar offset; every tap of every position is inside the padded image - no bounds test
 //  * weight rows are addressed as fixed VGPR offset + scalar k offset
 //  * the loop is unrolled over the two LDS buffers, so every LDS address is base + immediate
+//  * a k-step of a wave is 24 matrix instructions of 32 cycles, 88 vector-ALU instructions that split the next
+//    tile (they fit between the matrix instructions: leaving them out gains 5 %), 12 LDS reads and 6 LDS writes
+// What bounds it: two workgroups per CU (128 accumulator registers per lane) keep the matrix pipe 55 % busy at a
+// clock that power has pulled down to 2.05 GHz. 256 -> 256 planes 3x3 at 28 x 28, N = 64 (59.2 GFLOP):
+// 430 us with v_mfma_f32_32x32x2_f32, 307 us (193 TFLOP/s) on the parts.
 // Rows past M and columns past the batch are clamped to valid ones and dropped in the epilogue.
 // WM = 2: 128 x 128 tiles, the four waves as 2 x 2; WM = 1: 64 x 256 tiles, the four waves side by side,
 // for row counts whose last 128-row tile would be at most half full; a wave multiplies 64 x 64 either way.
@@ -927,10 +982,10 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   constexpr int TBM = WM == 0 ? 32 : 64 * WM, TBN = WM == 2 ? 128 : 256;
   constexpr int TI = WM == 0 ? 1 : 2;         // 32-row blocks of a wave
   constexpr int NA = WM == 2 ? 2 : 1;         // 16-byte groups of weights a lane loads per k-tile
-  constexpr int AP = TBM + 8, BP = TBN + 8;  // float4 per k-group row
+  constexpr int AP = TBM + 8, BP = TBN + 8;   // 16-byte groups (8 k of one part) per k-group row
   constexpr int NB = WM == 2 ? 8 : 16;        // image elements a lane gathers per k-tile
-  __shared__ float4 As[2][BK / 4][AP];
-  __shared__ float4 Bs[2][BK / 4][BP];
+  __shared__ u32x4 As[2][3][2][AP];           // [buffer][part][k-group of 8][row]
+  __shared__ u32x4 Bs[2][3][2][BP];
   __shared__ __attribute__((aligned(16))) float biasS[TBM];  // the tile's bias values: the epilogue reads them from here
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = WM == 2 ? wave >> 1 : 0, wn = WM == 2 ? wave & 1 : wave;
@@ -939,26 +994,23 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   const int m0 = mTile * TBM, j0 = nTile * TBN;
   if (t < TBM) biasS[t] = p.bias && m0 + t < p.M ? p.bias[m0 + t] : 0.f;  // visible after the first barrier
 
-  float16v acc[TI][2];
-
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void *)p.w, 0, p.wBytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, p.xBytes, 0x00020000);
   // weights: WM = 2 - a lane loads 8 consecutive k of row t / 2; WM = 1 - 4 consecutive k of row t / 4;
   //          WM = 0 - the same of row (t / 4) % 32: both halves of the workgroup fetch and park the same values
   // image:   WM = 2 - a lane gathers 8 taps of column t % 128; WM < 2 - all 16 taps of column t
   const int rowA = WM == 2 ? t >> 1 : WM == 1 ? t >> 2 : (t >> 2) & 31;
-  const int kgA = WM == 2 ? (t & 1) * 2 : t & 3;
+  const int kA = WM == 2 ? (t & 1) * 8 : (t & 3) * 4;
   const int colB = WM == 2 ? t & 127 : t;
-  const int kgB = WM == 2 ? (t >> 7) * 2 : 0;
-  const int aOff = (min(m0 + rowA, p.M - 1) * g.K + kgA * 4) * 4;
-  const int kB = __builtin_amdgcn_readfirstlane(kgB * 4);
-  int posOff;
-  {
-    const unsigned lg = min((unsigned)j0 + colB, (unsigned)p.Ncols - 1);  // Ncols < 2^31
+  const int kgB = WM == 2 ? t >> 7 : 0;
+  const int aOff = (min(m0 + rowA, p.M - 1) * g.K + kA) * 4;
+  const int kB = __builtin_amdgcn_readfirstlane(kgB * 8);
+  auto columnOffset = [&](unsigned col) {
     int n, oh, ow;
-    splitColumn(p, g, lg, n, oh, ow);
-    posOff = ((n * g.Cin * g.H + oh * g.dH) * g.W + ow * g.dW) * 4;
-  }
+    splitColumn(p, g, min(col, (unsigned)p.Ncols - 1), n, oh, ow);  // Ncols < 2^31
+    return ((n * g.Cin * g.H + oh * g.dH) * g.W + ow * g.dW) * 4;
+  };
+  const int posOff = columnOffset((unsigned)j0 + colB);
   const int ktBegin = by * p.ktPerSplit;  // by == 0 for whole tiles
   const int nkt = whole ? g.K / BK : min(g.K / BK, ktBegin + p.ktPerSplit);  // this workgroup reduces k-tiles [ktBegin, nkt)
 
@@ -991,40 +1043,67 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
       rb[4 * i + 3] = __builtin_amdgcn_raw_buffer_load_b32(xr, posOff, e[i].w, 0);
     }
   };
-  u32x4 *aDst = reinterpret_cast<u32x4 *>(&As[0][kgA][rowA]);
-  u32x4 *bDst = reinterpret_cast<u32x4 *>(&Bs[0][kgB][colB]);
-  constexpr int BUFA = (BK / 4) * AP, BUFB = (BK / 4) * BP;  // float4 per LDS buffer
+  constexpr int PA = 2 * AP, PB = 2 * BP;    // 16-byte groups of one part in one buffer
+  constexpr int BUFA = 3 * PA, BUFB = 3 * PB;  // of one buffer
+  u32x4 *aDst = &As[0][0][kA >> 3][rowA];
+  u32x4 *bDst = &Bs[0][0][kgB][colB];
   auto storeTiles = [&](auto bufc) {
     constexpr int b = decltype(bufc)::value;
+    if constexpr (WM == 2) {
+      unsigned h[4], m[4], l[4];
 #pragma unroll
-    for (int i = 0; i < NA; ++i) aDst[b * BUFA + i * AP] = ra[i];
+      for (int i = 0; i < 2; ++i) {
+        splitPair(ra[i].x, ra[i].y, h[2 * i], m[2 * i], l[2 * i]);
+        splitPair(ra[i].z, ra[i].w, h[2 * i + 1], m[2 * i + 1], l[2 * i + 1]);
+      }
+      aDst[b * BUFA] = u32x4{h[0], h[1], h[2], h[3]};
+      aDst[b * BUFA + PA] = u32x4{m[0], m[1], m[2], m[3]};
+      aDst[b * BUFA + 2 * PA] = u32x4{l[0], l[1], l[2], l[3]};
+    } else {  // 4 k: half of a group
+      unsigned h[2], m[2], l[2];
+      splitPair(ra[0].x, ra[0].y, h[0], m[0], l[0]);
+      splitPair(ra[0].z, ra[0].w, h[1], m[1], l[1]);
+      u32x2 *d = reinterpret_cast<u32x2 *>(aDst + b * BUFA) + ((kA >> 2) & 1);
+      d[0] = u32x2{h[0], h[1]};
+      d[2 * PA] = u32x2{m[0], m[1]};
+      d[4 * PA] = u32x2{l[0], l[1]};
+    }
 #pragma unroll
-    for (int i = 0; i < NB / 4; ++i) bDst[b * BUFB + i * BP] = u32x4{rb[4 * i], rb[4 * i + 1], rb[4 * i + 2], rb[4 * i + 3]};
+    for (int q = 0; q < NB / 8; ++q) {
+      unsigned h[4], m[4], l[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) splitPair(rb[8 * q + 2 * i], rb[8 * q + 2 * i + 1], h[i], m[i], l[i]);
+      bDst[b * BUFB + q * BP] = u32x4{h[0], h[1], h[2], h[3]};
+      bDst[b * BUFB + PB + q * BP] = u32x4{m[0], m[1], m[2], m[3]};
+      bDst[b * BUFB + 2 * PB + q * BP] = u32x4{l[0], l[1], l[2], l[3]};
+    }
   };
   const int grp = lane >> 5, idx = lane & 31;
-  const float4 *aSrc = &As[0][grp][wm * 64 + idx];
-  const float4 *bSrc = &Bs[0][grp][wn * 64 + idx];
+  const u32x4 *aSrc = &As[0][0][grp][wm * 64 + idx];
+  const u32x4 *bSrc = &Bs[0][0][grp][wn * 64 + idx];
   using Buf0 = std::integral_constant<int, 0>;
   using Buf1 = std::integral_constant<int, 1>;
 
-  // Software pipeline. While tile kt is multiplied out of one LDS buffer, tile kt + 1 waits in
-  // registers and tile kt + 2 is requested from memory:
-  //   first 16 MFMAs of kt | registers (kt + 1) -> other LDS buffer, global loads of kt + 2 |
-  //   last 16 MFMAs of kt | barrier
-  // The LDS stores and the load issue sit between the two MFMA halves, so the matrix pipe has
-  // queued work while they run and the only stall left at the barrier is the LDS read latency.
-  // The scheduling fences pin that order.
+  float16v acc[TI][2], lo[TI][2];
+
+  // Software pipeline. While tile kt is multiplied out of one LDS buffer, tile kt + 1 waits in registers - it is
+  // split and parked in the other buffer under the matrix instructions - and tile kt + 2 is requested from memory.
   auto step = [&](auto cur, auto nxt, int kt, bool store, bool load) {
     constexpr int C = decltype(cur)::value;
-    mfmaHalf<C * BUFA, C * BUFB>(aSrc, bSrc, acc);
-    __builtin_amdgcn_sched_barrier(0);
+    u32x4 a[3][TI], b[3][2];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i) a[s][i] = aSrc[C * BUFA + s * PA + 32 * i];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) b[s][j] = bSrc[C * BUFB + s * PB + 32 * j];
+    }
     if (store) storeTiles(nxt);
     if (load) {
       loadTiles(kt + 2);
       loadTaps(kt + 3);
     }
-    __builtin_amdgcn_sched_barrier(0);
-    mfmaHalf<C * BUFA + 2 * AP, C * BUFB + 2 * BP>(aSrc, bSrc, acc);
+    mfmaSplit<TI>(a, b, acc, lo);
     __syncthreads();
   };
 
@@ -1038,17 +1117,23 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   }
   __syncthreads();
   // the accumulators of a whole tile start from the bias (in LDS since the barrier): no addition in the epilogue
-  {
-    const int grpRow = (lane >> 5) * 4;
+  auto biasBlock = [&](int i) {
+    float16v v;
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
+    for (int q = 0; q < 4; ++q) {
+      float4 b4 = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (whole) b4 = *reinterpret_cast<const float4 *>(biasS + wm * 64 + i * 32 + 8 * q + grp * 4);
+      v[4 * q] = b4.x, v[4 * q + 1] = b4.y, v[4 * q + 2] = b4.z, v[4 * q + 3] = b4.w;
+    }
+    return v;
+  };
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float4 b4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (whole) b4 = *reinterpret_cast<const float4 *>(biasS + wm * 64 + i * 32 + 8 * q + grpRow);
+  for (int i = 0; i < TI; ++i) {
+    acc[i][0] = acc[i][1] = biasBlock(i);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j][4 * q] = b4.x, acc[i][j][4 * q + 1] = b4.y, acc[i][j][4 * q + 2] = b4.z, acc[i][j][4 * q + 3] = b4.w;
-      }
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) lo[i][j][v] = 0.f;
   }
   int kt = ktBegin;
   for (; kt + 3 < nkt; kt += 2) {  // tile kt sits in buffer 0, tile kt + 1 in registers
@@ -1059,11 +1144,47 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   step(Buf0{}, Buf1{}, kt, kt + 1 < nkt, kt + 2 < nkt);
   if (kt + 1 < nkt) step(Buf1{}, Buf0{}, kt + 1, kt + 2 < nkt, false);
   if (kt + 2 < nkt) step(Buf0{}, Buf1{}, kt + 2, false, false);
+
+  float bad = 0.f;  // NaN as soon as one sum is not finite
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        acc[i][j][v] += lo[i][j][v];
+        bad = __builtin_fmaf(acc[i][j][v], 0.f, bad);
+      }
+  if (__any(bad != bad)) {
+    // the wave's blocks again in fp32, operands straight from memory
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int cOff = columnOffset((unsigned)j0 + wn * 64 + j * 32 + idx);
+#pragma unroll
+      for (int i = 0; i < TI; ++i) {
+        const int rOff = min(m0 + wm * 64 + i * 32 + idx, p.M - 1) * g.K;
+        float16v c = biasBlock(i);
+#pragma unroll 1
+        for (int k = ktBegin * BK; k < nkt * BK; k += 8) {
+          float av[4], bv[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int kk = k + 2 * u + grp;
+            av[u] = p.w[rOff + kk];
+            bv[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, cOff + (LINEAR ? kk * p.tapStride : p.taps[kk]), 0, 0));
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u], bv[u], c, 0, 0, 0);
+        }
+        acc[i][j] = c;
+      }
+    }
+  }
   fwdEpilogue<TBN, TI>(p, g, acc, bx, by, m0, j0, wm, wn, grp, idx, biasS, whole ? 0 : 1, whole);
 }
 
 template <int WM, bool LINEAR = false>
-__global__ void __launch_bounds__(dev::kBlock, 3)
+__global__ void __launch_bounds__(dev::kBlock, 2)
 convFwdPaddedKernel(FwdArgs p, ConvGeom g) {
   int bx = blockIdx.x, by = 0;
   const bool whole = bx < p.full;
@@ -1092,7 +1213,7 @@ struct FwdBatch {
 static_assert(sizeof(FwdBatch) <= 4096, "kernel arguments are limited to 4 KB");
 
 template <int WM>
-__global__ void __launch_bounds__(dev::kBlock, 3)
+__global__ void __launch_bounds__(dev::kBlock, 2)
 convFwdPaddedBatchKernel(FwdBatch b) {
   int bx = blockIdx.x, by = 0, i = 0;
   const bool whole = bx < b.wholeTotal;

@@ -1,0 +1,94 @@
+"""Convolutions multiply fp32 operands as six products of bf16 parts (SpatialConvolutionMM,
+lib/THCUNN/generic/SpatialConvolutionMM.cu:58-486). Checked here: the error against a 64-bit sum stays below what
+fp32 additions alone would give, also for one-signed and badly scaled operands, and infinities, NaNs and values that
+would round up to infinity as bf16 come out exactly as an fp32 convolution gives them (an operand that is not finite
+must not spread to outputs it does not reach).
+
+Bound of the error: a chain of K fp32 additions rounds K times, each by at most 2^-24 of the partial sum, with random
+sign: about 2^-24 sqrt(K) / 2 of the result's norm for operands of mixed sign, and for one-signed operands (partial
+sums that grow to the result) less than that."""
+import numpy as np
+import pytest
+
+import cunn_amd
+
+pytestmark = pytest.mark.gpu
+
+from oracle import oracle as O  # noqa: E402
+
+# N, Cin, Cout, H, W, k, stride, pad
+CASES = [
+    (2, 64, 128, 12, 12, 3, 1, 1),
+    (3, 36, 70, 9, 11, 3, 2, 1),      # strided, ragged rows and columns
+    (2, 20, 40, 14, 10, 5, 1, 0),
+    (4, 512, 128, 7, 8, 1, 1, 0),     # 1x1 with a long reduction
+    (2, 3, 24, 21, 19, 3, 1, 1),      # three input planes
+]
+
+
+def _tensors(case, kind, seed=5):
+    N, Ci, Co, H, W, k, st, pad = case
+    rng = np.random.default_rng(seed)
+    oH, oW = (H + 2 * pad - k) // st + 1, (W + 2 * pad - k) // st + 1
+    x, w, gy = (rng.standard_normal(s) for s in ((N, Ci, H, W), (Co, Ci * k * k), (N, Co, oH, oW)))
+    if kind == "one-signed":
+        x, w, gy = np.abs(x), np.abs(w), np.abs(gy)
+    elif kind == "scaled":
+        x *= np.exp2(np.round(rng.standard_normal(x.shape) * 4))
+        gy *= np.exp2(np.round(rng.standard_normal(gy.shape) * 4))
+    elif kind == "tiny":
+        x, w = x * 1e-30, w * 1e-3
+    return tuple(v.astype(np.float32) for v in (x, w, gy))
+
+
+def _passes(case, x, w, gy, gyw):
+    """(output, gradInput from gy, gradWeight from gyw) of the library"""
+    N, Ci, Co, H, W, k, st, pad = case
+    THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
+    g = (k, k, st, st, pad, pad)
+    tx, tw, y, gx, gw = CT.from_numpy(x), CT.from_numpy(w), CT(), CT(), CT.from_numpy(np.zeros_like(w))
+    THNN.SpatialConvolutionMM_updateOutput(tx, y, tw, None, CT(), CT(), *g)
+    THNN.SpatialConvolutionMM_updateGradInput(tx, CT.from_numpy(gy), gx, tw, CT(), CT(), *g)
+    THNN.SpatialConvolutionMM_accGradParameters(tx, CT.from_numpy(gyw), gw, None, CT(), CT(), *g, 1.0)
+    return y.numpy(), gx.numpy(), gw.numpy()
+
+
+@pytest.mark.parametrize("kind", ["normal", "one-signed", "scaled", "tiny"])
+@pytest.mark.parametrize("case", CASES)
+def test_error_against_64_bit_sums(case, kind):
+    import torch
+    print("case", case, kind, flush=True)
+    N, Ci, Co, H, W, k, st, pad = case
+    x, w, gy = _tensors(case, kind)
+    dx, dw = (torch.from_numpy(v).double().requires_grad_() for v in (x, w.reshape(Co, Ci, k, k)))
+    y = torch.nn.functional.conv2d(dx, dw, stride=st, padding=pad)
+    y.backward(torch.from_numpy(gy).double())
+    terms = (Ci * k * k, Co * k * k, N * gy.shape[2] * gy.shape[3])
+    for got, ref, n in zip(_passes(case, x, w, gy, gy), (y.detach(), dx.grad, dw.grad), terms):
+        ref = ref.numpy().reshape(got.shape)
+        err = np.linalg.norm(got.astype(np.float64) - ref) / np.linalg.norm(ref)
+        assert err <= 2.0 ** -25 * np.sqrt(n) + 2.0 ** -24, (err, n)   # + one rounding of the result
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_non_finite_operands(case):
+    print("case", case, flush=True)
+    N, Ci, Co, H, W, k, st, pad = case
+    x, w, gy = _tensors(case, "normal", 6)
+    w *= 1e-3
+    x[0, 1, 2, 3], x[1, 0, 4, 4], x[N - 1, Ci - 1, H - 1, W - 1], x[0, 2, H - 1, 0] = np.inf, np.nan, 3.4e38, -3.4e38
+    gy[0, 3, 1, 2], gy[1, 0, 0, 0] = -np.inf, np.nan
+    gyw = gy * np.float32(1e-3)          # times 3.4e38 still finite: no sum overflows in one order and not in another
+    gy[N - 1, Co - 1, 2, 1] = 3.4e38
+    g = (k, k, st, st, pad, pad)
+    with np.errstate(all="ignore"):
+        gw = np.zeros_like(w)
+        ref = (O.convmm_updateOutput(x, w, None, *g), O.convmm_updateGradInput(x.shape, gy, w, *g),
+               O.convmm_accGradParameters(x, gyw, gw, None, *g, 1.0)[0])
+    for name, got, r in zip(("output", "gradInput", "gradWeight"), _passes(case, x, w, gy, gyw), ref):
+        print(name)
+        assert np.array_equal(np.isnan(got), np.isnan(r)) and np.array_equal(np.isposinf(got), np.isposinf(r))
+        assert np.array_equal(np.isneginf(got), np.isneginf(r))
+        fine = np.isfinite(r)
+        # relative to the largest term: 3.4e38 times a weight
+        np.testing.assert_allclose(got[fine], r[fine], rtol=1e-5, atol=max(1e-4, 1e-6 * np.abs(r[fine], dtype=np.float64).max()))
