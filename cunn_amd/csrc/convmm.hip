@@ -1586,6 +1586,260 @@ convGradWeightKernel(GradWeightArgs p, ConvGeom g) {
   }
 }
 
+// The large tiles on split operands (fp32 products on the bf16 matrix pipe, see the forward kernel): a matrix
+// instruction consumes 8 consecutive positions per lane, so the operands of a k-tile sit in LDS as 16-byte groups of
+// 8 positions, one array per part. Both loaders hand over 4 consecutive positions of a row or column at a time:
+//  * gradOutput: 16-byte loads, as they are in memory
+//  * image, B4: 4 consecutive positions of a column are 4 consecutive floats (unit stride along the row, and the 4
+//    positions never straddle two output rows - or the rows follow each other without a gap): 16-byte loads
+//  * image, else: a lane owns one position of the k-tile and gathers groups of 4 neighbouring columns (16 lanes read
+//    16 consecutive positions, 64-byte runs); the 4 lanes of a quad then transpose their 4 x 4 elements through DPP
+// WM = 2: 128 x 128 tiles of gradWeight (Cout x K), WM = 1: 64 x 256 tiles; a wave multiplies 64 x 64 either way.
+// A partial tile whose sums are not all finite is computed again with the fp32 instruction, straight from memory.
+// What bounds it: as the forward kernel, two workgroups per CU and a clock that power pulls down. Against the fp32
+// instruction: 256 x 2304 over 64 x 28 x 28 positions (59.2 GFLOP) 519 -> 334 us; 192 x 720 over 32 x 71 x 71 (64 x 256
+// tiles, gathers transposed) 462 -> 342 us; 256 x 2048, stride 2, over 64 x 14 x 14 142 -> 99 us.
+template <bool L16, int WM, bool B4>
+__global__ void __launch_bounds__(dev::kBlock, 2)
+convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
+  constexpr int TBM = 64 * WM, TBN = 256 / WM;
+  constexpr int AP = TBM + 8, BP = TBN + 8;     // 16-byte groups (8 positions of one part) per position-group row
+  constexpr int NQ = TBN / 64;                  // groups of 4 positions a lane parks per k-tile
+  constexpr int NT = B4 ? NQ : 4 * NQ;          // columns a lane fetches
+  __shared__ u32x4 As[2][3][2][AP];             // [buffer][part][group of 8 positions][row]
+  __shared__ u32x4 Bs[2][3][2][BP];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wm = WM == 2 ? wave >> 1 : 0, wn = WM == 2 ? wave & 1 : wave;
+  // workgroups that reduce the same positions (one split) are neighbours in the remapped order: same XCD, same L2
+  const int tilesPerSplit = p.mTiles * p.nTiles;
+  const int bid = dev::xcdRemap(blockIdx.x, gridDim.x);
+  const int split = bid / tilesPerSplit, tileIdx = bid - split * tilesPerSplit;
+  const int mTile = tileIdx % p.mTiles, nTile = tileIdx / p.mTiles;
+  const int m0 = mTile * TBM, j0 = nTile * TBN;
+  const int ktBegin = split * p.ktPerSplit;
+  const int ktEnd = min(p.totalKt, ktBegin + p.ktPerSplit);
+  const int kOob = 0x7fffffff;
+
+  // ---- gradOutput. WM = 2: row t >> 1, positions 8 * (t & 1) .. + 7 of the k-tile; WM = 1: row t >> 2, positions
+  //      4 * (t & 3) .. + 3
+  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc((void *)p.gy, 0, p.gyBytes, 0x00020000);
+  const int rowA = WM == 2 ? t >> 1 : t >> 2;
+  const int pgA = WM == 2 ? (t & 1) * 2 : t & 3;  // first group of 4 positions of the lane
+  const int rowOffA = min(m0 + rowA, p.M - 1) * g.L * 4;  // rows past M are clamped and dropped in the epilogue
+  const int imgStrideA = p.M * g.L * 4;
+  int nA, lA;  // L16: scalar image and position of the k-tile; else: of this lane's first group
+  {
+    const unsigned r = (unsigned)ktBegin * BK + (L16 ? 0 : pgA * 4);  // N * L < 2^31
+    nA = (int)(r / (unsigned)g.L);
+    lA = (int)(r - (unsigned)nA * (unsigned)g.L);
+  }
+  // ---- image. B4: positions 4 * (t & 3) .. + 3, columns (t >> 2) + 64 i;
+  //             else position t & 15, columns 4 * (t >> 4) + 64 i .. + 3
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, p.xBytes, 0x00020000);
+  const int rB = B4 ? (t & 3) * 4 : t & 15;
+  auto columnOffset = [&](int col) {  // byte offset of a column's tap; columns past K are dropped in the epilogue
+    const int k = min(col, p.Ncols - 1), KK = g.kH * g.kW;
+    const int c = dev::fastDiv(k, p.magicKK), rem = k - c * KK;
+    const int kh = dev::fastDiv(rem, p.magicKW), kw = rem - kh * g.kW;
+    return ((c * g.H + kh * g.dilH) * g.W + kw * g.dilW) * 4;
+  };
+  int tapOff[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) tapOff[i] = columnOffset(j0 + (B4 ? (t >> 2) + 64 * i : (t >> 4) * 4 + 64 * (i >> 2) + (i & 3)));
+  const int imgStrideB = g.Cin * g.H * g.W * 4;
+  const int rowStepB = g.dH * g.W * 4, colStepB = g.dW * 4;
+  int lB, nOffB;  // position inside the image, byte offset of the image (>= xBytes past the batch: loads return 0)
+  {
+    const unsigned r = (unsigned)ktBegin * BK + rB;
+    const int n = (int)(r / (unsigned)g.L);
+    lB = (int)(r - (unsigned)n * (unsigned)g.L);
+    nOffB = n * imgStrideB;
+  }
+  // byte offset of position l of the image at nOff (positions behind the image's last one exist when the gradOutput
+  // rows were padded to a multiple of 4: their gradOutput is zero, they read the image at position 0)
+  auto positionOffset = [&](int l, int nOff) {
+    const int lq = l < p.Lvalid ? l : 0;
+    const int oh = dev::fastDiv(lq, p.magicOW), ow = lq - oh * g.oW;
+    return nOff + oh * rowStepB + ow * colStepB;
+  };
+
+  u32x4 ra[WM];
+  u32x4 rb[NQ];                 // B4: 4 positions of a column
+  unsigned re[B4 ? 1 : NT];     // else: one position of each column
+  // loads the k-tile the position counters stand on, then advances them by BK (L >= BK: one wrap at most)
+  auto loadTiles = [&]() {
+    if constexpr (L16) {
+      // N*L is a multiple of BK here, so every k-tile lies inside the batch (the scalar offset is not range-checked)
+      const int so = __builtin_amdgcn_readfirstlane(nA * imgStrideA + lA * 4);
+#pragma unroll
+      for (int i = 0; i < WM; ++i) ra[i] = __builtin_amdgcn_raw_buffer_load_b128(gr, rowOffA + pgA * 16 + 16 * i, so, 0);
+    } else {
+      ra[0] = __builtin_amdgcn_raw_buffer_load_b128(gr, nA < g.N ? nA * imgStrideA + rowOffA + lA * 4 : kOob, 0, 0);
+      if constexpr (WM == 2) {
+        int n1 = nA, l1 = lA + 4;
+        if (l1 >= g.L) l1 -= g.L, ++n1;
+        ra[1] = __builtin_amdgcn_raw_buffer_load_b128(gr, n1 < g.N ? n1 * imgStrideA + rowOffA + l1 * 4 : kOob, 0, 0);
+      }
+    }
+    lA += BK;
+    if (lA >= g.L) lA -= g.L, ++nA;
+    const unsigned posOff = (unsigned)positionOffset(lB, nOffB);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      if constexpr (B4)
+        rb[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(posOff + (unsigned)tapOff[i]), 0, 0);
+      else
+        re[i] = __builtin_amdgcn_raw_buffer_load_b32(xr, (int)(posOff + (unsigned)tapOff[i]), 0, 0);
+    }
+    lB += BK;
+    if (lB >= g.L) lB -= g.L, nOffB += imgStrideB;
+  };
+  constexpr int PA = 2 * AP, PB = 2 * BP;      // 16-byte groups of one part in one buffer
+  constexpr int BUFA = 3 * PA, BUFB = 3 * PB;  // of one buffer
+  u32x4 *aDst = &As[0][0][pgA >> 1][rowA];
+  const int pgB = B4 ? t & 3 : (t & 15) >> 2, colB = B4 ? t >> 2 : (t >> 4) * 4 + (t & 3);
+  u32x2 *bDst = reinterpret_cast<u32x2 *>(&Bs[0][0][pgB >> 1][colB]) + (pgB & 1);
+  // The workgroups of the first column tile also sum the gradOutput elements they pass on (each element of a
+  // row is loaded by exactly one lane of exactly one of them): the bias gradient without a second pass over gy.
+  const bool rowSums = nTile == 0 && p.biasPartial != nullptr;
+  float rowSum = 0.f;
+  auto split4 = [](const u32x4 &v, u32x2 (&part)[3]) {
+    unsigned h[2], m[2], l[2];
+    splitPair(v.x, v.y, h[0], m[0], l[0]);
+    splitPair(v.z, v.w, h[1], m[1], l[1]);
+    part[0] = u32x2{h[0], h[1]}, part[1] = u32x2{m[0], m[1]}, part[2] = u32x2{l[0], l[1]};
+  };
+  auto storeTiles = [&](auto bufc) {
+    constexpr int buf = decltype(bufc)::value;
+    u32x2 pa[WM][3];
+#pragma unroll
+    for (int i = 0; i < WM; ++i) split4(ra[i], pa[i]);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      if constexpr (WM == 2)
+        aDst[buf * BUFA + s * PA] = u32x4{pa[0][s].x, pa[0][s].y, pa[1][s].x, pa[1][s].y};
+      else
+        (reinterpret_cast<u32x2 *>(aDst + buf * BUFA + s * PA))[pgA & 1] = pa[0][s];
+    }
+    if (rowSums) {
+#pragma unroll
+      for (int i = 0; i < WM; ++i) {
+        // (element by element: a bit cast applied to a vector element expression reads element 0 here)
+        const unsigned ex = ra[i].x, ey = ra[i].y, ez = ra[i].z, ew = ra[i].w;
+        rowSum += (__uint_as_float(ex) + __uint_as_float(ey)) + (__uint_as_float(ez) + __uint_as_float(ew));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      if constexpr (!B4) rb[i] = dev::quadTranspose(re[4 * i], re[4 * i + 1], re[4 * i + 2], re[4 * i + 3]);
+      u32x2 pb[3];
+      split4(rb[i], pb);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) bDst[2 * (buf * BUFB + s * PB + 64 * i)] = pb[s];
+    }
+  };
+  const int grp = lane >> 5, idx = lane & 31;
+  const u32x4 *aSrc = &As[0][0][grp][wm * 64 + idx];
+  const u32x4 *bSrc = &Bs[0][0][grp][wn * 64 + idx];
+  using Buf0 = std::integral_constant<int, 0>;
+  using Buf1 = std::integral_constant<int, 1>;
+
+  float16v acc[2][2], lo[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = lo[i][j][v] = 0.f;
+
+  // same software pipeline as the forward kernel: tile kt in LDS, kt + 1 in registers, kt + 2 requested
+  auto step = [&](auto cur, auto nxt, bool store, bool load) {
+    constexpr int C = decltype(cur)::value;
+    u32x4 a[3][2], b[3][2];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) a[s][i] = aSrc[C * BUFA + s * PA + 32 * i];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) b[s][j] = bSrc[C * BUFB + s * PB + 32 * j];
+    }
+    if (store) storeTiles(nxt);
+    if (load) loadTiles();
+    mfmaSplit<2>(a, b, acc, lo);
+    __syncthreads();
+  };
+  if (ktBegin < ktEnd) {
+    loadTiles();
+    storeTiles(Buf0{});
+    if (ktBegin + 1 < ktEnd) loadTiles();
+    __syncthreads();
+    int kt = ktBegin;
+    for (; kt + 3 < ktEnd; kt += 2) {  // tile kt sits in buffer 0, tile kt + 1 in registers
+      step(Buf0{}, Buf1{}, true, true);
+      step(Buf1{}, Buf0{}, true, true);
+    }
+    // one to three tiles left
+    step(Buf0{}, Buf1{}, kt + 1 < ktEnd, kt + 2 < ktEnd);
+    if (kt + 1 < ktEnd) step(Buf1{}, Buf0{}, kt + 2 < ktEnd, false);
+    if (kt + 2 < ktEnd) step(Buf0{}, Buf1{}, false, false);
+  }
+
+  float bad = 0.f;  // NaN as soon as one sum is not finite
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        acc[i][j][v] += lo[i][j][v];
+        bad = __builtin_fmaf(acc[i][j][v], 0.f, bad);
+      }
+  if (__any(bad != bad)) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const unsigned tap = (unsigned)columnOffset(j0 + wn * 64 + j * 32 + idx);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int rOff = min(m0 + wm * 64 + i * 32 + idx, p.M - 1) * g.L * 4;
+        float16v c;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) c[v] = 0.f;
+#pragma unroll 1
+        for (int r0 = ktBegin * BK; r0 < ktEnd * BK; r0 += 2) {
+          const int r = r0 + grp, n = (int)((unsigned)r / (unsigned)g.L), l = r - n * g.L;
+          const float av = __uint_as_float(
+              __builtin_amdgcn_raw_buffer_load_b32(gr, n < g.N ? n * imgStrideA + rOff + l * 4 : kOob, 0, 0));
+          const float bv = __uint_as_float(
+              __builtin_amdgcn_raw_buffer_load_b32(xr, (int)((unsigned)positionOffset(l, n * imgStrideB) + tap), 0, 0));
+          c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
+        }
+        acc[i][j] = c;
+      }
+    }
+  }
+
+  // lane holds column (lane & 31), rows 8*(v/4) + 4*(lane/32) + v%4 of each 32x32 tile
+  float *dst = p.partial + (long)split * p.M * p.Ncols;
+#pragma unroll
+  for (int tj = 0; tj < 2; ++tj) {
+    const int col = j0 + wn * 64 + tj * 32 + idx;
+    if (col >= p.Ncols) continue;
+#pragma unroll
+    for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int row = m0 + wm * 64 + ti * 32 + 8 * (v >> 2) + grp * 4 + (v & 3);
+        if (row < p.M) dst[(long)row * p.Ncols + col] = acc[ti][tj][v];
+      }
+  }
+  if (rowSums) {
+    // the 2 (WM = 2) or 4 (WM = 1) lanes that loaded parts of a row are neighbours inside a quad
+    rowSum = dev::dppAdd<0xB1>(rowSum);
+    if (WM == 1) rowSum = dev::dppAdd<0x4E>(rowSum);
+    if ((t & (WM == 2 ? 1 : 3)) == 0 && m0 + rowA < p.M) p.biasPartial[(long)split * p.M + m0 + rowA] = rowSum;
+  }
+}
+
 // gW[i] += scale * sum_s partial[s][i] in a fixed association: a workgroup owns 64 consecutive float4
 // of gW; its 4 lane groups each sum the splits s = group, group + 4, ... with 4 independent
 // accumulators (16 16-byte loads in flight per lane), then the groups are added in order through
@@ -2775,9 +3029,9 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   auto bigKernel = [](auto l16c, auto wmc, auto b4c) {
     constexpr bool L = decltype(l16c)::value, B = decltype(b4c)::value;
     constexpr int W = decltype(wmc)::value;
-    return BigKernel{(const void *)convGradWeightKernel<L, W, 2, 2, B>,
+    return BigKernel{(const void *)convGradWeightSplitKernel<L, W, B>,
                      [](dim3 grid, hipStream_t st, const GradWeightArgs &q, const ConvGeom &gk) {
-                       convGradWeightKernel<L, W, 2, 2, B><<<grid, dev::kBlock, 0, st>>>(q, gk);
+                       convGradWeightSplitKernel<L, W, B><<<grid, dev::kBlock, 0, st>>>(q, gk);
                      }};
   };
   auto pickBig = [&](auto l16c, auto wmc) { return b4 ? bigKernel(l16c, wmc, std::true_type{}) : bigKernel(l16c, wmc, std::false_type{}); };

@@ -18,6 +18,20 @@ __device__ __forceinline__ float dppAdd(float v) {
   return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
+// 4 x 4 transpose inside each quad: lane q of a quad brings element q of four rows and leaves with the four elements of
+// row q. Two exchange steps (lane xor 1, lane xor 2), each one select per element with the DPP move folded in.
+__device__ __forceinline__ unsigned dppXor1(unsigned v) { return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true); }
+__device__ __forceinline__ unsigned dppXor2(unsigned v) { return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true); }
+typedef unsigned int quad_u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ quad_u32x4 quadTranspose(unsigned r0, unsigned r1, unsigned r2, unsigned r3) {
+  const bool odd = threadIdx.x & 1, upper = threadIdx.x & 2;
+  // after step 1 lane q holds elements (2 (q / 2), + 1) of rows q % 2 (s0, s1) and q % 2 + 2 (s2, s3)
+  const unsigned x0 = dppXor1(r0), x1 = dppXor1(r1), x2 = dppXor1(r2), x3 = dppXor1(r3);
+  const unsigned s0 = odd ? x1 : r0, s1 = odd ? r1 : x0, s2 = odd ? x3 : r2, s3 = odd ? r3 : x2;
+  const unsigned y0 = dppXor2(s0), y1 = dppXor2(s1), y2 = dppXor2(s2), y3 = dppXor2(s3);
+  return quad_u32x4{upper ? y2 : s0, upper ? y3 : s1, upper ? s2 : y0, upper ? s3 : y1};
+}
+
 // Sum over the 64 lanes of a wavefront, returned in every lane (wave-uniform).
 // Four DPP steps fold each row of 16 lanes (quad xor 1, quad xor 2, half-row
 // mirror, row mirror), then the four row sums are read as scalars and added.

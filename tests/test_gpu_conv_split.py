@@ -23,6 +23,14 @@ CASES = [
     (2, 20, 40, 14, 10, 5, 1, 0),
     (4, 512, 128, 7, 8, 1, 1, 0),     # 1x1 with a long reduction
     (2, 3, 24, 21, 19, 3, 1, 1),      # three input planes
+    # the weight gradient's large tiles: 128 x 128 and 64 x 256, k-tiles inside an image or not, 16-byte or transposed gathers
+    (2, 64, 120, 16, 16, 3, 2, 1),
+    (3, 64, 120, 9, 12, 3, 1, 1),
+    (2, 64, 128, 25, 25, 3, 2, 1),
+    (2, 28, 60, 16, 16, 3, 1, 1),
+    (2, 28, 60, 16, 16, 3, 2, 1),
+    (3, 28, 60, 9, 12, 3, 1, 1),
+    (3, 28, 60, 13, 14, 3, 1, 1),
 ]
 
 
