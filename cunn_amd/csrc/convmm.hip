@@ -536,31 +536,63 @@ __device__ __forceinline__ void flipWeights(const FlipJob &f, int block, int blo
   }
 }
 
-// xp(nc, Hp, Wp) = x(nc, H, W) at row padTop, column padLeft inside zeros. grid = (planes, chunks of a plane);
-// VEC: a lane produces 4 consecutive floats of the bordered plane with one 16-byte store
-// (plane size a multiple of 4 floats, 16-byte aligned destination).
-template <bool VEC>
+// xp(nc, Hp, Wp) = x(nc, H, W) at row padTop, column padLeft inside zeros, for any plane size and count: a workgroup
+// writes one run of kPadRun floats of the destination with 16-byte stores, wherever planes begin and end in it. One
+// scalar division per workgroup locates the run; inside it a lane's offsets are small, so the reciprocal divisions
+// are exact (a dividend below d + kPadRun with d < kPadRun; a larger d is passed at most once). The four elements of
+// a group are found by stepping. Bound by memory: 6144 planes 71 x 71 -> 75 x 75 (262 MB) 103 us with a lane per
+// element and a workgroup per 256 elements of a plane, 48 us (5.4 TB/s) in this form.
+constexpr int kPadRun = 4096;
 __global__ void __launch_bounds__(dev::kBlock)
-padPlanesKernel(const float *__restrict__ x, float *__restrict__ xp, int H, int W, int padTop, int padLeft, int Hp, int Wp,
-                int planes, int *taps, int tapEntries, ConvGeom tg) {
-  if ((int)blockIdx.x == planes) {  // one more column of workgroups builds the tap table of the convolution that follows
-    for (int k = blockIdx.y * dev::kBlock + threadIdx.x; k < tapEntries; k += gridDim.y * dev::kBlock) taps[k] = tapOffset(k, tg);
+padPlanesRunKernel(const float *__restrict__ x, float *__restrict__ xp, int H, int W, int padTop, int padLeft, int Hp, int Wp,
+                   long total, int copyBlocks, bool vec, int *taps, int tapEntries, ConvGeom tg, int tapBlocks, FlipJob flip) {
+  if ((int)blockIdx.x >= copyBlocks + tapBlocks) {  // the weights of the convolution that follows, flipped
+    flipWeights(flip, blockIdx.x - copyBlocks - tapBlocks, gridDim.x - copyBlocks - tapBlocks);
     return;
   }
-  const unsigned magic = dev::magicOf(Wp);
-  const float *src = x + (long)blockIdx.x * H * W;
-  float *dst = xp + (long)blockIdx.x * Hp * Wp;
-  auto fetch = [&](int j) {
-    const int hp = dev::fastDiv(j, magic), wp = j - hp * Wp;
-    const int h = hp - padTop, w = wp - padLeft;
-    return (((unsigned)h < (unsigned)H) & ((unsigned)w < (unsigned)W)) ? src[h * W + w] : 0.f;
-  };
-  const int i = blockIdx.y * dev::kBlock + threadIdx.x;
-  if (VEC) {
-    if (i * 4 < Hp * Wp)
-      *reinterpret_cast<float4 *>(dst + i * 4) = make_float4(fetch(i * 4), fetch(i * 4 + 1), fetch(i * 4 + 2), fetch(i * 4 + 3));
-  } else {
-    if (i < Hp * Wp) dst[i] = fetch(i);
+  if ((int)blockIdx.x >= copyBlocks) {              // its tap table
+    for (int k = (blockIdx.x - copyBlocks) * dev::kBlock + threadIdx.x; k < tapEntries; k += tapBlocks * dev::kBlock)
+      taps[k] = tapOffset(k, tg);
+    return;
+  }
+  const int plane = Hp * Wp;
+  const unsigned magicPlane = dev::magicOf(plane), magicW = dev::magicOf(Wp);
+  const long e0 = (long)blockIdx.x * kPadRun;
+  const long pl0 = e0 / plane;
+  const int r0 = (int)(e0 - pl0 * plane), h0 = r0 / Wp, c0 = r0 - h0 * Wp;
+  const float *src = x + pl0 * H * W;
+  float v[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int o = (u * dev::kBlock + threadIdx.x) * 4;
+    const int r = r0 + o;
+    int pl = plane < kPadRun ? dev::fastDiv(r, magicPlane) : r >= plane;
+    const int j = pl ? r - pl * plane : c0 + o;
+    int hp = Wp < kPadRun ? dev::fastDiv(j, magicW) : j >= Wp;
+    int wp = j - hp * Wp;
+    if (!pl) hp += h0;
+    const int left = (int)min(total - e0, (long)kPadRun) - o;  // elements of the destination from here on
+    int h = hp - padTop, w = wp - padLeft, at = (pl * H + h) * W + w;  // (spans less than a run past a plane: an int)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[u][k] = (((unsigned)h < (unsigned)H) & ((unsigned)w < (unsigned)W) & (k < left)) ? src[at] : 0.f;
+      ++w, ++at;
+      if (w == Wp - padLeft) {
+        w = -padLeft, ++h, at += W - Wp;
+        if (h == Hp - padTop) h = -padTop, at += (H - Hp) * W;
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const long e = e0 + (u * dev::kBlock + threadIdx.x) * 4;
+    if (vec && e + 4 <= total) {
+      *reinterpret_cast<float4 *>(xp + e) = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (e + k < total) xp[e + k] = v[u][k];
+    }
   }
 }
 
@@ -632,36 +664,26 @@ void launchPadPlanes(hipStream_t s, const float *x, float *xp, long planes, int 
   const int plane = Hp * Wp;
   const FlipJob fj = flip ? *flip : FlipJob{};
   const int flipBlocks = flip ? (int)std::min<long>(kFlipBlocks, ((long)fj.Cout * fj.Cin * fj.kH * fj.kW + dev::kBlock - 1) / dev::kBlock) : 0;
-  auto flipAlone = [&]() {
-    if (!flip) return;
-    flipWeightKernel<<<launch::directGrid((long)fj.Cout * fj.Cin * fj.kH * fj.kW, dev::kBlock), dev::kBlock, 0, s>>>(
-        fj.w, fj.wf, fj.Cout, fj.Cin, fj.kH, fj.kW);
-  };
   if (launch::ceilDiv(plane, dev::kBlock) > 65535) error("SpatialConvolutionMM: image plane too large");
-  const unsigned gx = (unsigned)planes + (taps ? 1 : 0);
+  const int tapBlocks = taps ? std::max(1, std::min(16, launch::ceilDiv(tapEntries, dev::kBlock))) : 0;
   const ConvGeom g = tg ? *tg : ConvGeom{};
   const long total4 = planes * (plane / 4);
   // (the reciprocal division of a group index by the groups per plane is exact while index * divisor < 2^32)
   if (plane % 4 == 0 && plane < 4096 && launch::aligned16(xp) && total4 * (plane / 4) < 0xffffffffL) {
     const int copyBlocks = (int)std::min<long>((total4 + dev::kBlock - 1) / dev::kBlock, 16384);
-    const int tapBlocks = taps ? std::max(1, std::min(16, launch::ceilDiv(tapEntries, dev::kBlock))) : 0;
     padPlanesFlatKernel<false><<<copyBlocks + tapBlocks + flipBlocks, dev::kBlock, 0, s>>>(
         x, xp, H, W, padTop, padLeft, Hp, Wp, total4, copyBlocks, taps, tapEntries, g, tapBlocks, fj);
   } else if (plane < 1024 && launch::aligned16(xp) && planes * plane * (long)plane < 0xffffffffL) {
     // small planes of any size (a bordered 7x7 or 13x13 plane): a workgroup per plane would leave most of its lanes idle
     const long total = planes * plane;
     const int copyBlocks = (int)std::min<long>(((total + 3) / 4 + dev::kBlock - 1) / dev::kBlock, 16384);
-    const int tapBlocks = taps ? std::max(1, std::min(16, launch::ceilDiv(tapEntries, dev::kBlock))) : 0;
     padPlanesFlatKernel<true><<<copyBlocks + tapBlocks + flipBlocks, dev::kBlock, 0, s>>>(
         x, xp, H, W, padTop, padLeft, Hp, Wp, total, copyBlocks, taps, tapEntries, g, tapBlocks, fj);
-  } else if (plane % 4 == 0 && launch::aligned16(xp)) {
-    flipAlone();
-    padPlanesKernel<true><<<dim3(gx, launch::ceilDiv(plane / 4, dev::kBlock)), dev::kBlock, 0, s>>>(
-        x, xp, H, W, padTop, padLeft, Hp, Wp, (int)planes, taps, tapEntries, g);
   } else {
-    flipAlone();
-    padPlanesKernel<false><<<dim3(gx, launch::ceilDiv(plane, dev::kBlock)), dev::kBlock, 0, s>>>(
-        x, xp, H, W, padTop, padLeft, Hp, Wp, (int)planes, taps, tapEntries, g);
+    const long total = planes * plane, copyBlocks = (total + kPadRun - 1) / kPadRun;
+    if (copyBlocks + tapBlocks + flipBlocks > 0x7fffffffL) error("SpatialConvolutionMM: batch too large");
+    padPlanesRunKernel<<<(unsigned)copyBlocks + tapBlocks + flipBlocks, dev::kBlock, 0, s>>>(
+        x, xp, H, W, padTop, padLeft, Hp, Wp, total, (int)copyBlocks, launch::aligned16(xp), taps, tapEntries, g, tapBlocks, fj);
   }
   THC_HIP_CHECK(hipGetLastError());
 }

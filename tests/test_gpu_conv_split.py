@@ -31,6 +31,10 @@ CASES = [
     (2, 28, 60, 16, 16, 3, 2, 1),
     (3, 28, 60, 9, 12, 3, 1, 1),
     (3, 28, 60, 13, 14, 3, 1, 1),
+    # bordered copies in runs: planes of an odd size, larger than a run, smaller with several to a run, wide rows
+    (2, 8, 24, 67, 61, 3, 1, 1),
+    (33, 64, 8, 37, 35, 3, 1, 1),
+    (1, 8, 16, 3, 4500, 3, 1, 1),
 ]
 
 
