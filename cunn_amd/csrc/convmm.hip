@@ -958,16 +958,16 @@ __device__ __forceinline__ void splitPair(unsigned x0, unsigned x1, unsigned &h,
 
 __device__ __forceinline__ bf16x8 asBf16(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
-// One k-step of 16 of one wave: TI x 2 blocks of 32 x 32. a[s][i], b[s][j]: part s (h, m, l) of the lane's 8
-// consecutive k (k-group lane / 32) of row / column lane % 32 of a block.
-template <int TI>
-__device__ __forceinline__ void mfmaSplit(const u32x4 (&a)[3][TI], const u32x4 (&b)[3][2], float16v (&hi)[TI][2],
-                                          float16v (&lo)[TI][2]) {
-  auto all = [&](int sa, int sb, float16v (&acc)[TI][2]) {
+// One k-step of 16 of one wave: TI x TJ blocks of 32 x 32. a[s][i], b[s][j]: part s (h, m, l) of the lane's 8
+// k (k-group lane / 32) of row / column lane % 32 of a block.
+template <int TI, int TJ>
+__device__ __forceinline__ void mfmaSplit(const u32x4 (&a)[3][TI], const u32x4 (&b)[3][TJ], float16v (&hi)[TI][TJ],
+                                          float16v (&lo)[TI][TJ]) {
+  auto all = [&](int sa, int sb, float16v (&acc)[TI][TJ]) {
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < TJ; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(asBf16(a[sa][i]), asBf16(b[sb][j]), acc[i][j], 0, 0, 0);
   };
   all(0, 0, hi);
@@ -1125,7 +1125,7 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
       loadTiles(kt + 2);
       loadTaps(kt + 3);
     }
-    mfmaSplit<TI>(a, b, acc, lo);
+    mfmaSplit(a, b, acc, lo);
     __syncthreads();
   };
 
@@ -1203,6 +1203,173 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
     }
   }
   fwdEpilogue<TBN, TI>(p, g, acc, bx, by, m0, j0, wm, wn, grp, idx, biasS, whole ? 0 : 1, whole);
+}
+
+// Forward kernel for short calls (planDirect): a workgroup computes a tile of 32 T x 32 T, its four waves a quarter of
+// K each, folded through LDS at the end; both operands go from memory straight into the registers that the matrix
+// instructions read (no LDS, no barrier in the loop). So a short call fills the chip without partial tiles in memory and
+// a second launch. Bound by latency: the loads of D k-steps are in flight, then by the weight loads (a 16-byte load of
+// 32 rows touches 64 cache lines). Lanes 0-31 work on the first half of the input planes, lanes 32-63 on the second half
+// (the order of a sum's terms is free), so that a tap's offset is the same for the whole wave: a scalar.
+// Needs whole k-steps: K % 16 == 0 and Cin even. Operands as in the padded kernel (images with their border, 16-byte
+// loadable weight rows, tap table); the grid is the number of tiles.
+template <int T, bool LINEAR>
+__global__ void __launch_bounds__(dev::kBlock, T == 2 ? 2 : 3)
+convFwdDirectKernel(FwdArgs p, ConvGeom g) {
+  constexpr int TI = T, TJ = T;                            // blocks of 32 x 32
+  constexpr int D = T == 1 ? 4 : 2;                        // k-steps in flight
+  constexpr int RQ = TI * TJ * 4;                          // groups of 4 accumulator registers
+  __shared__ float4 red[4][RQ][dev::kWave];
+  const int lane = threadIdx.x & 63, slice = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = lane >> 5, idx = lane & 31;
+  const int tile = dev::xcdRemap(blockIdx.x, gridDim.x);    // (neighbours share columns: same XCD, same L2)
+  const int nTile = tile / p.mTiles, mTile = tile - nTile * p.mTiles;
+  const int m0 = mTile * 32 * TI, j0 = nTile * 32 * TJ;
+
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void *)p.w, 0, p.wBytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, p.xBytes, 0x00020000);
+  const int halfK = g.K >> 1, halfX = (g.Cin >> 1) * g.H * g.W * 4;
+  int rowOff[TI], posOff[TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i) rowOff[i] = (min(m0 + i * 32 + idx, p.M - 1) * g.K + grp * halfK) * 4;
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) {
+    int n, oh, ow;
+    splitColumn(p, g, min((unsigned)(j0 + j * 32 + idx), (unsigned)p.Ncols - 1), n, oh, ow);
+    posOff[j] = ((n * g.Cin * g.H + oh * g.dH) * g.W + ow * g.dW) * 4 + grp * halfX;
+  }
+  const int steps = halfK >> 3, perSlice = (steps + 3) / 4;
+  const int s0 = slice * perSlice, s1 = min(steps, s0 + perSlice);
+
+  u32x4 ra[D][TI][2];
+  unsigned rb[D][TJ][8];
+  int4 t0, t1;                                             // the taps of the next step to be loaded
+  auto loadTaps = [&](int step) {
+    if (LINEAR) return;
+    const int4 *tp = reinterpret_cast<const int4 *>(p.taps + min(step, steps - 1) * 8);
+    t0 = tp[0], t1 = tp[1];
+  };
+  auto load = [&](auto dc, int step) {
+    constexpr int d = decltype(dc)::value;
+    // (steps past the slice: empty resources, everything reads as 0)
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void *)p.w, 0, step < s1 ? p.wBytes : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, step < s1 ? p.xBytes : 0, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) ra[d][i][q] = __builtin_amdgcn_raw_buffer_load_b128(wr, rowOff[i] + 16 * q, step * 32, 0);
+    const int tap[8] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        rb[d][j][e] = __builtin_amdgcn_raw_buffer_load_b32(xr, posOff[j], LINEAR ? (step * 8 + e) * p.tapStride : tap[e], 0);
+    loadTaps(step + 1);
+  };
+  float16v acc[TI][TJ], lo[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = lo[i][j][v] = 0.f;
+  auto split8 = [](const unsigned (&v)[8], u32x4 &h, u32x4 &m, u32x4 &l) {
+    unsigned ph[4], pm[4], pl[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) splitPair(v[2 * q], v[2 * q + 1], ph[q], pm[q], pl[q]);
+    h = u32x4{ph[0], ph[1], ph[2], ph[3]}, m = u32x4{pm[0], pm[1], pm[2], pm[3]}, l = u32x4{pl[0], pl[1], pl[2], pl[3]};
+  };
+  auto step = [&](auto dc, int next) {
+    constexpr int d = decltype(dc)::value;
+    u32x4 a[3][TI], b[3][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      const unsigned v[8] = {ra[d][i][0].x, ra[d][i][0].y, ra[d][i][0].z, ra[d][i][0].w,
+                             ra[d][i][1].x, ra[d][i][1].y, ra[d][i][1].z, ra[d][i][1].w};
+      split8(v, a[0][i], a[1][i], a[2][i]);
+    }
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) split8(rb[d][j], b[0][j], b[1][j], b[2][j]);
+    // (fences: left alone the scheduler gathers the loads of several steps in front of one wait)
+    __builtin_amdgcn_sched_barrier(0);
+    load(dc, next);
+    __builtin_amdgcn_sched_barrier(0);
+    mfmaSplit(a, b, acc, lo);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto each = [](auto f) {
+    f(std::integral_constant<int, 0>{});
+    f(std::integral_constant<int, 1>{});
+    if constexpr (D == 4) f(std::integral_constant<int, 2>{}), f(std::integral_constant<int, 3>{});
+  };
+  if (s0 < s1) {
+    loadTaps(s0);
+    each([&](auto dc) { load(dc, s0 + decltype(dc)::value); });
+#pragma unroll 1
+    for (int k = s0; k < s1; k += D) each([&](auto dc) { step(dc, k + D + decltype(dc)::value); });
+  }
+  float bad = 0.f;  // NaN as soon as one sum is not finite
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        acc[i][j][v] += lo[i][j][v];
+        bad = __builtin_fmaf(acc[i][j][v], 0.f, bad);
+      }
+  if (__any(bad != bad)) {  // the slice again in fp32
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) {
+        float16v c;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) c[v] = 0.f;
+#pragma unroll 1
+        for (int k = s0 * 8; k < s1 * 8; ++k) {
+          const float av = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wr, rowOff[i], k * 4, 0));
+          const float bv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, posOff[j], LINEAR ? k * p.tapStride : p.taps[k], 0));
+          c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
+        }
+        acc[i][j] = c;
+      }
+  }
+
+  // rows 8 * (r % 4) + 4 * (lane / 32) .. + 3 of block (r / 4 / TJ, r / 4 % TJ) at column lane % 32
+  auto finish = [&](int r, float4 v) {
+    const int row = m0 + r / (4 * TJ) * 32 + 8 * (r & 3) + 4 * grp;
+    const unsigned col = (unsigned)j0 + (r >> 2) % TJ * 32 + idx;
+    if (col >= (unsigned)p.Ncols) return;
+    int n, oh, ow;
+    splitColumn(p, g, col, n, oh, ow);
+    float *dst = p.out + (long)n * p.outImg + (long)oh * p.outSH + ow * p.outSW + (long)row * p.outRow;
+    const float vals[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (row + e < p.M) {
+        float o = vals[e] + (p.bias ? p.bias[row + e] : 0.f);
+        if (p.relu) o = o > 0.f ? o : 0.f;
+        dst[(long)e * p.outRow] = o;
+      }
+  };
+#pragma unroll
+  for (int r = 0; r < RQ; ++r) {
+    const float16v &c = acc[r / (4 * TJ)][(r >> 2) % TJ];
+    red[slice][r][lane] = make_float4(c[4 * (r & 3)], c[4 * (r & 3) + 1], c[4 * (r & 3) + 2], c[4 * (r & 3) + 3]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < RQ / 4; ++u) {  // each wave folds and stores a quarter
+    const int r = slice * (RQ / 4) + u;
+    float4 v = red[0][r][lane];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) {
+      const float4 w = red[q][r][lane];
+      v.x += w.x, v.y += w.y, v.z += w.z, v.w += w.w;
+    }
+    finish(r, v);
+  }
 }
 
 template <int WM, bool LINEAR = false>
@@ -1787,7 +1954,7 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     }
     if (store) storeTiles(nxt);
     if (load) loadTiles();
-    mfmaSplit<2>(a, b, acc, lo);
+    mfmaSplit(a, b, acc, lo);
     __syncthreads();
   };
   if (ktBegin < ktEnd) {
@@ -2155,6 +2322,7 @@ bool forceGeneric() { return g_switches.convGeneric == 1; }
 // that the last whole tiles free.
 struct FwdPlan {
   int bm, bn;          // tile shape: 128 x 128, or 64 x 256 when that wastes fewer rows (padded kernel only)
+  int direct;          // != 0: convFwdDirectKernel, tiles of 32 * direct rows and columns
   int mTiles, total, full, tail, nSplit, ktPerSplit;
   int tapEntries;      // > 0: the padded kernel applies; entries of the tap table at the start of the scratch
   long paddedFloats;   // floats of the zero-bordered copy of the images (0: no border needed, or generic kernel)
@@ -2204,8 +2372,33 @@ void planTiles(FwdPlan &pl, int M, long Ncols, int nkt, bool wideOk) {
 }
 inline long partialFloats(const FwdPlan &pl) { return pl.tail ? (long)pl.tail * pl.nSplit * BM * BN : 0; }
 
+// Whether a short call runs on convFwdDirectKernel: one launch, against workgroup tiles that would leave CUs idle or
+// have K split over workgroups, with partial tiles in memory and a second launch that folds them. Both times in us,
+// fitted to measured calls (tiled / direct): 512 -> 512 1x1 on 14x14, N = 1: 9.8 / 6.3; 256 -> 256 1x1 on 14x14, N = 8:
+// 12.8 / 7.7; 128 -> 128 3x3 on 28x28, N = 2: 20.4 / 14.6; 256 -> 64 1x1 on 56x56, N = 8: 19.5 / 15.6; 64 -> 128 1x1 on
+// 28x28, N = 16: 9.4 / 10.6; 128 -> 512 1x1 on 28x28, N = 8: 13.7 / 20.7; 256 -> 256 3x3 on 14x14, N = 1: 18.0 / 21.8.
+// 32 x 32 tiles while those are few, then 64 x 64 (fewer loads per product; the line between them: 64 -> 64 3x3 on
+// 56x56, N = 4, 784 tiles of 32 x 32: 23.9 / 20.0; 256 -> 256 1x1 on 14x14, N = 8, 392 tiles: 7.7 / 9.8).
+void planDirect(FwdPlan &pl, int M, long Ncols, int nkt) {
+  const int force = g_switches.convDirect;
+  if (force == 0) return;
+  const long tiles32 = (long)tiles(M, 32) * tiles(Ncols, 32);
+  const bool small = tiles32 <= 512;
+  if (force < 0) {
+    if (pl.total >= residentSlots(nullptr)) return;  // a workgroup tile for every CU: the tiled kernel is better at any size
+    const double tiled = 6.0 + 0.85 * pl.ktPerSplit + (pl.tail > 0 ? 5.0 + 0.02 * pl.tail * pl.nSplit : 0.0);
+    const double direct = 4.5 + 0.002 * tiles32 + std::max(0.13 * nkt, (small ? 0.65e-3 : 0.45e-3) * tiles32 * nkt);
+    if (direct >= tiled) return;
+  }
+  pl.direct = force > 0 ? force : small ? 1 : 2;
+  pl.bm = pl.bn = 32 * pl.direct;
+  pl.mTiles = (int)tiles(M, pl.bm);
+  pl.total = pl.full = pl.mTiles * (int)tiles(Ncols, pl.bn);
+  pl.tail = 0, pl.nSplit = 1, pl.ktPerSplit = nkt;
+}
+
 // wAligned: the weights start on a 16-byte boundary (else the padded kernel works on an aligned copy)
-FwdPlan planFwdImplicit(int M, int nImages, const ConvGeom &g, bool wAligned = true) {
+FwdPlan planFwdImplicit(int M, int nImages, const ConvGeom &g, bool wAligned = true, bool direct = true) {
   FwdPlan pl{};
   const int nkt = launch::ceilDiv(g.K, BK);
   const long padded = (long)nImages * g.Cin * (g.H + 2 * g.padH) * (g.W + 2 * g.padW);
@@ -2214,6 +2407,7 @@ FwdPlan planFwdImplicit(int M, int nImages, const ConvGeom &g, bool wAligned = t
   const int Kp = nkt * BK;
   const bool fast = !forceGeneric() && padded * 4 < 0x7fffffffL && (long)M * Kp * 4 < 0x7fffffffL;
   planTiles(pl, M, (long)nImages * g.L, nkt, fast);
+  if (fast && direct && g.K % BK == 0 && g.Cin % 2 == 0) planDirect(pl, M, (long)nImages * g.L, nkt);
   pl.tapEntries = fast ? Kp + 2 * BK : 0;  // spare entries: the kernel reads tap offsets up to two k-tiles ahead
   pl.paddedFloats = fast && (g.padH > 0 || g.padW > 0) ? padded : 0;
   pl.weightFloats = fast && (Kp != g.K || !wAligned) ? (long)M * Kp : 0;
@@ -2227,6 +2421,18 @@ void launchFwdKernels(hipStream_t s, const FwdPlan &pl, FwdArgs p, float *partia
   p.mTiles = pl.mTiles;
   p.bm = pl.bm, p.bn = pl.bn;
   p.full = pl.full, p.tail = pl.tail;
+  if (pl.direct) {
+    if (pl.direct == 1 && p.tapStride > 0)
+      convFwdDirectKernel<1, true><<<pl.total, dev::kBlock, 0, s>>>(p, gk);
+    else if (pl.direct == 1)
+      convFwdDirectKernel<1, false><<<pl.total, dev::kBlock, 0, s>>>(p, gk);
+    else if (p.tapStride > 0)
+      convFwdDirectKernel<2, true><<<pl.total, dev::kBlock, 0, s>>>(p, gk);
+    else
+      convFwdDirectKernel<2, false><<<pl.total, dev::kBlock, 0, s>>>(p, gk);
+    THC_HIP_CHECK(hipGetLastError());
+    return;
+  }
   if (fast) {
     // one launch: the tiles reduced by one workgroup first, then the splits of the tail tiles, which fill
     // the slots that the last whole tiles leave
@@ -2416,6 +2622,14 @@ bool convPointwise(THCState *state, const ConvGeom &g, const float *x, const flo
   const long P = (long)g.N * g.L;
   PwShape sh;
   if (g.L % 4 != 0 || g.Cout % 8 != 0 || P < 32 || !pwShape(g.Cout, g.K, &sh)) return false;
+  // The shortest forward calls (an image or two of 14x14 and smaller planes) go to the direct kernel; those with the
+  // transposed weights stay (direct needs a launch that transposes). us, this one / direct: 64 -> 64, N = 1, 56x56:
+  // 7.8 / 5.6, transposed 7.5 / 8.4; 128 -> 128: 7.2 / 6.5. The 256-row shape has a long start (14 us): on mid-sized
+  // calls it loses to the other kernels in both directions (64 -> 256, N = 1 on 56x56: 14.4 / 7.5; N = 8: 17.7 / 13.9;
+  // N = 16: 21.6 / 23.3).
+  if (g_switches.convPointwise == 1 && g_switches.convDirect < 0 &&
+      ((sh.mr == 2 && P >= 1024 && P < 40000) || (!transW && P <= 512)))
+    return false;
   // Short runs: with fewer than three chunks per workgroup the pipeline (chunk c multiplied, c + 1 in registers,
   // c + 2 in flight) never fills; chunks of half the size do better there (128 -> 128 at 28 x 28, N = 64, 7 column
   // tiles per workgroup: 28.2 -> 24.7 us, the tiled GEMM 25.8; at 56 x 56, 25 tiles per workgroup: 70 -> 76 us).
@@ -2852,9 +3066,9 @@ void convGradInput(THCState *state, const ConvGeom &g, const float *gy, const fl
     OutMap om{(long)g.Cin * g.H * g.W, g.H * g.W, 2 * g.W, 2, 1};
     int group = (int)std::min<long>(g.N, std::max<long>(1, 0x7fffffffL / 2 / t.L));
     group = (int)std::min<long>(group, std::max<long>(1, ((1L << 31) - 1 - 4096) / ((long)g.Cout * t.L * 4)));
-    FwdPlan pl = planFwdImplicit(t.Cout, std::min(group, g.N), t);
+    FwdPlan pl = planFwdImplicit(t.Cout, std::min(group, g.N), t, true, false);
     long need = pl.scratchFloats;
-    if (g.N % group != 0) need = std::max(need, planFwdImplicit(t.Cout, g.N % group, t).scratchFloats);
+    if (g.N % group != 0) need = std::max(need, planFwdImplicit(t.Cout, g.N % group, t, true, false).scratchFloats);
     const long wfFloats = ((long)g.Cout * g.K + 3) / 4 * 4;
     Temp tmp;
     float *buf = scratchFloats(state, scratchBuf, wfFloats + need, tmp, bufName);
@@ -2862,7 +3076,7 @@ void convGradInput(THCState *state, const ConvGeom &g, const float *gy, const fl
     THC_HIP_CHECK(hipGetLastError());
     for (int n0 = 0; n0 < g.N; n0 += group) {
       int cnt = std::min(group, g.N - n0);
-      if (cnt != std::min(group, g.N)) pl = planFwdImplicit(t.Cout, cnt, t);
+      if (cnt != std::min(group, g.N)) pl = planFwdImplicit(t.Cout, cnt, t, true, false);
       launchFwdImplicit(s, pl, buf + wfFloats, buf, gy + (long)n0 * g.Cout * g.L, gi + (long)n0 * g.Cin * g.H * g.W, bias,
                         t.Cout, cnt, t, false, &om);
     }

@@ -178,6 +178,7 @@ struct Switches {
   int convGeneric = 0;    // 1: first-generation convolution kernels
   int convGradInput = 0;  // 1: phase route, 2: gradient-column route, 3: few-plane kernel with run-time tap loops, 0: by shape
   int convPointwise = 1;  // 0: never the weight-stationary 1x1 kernel; n > 1: at most n workgroups per row block
+  int convDirect = -1;    // 0: never the forward kernel for short calls, 1 / 2: always, with 32 x 32 / 64 x 64 tiles, -1: by shape
 };
 extern Switches g_switches;
 

@@ -68,8 +68,12 @@ def _passes(case, x, w, gy, gyw):
 @pytest.mark.parametrize("kind", ["normal", "one-signed", "scaled", "tiny"])
 @pytest.mark.parametrize("case", CASES)
 def test_error_against_64_bit_sums(case, kind):
-    import torch
     print("case", case, kind, flush=True)
+    _check_error(case, kind)
+
+
+def _check_error(case, kind):
+    import torch
     N, Ci, Co, H, W, k, st, pad = case
     x, w, gy = _tensors(case, kind)
     dx, dw = (torch.from_numpy(v).double().requires_grad_() for v in (x, w.reshape(Co, Ci, k, k)))
@@ -85,11 +89,15 @@ def test_error_against_64_bit_sums(case, kind):
 @pytest.mark.parametrize("case", CASES)
 def test_non_finite_operands(case):
     print("case", case, flush=True)
+    _check_non_finite(case)
+
+
+def _check_non_finite(case, passes=3):
     N, Ci, Co, H, W, k, st, pad = case
     x, w, gy = _tensors(case, "normal", 6)
     w *= 1e-3
-    x[0, 1, 2, 3], x[1, 0, 4, 4], x[N - 1, Ci - 1, H - 1, W - 1], x[0, 2, H - 1, 0] = np.inf, np.nan, 3.4e38, -3.4e38
-    gy[0, 3, 1, 2], gy[1, 0, 0, 0] = -np.inf, np.nan
+    x[0, 1, 2, 3], x[1 % N, 0, 4 % H, 4], x[N - 1, Ci - 1, H - 1, W - 1], x[0, 2, H - 1, 0] = np.inf, np.nan, 3.4e38, -3.4e38
+    gy[0, 3, 1, 2], gy[1 % N, 0, 0, 0] = -np.inf, np.nan
     gyw = gy * np.float32(1e-3)          # times 3.4e38 still finite: no sum overflows in one order and not in another
     gy[N - 1, Co - 1, 2, 1] = 3.4e38
     g = (k, k, st, st, pad, pad)
@@ -97,10 +105,36 @@ def test_non_finite_operands(case):
         gw = np.zeros_like(w)
         ref = (O.convmm_updateOutput(x, w, None, *g), O.convmm_updateGradInput(x.shape, gy, w, *g),
                O.convmm_accGradParameters(x, gyw, gw, None, *g, 1.0)[0])
-    for name, got, r in zip(("output", "gradInput", "gradWeight"), _passes(case, x, w, gy, gyw), ref):
+    for name, got, r in list(zip(("output", "gradInput", "gradWeight"), _passes(case, x, w, gy, gyw), ref))[:passes]:
         print(name)
         assert np.array_equal(np.isnan(got), np.isnan(r)) and np.array_equal(np.isposinf(got), np.isposinf(r))
         assert np.array_equal(np.isneginf(got), np.isneginf(r))
         fine = np.isfinite(r)
         # relative to the largest term: 3.4e38 times a weight
         np.testing.assert_allclose(got[fine], r[fine], rtol=1e-5, atol=max(1e-4, 1e-6 * np.abs(r[fine], dtype=np.float64).max()))
+
+
+# ---- the kernel for short calls: every tile shape, ragged rows and columns, fewer k-steps than waves, uneven slices ----
+DIRECT = [
+    (1, 16, 8, 5, 5, 1, 1, 0),       # one k-step: three of the four waves have none
+    (1, 32, 40, 7, 7, 1, 1, 0),
+    (1, 512, 130, 7, 7, 1, 1, 0),
+    (2, 80, 33, 9, 8, 1, 1, 0),      # five k-steps
+    (1, 16, 65, 13, 11, 3, 1, 1),
+    (3, 48, 24, 10, 9, 3, 2, 1),
+    (2, 32, 64, 9, 9, 5, 1, 0),
+    (1, 512, 512, 14, 14, 1, 1, 0),
+]
+
+
+@pytest.mark.parametrize("shape", ["1", "2", None])
+@pytest.mark.parametrize("case", DIRECT)
+def test_short_calls(case, shape):
+    print("case", case, shape, flush=True)
+    cunn_amd.set_switch("THCUNN_CONV_DIRECT", shape)
+    try:
+        for kind in ("normal", "one-signed", "tiny"):
+            _check_error(case, kind)
+        _check_non_finite(case, passes=2)    # forward and gradInput
+    finally:
+        cunn_amd.set_switch("THCUNN_CONV_DIRECT", None)
