@@ -82,6 +82,7 @@ class _Base:
         self._lib = _lib.load()
         st = state()
         self._h = handle if handle is not None else getattr(self._lib, self._prefix + "_new")(st)
+        self._as_parameter_ = self._h   # what ctypes passes when the tensor is an argument
         self._keep = keepalive
 
     # -- construction -------------------------------------------------------
@@ -158,7 +159,7 @@ class _Base:
                 getattr(self._lib, self._prefix + "_free")(_state, self._h)
         except Exception:
             pass
-        self._h = None
+        self._h = self._as_parameter_ = None
 
 
 class CudaTensor(_Base):

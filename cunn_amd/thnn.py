@@ -4,18 +4,8 @@ THCState and forwards the remaining arguments unchanged. Tensor arguments are
 `CudaTensor` / `CudaLongTensor` handles or ``None`` for ``[OPTIONAL]`` ones."""
 from __future__ import annotations
 
-import ctypes as C
-
 from . import _lib
-from .tensor import _Base, check, state
-
-
-def _arg(a):
-    if a is None:
-        return None
-    if isinstance(a, _Base):
-        return a.handle
-    return a
+from .tensor import _pending, check, state
 
 
 class _Namespace:
@@ -31,9 +21,11 @@ class _Namespace:
                 raise AttributeError(f"THNN has no function {name!r}")
             cfn = getattr(_lib.load(), "THNN_Cuda" + name)
 
+            # the tensors convert themselves (_Base._as_parameter_): the call costs the binder no loop over the arguments
             def fn(*args, _cfn=cfn):
-                _cfn(state(), *[_arg(a) for a in args])
-                check()
+                _cfn(state(), *args)
+                if _pending:
+                    check()
 
             fn.__name__ = name
             self._fns[name] = fn
