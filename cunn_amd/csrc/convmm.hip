@@ -897,37 +897,6 @@ convFwdImplicitKernel(FwdArgs p, ConvGeom g) {
   fwdEpilogue(p, g, acc, blockIdx.x, blockIdx.y, m0, j0, wm, wn, grp, idx);
 }
 
-// One half of a k-tile for one wave: 4 ds_read_b128 (two k-groups... one per lane group) and 16 MFMAs.
-// aSrc / bSrc point at the lane's operands of k-group (lane / 32) in buffer 0; OA / OB are the float4
-// offsets of the buffer and super-step, compile-time so that they fold into the LDS instruction.
-template <int OA, int OB>
-__device__ __forceinline__ void mfmaHalf(const float4 *aSrc, const float4 *bSrc, float16v (&acc)[2][2]) {
-  const float4 a0 = aSrc[OA], a1 = aSrc[OA + 32];
-  const float4 b0 = bSrc[OB], b1 = bSrc[OB + 32];
-  const float av0[4] = {a0.x, a0.y, a0.z, a0.w}, av1[4] = {a1.x, a1.y, a1.z, a1.w};
-  const float bv0[4] = {b0.x, b0.y, b0.z, b0.w}, bv1[4] = {b1.x, b1.y, b1.z, b1.w};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(av0[j], bv0[j], acc[0][0], 0, 0, 0);
-    acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av0[j], bv1[j], acc[0][1], 0, 0, 0);
-    acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(av1[j], bv0[j], acc[1][0], 0, 0, 0);
-    acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av1[j], bv1[j], acc[1][1], 0, 0, 0);
-  }
-}
-// the same for a wave that multiplies 32 rows: 3 ds_read_b128 and 8 MFMAs
-template <int OA, int OB>
-__device__ __forceinline__ void mfmaHalf(const float4 *aSrc, const float4 *bSrc, float16v (&acc)[1][2]) {
-  const float4 a0 = aSrc[OA];
-  const float4 b0 = bSrc[OB], b1 = bSrc[OB + 32];
-  const float av0[4] = {a0.x, a0.y, a0.z, a0.w};
-  const float bv0[4] = {b0.x, b0.y, b0.z, b0.w}, bv1[4] = {b1.x, b1.y, b1.z, b1.w};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(av0[j], bv0[j], acc[0][0], 0, 0, 0);
-    acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av0[j], bv1[j], acc[0][1], 0, 0, 0);
-  }
-}
-
 // ---- fp32 products on the bf16 matrix pipe ------------------------------------------------------
 // A float is the exact sum of three bf16 values h + m + l (8 significant bits each, every remainder exact), and the
 // product of two bf16 values is exact in fp32. x * w is computed as the six products hh + hm + mh + mm + hl + lh; the
@@ -1523,6 +1492,7 @@ fwdTailFixupBatchKernel(FwdBatch b) {
 // 16 consecutive lanes gather 16 consecutive positions (64-byte runs of x).
 // L16: L % 16 == 0 - a k-tile never crosses an image, so the gradOutput offsets are a
 // fixed VGPR part plus a scalar part.
+constexpr int kSmallPositions = 64;  // positions of a k-tile of the small tiles (BK of the large ones)
 struct GradWeightArgs {
   const float *gy;  // (N, M, L)
   const float *x;   // (N, Cin, H, W) of g: images with their zero border
@@ -1530,247 +1500,210 @@ struct GradWeightArgs {
   float *biasPartial;  // (splits, M) row sums of gy per split, or null: the bias gradient comes out of the same pass
   int M, Ncols;     // Cout, K
   int mTiles, nTiles;
-  int totalKt, ktPerSplit;  // k-tiles of BK positions over the N*L positions; per split
+  int totalKt, ktPerSplit;  // k-tiles of BK (small tiles: kSmallPositions) positions over the N*L positions; per split
   int gyBytes, xBytes;      // < 2^31
   unsigned magicOW;
   unsigned magicKK, magicKW;  // reciprocals of kH * kW and kW (dev::magicOf)
   int Lvalid;               // positions of an image (g.L may count the padding of the gradOutput rows)
 };
 
-// WM = 2: 128 x 128 tiles of gradWeight (Cout x K), WM = 1: 64 x 256 tiles (as in the forward kernel).
-// WM = 0: 64 x 64 tiles for small gradWeights (first layers, narrow 1x1 convolutions), where the large tiles
-// would spend most of their multiplications on padding: the four waves all own the whole tile and take one
-// position group (4 of the 16 positions) of every k-tile each, i.e. a wave is a split of its own - it stores
-// its partial under split index 4 * split + wave and the fold adds them like any other splits.
-template <int OA, int OB, int TI, int TJ>
-__device__ __forceinline__ void mfmaGroupPair(const float *aSrc, const float *bSrc, float16v (&acc)[TI][TJ]) {
-  // lanes 0-31 hold position OA / OB of the group, lanes 32-63 the next one (aSrc / bSrc already point there)
-  float a[TI], b[TJ];
-#pragma unroll
-  for (int i = 0; i < TI; ++i) a[i] = aSrc[OA + i * 32 * 4];
-#pragma unroll
-  for (int j = 0; j < TJ; ++j) b[j] = bSrc[OB + j * 32 * 4];
-#pragma unroll
-  for (int i = 0; i < TI; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-}
-
-// (TI, TJ): 32-row and 32-column blocks of a small tile (WMODE = 0 only): 64 x 64, 32 x 64, 32 x 128, 64 x 32 ...
-// B4: 4 consecutive positions of a column are 4 consecutive floats of the image (unit stride along the row, and the
-// 4 positions never straddle two output rows - or the rows follow each other without a gap): a lane then fetches
-// one such group for each of its columns with one 16-byte load (any 4-byte alignment) and parks it with one
-// ds_write_b128, a quarter of the instructions of the element-wise gather.
-template <bool L16, int WMODE, int TI = 2, int TJ = 2, bool B4 = false>
-__global__ void __launch_bounds__(dev::kBlock, 3)
-convGradWeightKernel(GradWeightArgs p, ConvGeom g) {
-  constexpr bool TINY = WMODE == 0;
-  static_assert(TINY || (TI == 2 && TJ == 2), "block counts are a parameter of the small tiles only");
-  static_assert(!(TINY && B4), "the small tiles gather element by element");
-  constexpr int WM = TINY ? 1 : WMODE;  // loader layout: 64 rows as in the 64 x 256 shape
-  constexpr int TBM = TINY ? 32 * TI : 64 * WM, TBN = TINY ? 32 * TJ : 256 / WM;
-  constexpr int AP = TBM + 8;   // float4 per position-group row of As
-  constexpr int GP = TBN + 4;   // of Bs: the 4 groups of a wave's scalar stores hit disjoint banks
-  constexpr int NB = B4 ? TBN / 64 : TBN / 16;  // columns a lane gathers per k-tile
-  constexpr int CS = B4 ? 64 : 16;              // distance between a lane's columns
-  __shared__ float4 As[2][BK / 4][AP];
-  __shared__ float4 Bs[2][BK / 4][GP];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = WM == 2 ? wave >> 1 : 0, wn = TINY ? 0 : (WM == 2 ? wave & 1 : wave);
-  // workgroups that reduce the same positions (one split) are neighbours in the remapped order: same XCD, same L2
+// Small gradWeights (first layers, narrow 1x1 convolutions), where the large tiles would spend most of their
+// multiplications on padding: tiles of 32 TI x 32 TJ. A k-tile is 64 positions, every wave multiplies 16 of them with the
+// whole tile, and the four sums are added through LDS at the end. Split operands as in the large tiles. Loads: 16 lanes
+// fetch 256 consecutive bytes of a gradOutput row with 16-byte loads; a wave gathers one column of the image at 64
+// consecutive positions, the tap being a scalar, and transposes 4 x 4 elements inside quads so that LDS holds whole groups
+// of positions. One LDS buffer and registers for the next k-tile: two to four workgroups per CU cover the barriers.
+// Bound by the vector ALU (24 elements split per lane against 12 matrix instructions of a wave for 64 x 32).
+template <int TI, int TJ>
+__global__ void __launch_bounds__(dev::kBlock, TI * TJ >= 4 ? 2 : 3)
+convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
+  constexpr int TBM = 32 * TI, TBN = 32 * TJ, KP = kSmallPositions;
+  constexpr int AP = TBM + 4, BP = TBN + 4;   // a row of 16-byte groups; +4: the 8 position groups of a store spread over the banks
+  constexpr int NA = TBM / 16, NC = TBN / 4;  // 16-byte gradOutput loads and gathered columns of a lane per k-tile
+  constexpr int RQ = TI * TJ * 4;             // groups of 4 accumulator registers
+  constexpr int TILE = 3 * 8 * (AP + BP), FOLD = 4 * RQ * dev::kWave;
+  __shared__ u32x4 lds[TILE > FOLD ? TILE : FOLD];  // [part][group of 8 positions][row], then [..][column]; at the end the sums
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int tilesPerSplit = p.mTiles * p.nTiles;
-  const int bid = dev::xcdRemap(blockIdx.x, gridDim.x);
+  const int bid = dev::xcdRemap(blockIdx.x, gridDim.x);  // the tiles of one split are neighbours: same XCD, same L2
   const int split = bid / tilesPerSplit, tileIdx = bid - split * tilesPerSplit;
   const int mTile = tileIdx % p.mTiles, nTile = tileIdx / p.mTiles;
   const int m0 = mTile * TBM, j0 = nTile * TBN;
   const int ktBegin = split * p.ktPerSplit;
   const int ktEnd = min(p.totalKt, ktBegin + p.ktPerSplit);
-  const int kOob = 0x7fffffff;
 
-  float16v acc[TI][TJ];
+  // (n, l) of a position; positions past the batch have n == N
+  auto locate = [&](unsigned r, int &n, int &l) {
+    n = min((int)(r / (unsigned)g.L), g.N), l = (int)(r - (unsigned)n * (unsigned)g.L);
+  };
+  auto advance = [&](int &n, int &l) {
+    for (l += KP; l >= g.L && n < g.N; ++n) l -= g.L;
+  };
+  // ---- gradOutput: rows (t >> 4) + 16 i, positions 4 * (t & 15) .. + 3 of the k-tile
+  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc((void *)p.gy, 0, p.gyBytes, 0x00020000);
+  const int imgStrideA = p.M * g.L * 4;
+  int rowOffA[NA], nA, lA;
+#pragma unroll
+  for (int i = 0; i < NA; ++i) rowOffA[i] = min(m0 + (t >> 4) + 16 * i, p.M - 1) * g.L * 4;  // rows past M: dropped in the end
+  locate((unsigned)ktBegin * KP + (t & 15) * 4, nA, lA);
+  // ---- image: position `lane` of the k-tile, columns NC * wave .. + NC - 1
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, p.xBytes, 0x00020000);
+  auto columnOffset = [&](int col) {  // byte offset of a column's tap; columns past K are dropped in the end
+    const int k = min(col, p.Ncols - 1), KK = g.kH * g.kW;
+    const int c = dev::fastDiv(k, p.magicKK), rem = k - c * KK;
+    const int kh = dev::fastDiv(rem, p.magicKW), kw = rem - kh * g.kW;
+    return ((c * g.H + kh * g.dilH) * g.W + kw * g.dilW) * 4;
+  };
+  int tap[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) tap[i] = __builtin_amdgcn_readfirstlane(columnOffset(j0 + wave * NC + i));
+  const int imgStrideB = g.Cin * g.H * g.W * 4;
+  int nB, lB;
+  locate((unsigned)ktBegin * KP + lane, nB, lB);
+  // byte offset of a position; past the batch, and past the image's last position (gradOutput rows padded to a multiple
+  // of 4, zeros there): out of range, reads as 0
+  auto positionOffset = [&](int n, int l) {
+    const int oh = dev::fastDiv(l, p.magicOW), ow = l - oh * g.oW;
+    return n < g.N && l < p.Lvalid ? n * imgStrideB + (oh * g.dH * g.W + ow * g.dW) * 4 : 0x7fffffff;
+  };
+
+  u32x4 ra[NA];
+  unsigned rb[NC];
+  auto loadTiles = [&]() {
+    const int offA = nA < g.N ? nA * imgStrideA + lA * 4 : 0x7fffffff;
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      ra[i] = __builtin_amdgcn_raw_buffer_load_b128(gr, (int)((unsigned)offA + (unsigned)rowOffA[i]), 0, 0);
+    const int offB = positionOffset(nB, lB);
+#pragma unroll
+    for (int i = 0; i < NC; ++i) rb[i] = __builtin_amdgcn_raw_buffer_load_b32(xr, offB, tap[i], 0);
+    advance(nA, lA);
+    advance(nB, lB);
+  };
+  u32x2 *aDst = reinterpret_cast<u32x2 *>(lds + ((t & 15) >> 1) * AP + (t >> 4)) + (t & 1);
+  u32x2 *bDst = reinterpret_cast<u32x2 *>(lds + 24 * AP + (lane >> 3) * BP + wave * NC + (lane & 3)) + ((lane >> 2) & 1);
+  const bool rowSums = nTile == 0 && p.biasPartial != nullptr;  // the bias gradient rides along
+  float rowSum[NA] = {};
+  auto split4 = [](const u32x4 &v, u32x2 (&part)[3]) {
+    unsigned h[2], m[2], l[2];
+    splitPair(v.x, v.y, h[0], m[0], l[0]);
+    splitPair(v.z, v.w, h[1], m[1], l[1]);
+    part[0] = u32x2{h[0], h[1]}, part[1] = u32x2{m[0], m[1]}, part[2] = u32x2{l[0], l[1]};
+  };
+  auto storeTiles = [&]() {
+    u32x2 part[3];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      split4(ra[i], part);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) aDst[2 * (s * 8 * AP + 16 * i)] = part[s];
+      if (rowSums) {
+        const unsigned ex = ra[i].x, ey = ra[i].y, ez = ra[i].z, ew = ra[i].w;
+        rowSum[i] += (__uint_as_float(ex) + __uint_as_float(ey)) + (__uint_as_float(ez) + __uint_as_float(ew));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NC / 4; ++i) {
+      split4(dev::quadTranspose(rb[4 * i], rb[4 * i + 1], rb[4 * i + 2], rb[4 * i + 3]), part);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) bDst[2 * (s * 8 * BP + 4 * i)] = part[s];
+    }
+  };
+  const int grp = lane >> 5, idx = lane & 31;
+  const u32x4 *aSrc = lds + (2 * wave + grp) * AP + idx, *bSrc = lds + 24 * AP + (2 * wave + grp) * BP + idx;
+
+  float16v acc[TI][TJ], lo[TI][TJ];
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
     for (int j = 0; j < TJ; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-  // ---- A loader. WM = 2: row o = t >> 1, positions 8 * (t & 1) .. + 7 of the k-tile as two float4;
-  //                WM = 1: row o = t >> 2, positions 4 * (t & 3) .. + 3 as one float4 (32-row tiles: both halves
-  //                of the workgroup fetch and park the same rows)
-  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc((void *)p.gy, 0, p.gyBytes, 0x00020000);
-  const int rowA = WM == 2 ? t >> 1 : (t >> 2) & (TBM - 1);
-  const int pgA = WM == 2 ? (t & 1) * 2 : t & 3;  // first position group (of 4 positions) of the lane
-  const int rowOffA = min(m0 + rowA, p.M - 1) * g.L * 4;  // rows past M are clamped and dropped in the epilogue
-  const int imgStrideA = p.M * g.L * 4;
-  int nA, lA;  // L16: scalar image and position of the k-tile; else: of this lane's first group
-  {
-    const unsigned r = (unsigned)ktBegin * BK + (L16 ? 0 : pgA * 4);  // N * L < 2^31
-    nA = (int)(r / (unsigned)g.L);
-    lA = (int)(r - (unsigned)nA * (unsigned)g.L);
-  }
-  // ---- B loader: position t & 15 of the k-tile, columns (t >> 4) + 16 i
-  //      (B4: positions 4 * (t & 3) .. + 3, columns (t >> 2) + 64 i)
-  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, p.xBytes, 0x00020000);
-  const int rB = B4 ? (t & 3) * 4 : t & 15, cB = B4 ? t >> 2 : t >> 4;
-  int tapOff[NB];
-  {
-    const int KK = g.kH * g.kW;
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int k = min(j0 + cB + CS * i, p.Ncols - 1);  // columns past K are dropped in the epilogue
-      const int c = dev::fastDiv(k, p.magicKK), rem = k - c * KK;
-      const int kh = dev::fastDiv(rem, p.magicKW), kw = rem - kh * g.kW;
-      tapOff[i] = ((c * g.H + kh * g.dilH) * g.W + kw * g.dilW) * 4;
-    }
-  }
-  const int imgStrideB = g.Cin * g.H * g.W * 4;
-  const int rowStepB = g.dH * g.W * 4, colStepB = g.dW * 4;
-  int lB, nOffB;  // position inside the image, byte offset of the image (>= xBytes past the batch: loads return 0)
-  {
-    const unsigned r = (unsigned)ktBegin * BK + rB;
-    const int n = (int)(r / (unsigned)g.L);
-    lB = (int)(r - (unsigned)n * (unsigned)g.L);
-    nOffB = n * imgStrideB;
-  }
-
-  u32x4 ra[WM];
-  unsigned rb[B4 ? 1 : NB];
-  u32x4 rb4[B4 ? NB : 1];
-  // loads the k-tile the position counters stand on, then advances them by BK (L >= BK: one wrap at most)
-  auto loadTiles = [&]() {
-    if constexpr (L16) {
-      // N*L is a multiple of BK here, so every k-tile lies inside the batch (the scalar offset is not range-checked)
-      const int so = __builtin_amdgcn_readfirstlane(nA * imgStrideA + lA * 4);
-#pragma unroll
-      for (int i = 0; i < WM; ++i) ra[i] = __builtin_amdgcn_raw_buffer_load_b128(gr, rowOffA + pgA * 16 + 16 * i, so, 0);
-      lA += BK;
-      if (lA >= g.L) lA -= g.L, ++nA;
-    } else {
-      const int o0 = nA < g.N ? nA * imgStrideA + rowOffA + lA * 4 : kOob;
-      ra[0] = __builtin_amdgcn_raw_buffer_load_b128(gr, o0, 0, 0);
-      if constexpr (WM == 2) {
-        int n1 = nA, l1 = lA + 4;
-        if (l1 >= g.L) l1 -= g.L, ++n1;
-        const int o1 = n1 < g.N ? n1 * imgStrideA + rowOffA + l1 * 4 : kOob;
-        ra[WM - 1] = __builtin_amdgcn_raw_buffer_load_b128(gr, o1, 0, 0);
-      }
-      lA += BK;
-      if (lA >= g.L) lA -= g.L, ++nA;
-    }
-    {
-      // (positions behind the image's last one exist when the gradOutput rows were padded to a multiple of 4:
-      // their gradOutput is zero, they read the image at position 0)
-      const int lq = lB < p.Lvalid ? lB : 0;
-      const int oh = dev::fastDiv(lq, p.magicOW), ow = lq - oh * g.oW;
-      const int posOff = nOffB + oh * rowStepB + ow * colStepB;
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        if constexpr (B4)
-          rb4[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)((unsigned)posOff + (unsigned)tapOff[i]), 0, 0);
-        else
-          rb[i] = __builtin_amdgcn_raw_buffer_load_b32(xr, (int)((unsigned)posOff + (unsigned)tapOff[i]), 0, 0);
-      }
-      lB += BK;
-      if (lB >= g.L) lB -= g.L, nOffB += imgStrideB;
-    }
-  };
-  u32x4 *aDst = reinterpret_cast<u32x4 *>(&As[0][pgA][rowA]);
-  unsigned *bDst = reinterpret_cast<unsigned *>(&Bs[0][rB >> 2][cB]) + (rB & 3);
-  u32x4 *bDst4 = reinterpret_cast<u32x4 *>(&Bs[0][rB >> 2][cB]);
-  constexpr int BUFA = (BK / 4) * AP, BUFB = (BK / 4) * GP;  // float4 per LDS buffer
-  // The workgroups of the first column tile also sum the gradOutput elements they pass on (each element of a
-  // row is loaded by exactly one lane of exactly one of them): the bias gradient without a second pass over gy.
-  const bool rowSums = nTile == 0 && p.biasPartial != nullptr;
-  float rowSum = 0.f;
-  auto storeTiles = [&](auto bufc) {
-    constexpr int buf = decltype(bufc)::value;
-#pragma unroll
-    for (int i = 0; i < WM; ++i) aDst[buf * BUFA + i * AP] = ra[i];
-    if (rowSums) {
-#pragma unroll
-      for (int i = 0; i < WM; ++i)
-      {
-        // (element by element: a bit cast applied to a vector element expression reads element 0 here)
-        const unsigned ex = ra[i].x, ey = ra[i].y, ez = ra[i].z, ew = ra[i].w;
-        rowSum += (__uint_as_float(ex) + __uint_as_float(ey)) + (__uint_as_float(ez) + __uint_as_float(ew));
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      if constexpr (B4)
-        bDst4[buf * BUFB + 64 * i] = rb4[i];
-      else
-        bDst[buf * BUFB * 4 + 64 * i] = rb[i];  // column + 16 = 16 float4 further
-    }
-  };
-  const int grp = lane >> 5, idx = lane & 31;
-  const float4 *aSrc = &As[0][grp][wm * 64 + idx];
-  const float4 *bSrc = &Bs[0][grp][wn * 64 + idx];
-  // small tiles: this wave's position group, element grp (then grp + 2) of its float4
-  const float *aTiny = reinterpret_cast<const float *>(&As[0][wave][idx]) + grp;
-  const float *bTiny = reinterpret_cast<const float *>(&Bs[0][wave][idx]) + grp;
-  using Buf0 = std::integral_constant<int, 0>;
-  using Buf1 = std::integral_constant<int, 1>;
-
-  // same software pipeline as the forward kernel: tile kt in LDS, kt + 1 in registers, kt + 2 requested
-  auto step = [&](auto cur, auto nxt, bool store, bool load) {
-    constexpr int C = decltype(cur)::value;
-    if constexpr (TINY)
-      mfmaGroupPair<C * BUFA * 4, C * BUFB * 4, TI, TJ>(aTiny, bTiny, acc);
-    else
-      mfmaHalf<C * BUFA, C * BUFB>(aSrc, bSrc, acc);
-    __builtin_amdgcn_sched_barrier(0);
-    if (store) storeTiles(nxt);
-    if (load) loadTiles();
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (TINY)
-      mfmaGroupPair<C * BUFA * 4 + 2, C * BUFB * 4 + 2, TI, TJ>(aTiny, bTiny, acc);
-    else
-      mfmaHalf<C * BUFA + 2 * AP, C * BUFB + 2 * GP>(aSrc, bSrc, acc);
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = lo[i][j][v] = 0.f;
+  loadTiles();
+#pragma unroll 1
+  for (int kt = ktBegin; kt < ktEnd; ++kt) {
+    storeTiles();
     __syncthreads();
-  };
-  if (ktBegin < ktEnd) {
-    loadTiles();
-    storeTiles(Buf0{});
-    if (ktBegin + 1 < ktEnd) loadTiles();
-    __syncthreads();
-    int kt = ktBegin;
-    for (; kt + 3 < ktEnd; kt += 2) {  // tile kt sits in buffer 0, tile kt + 1 in registers
-      step(Buf0{}, Buf1{}, true, true);
-      step(Buf1{}, Buf0{}, true, true);
+    u32x4 a[3][TI], b[3][TJ];
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i) a[s][i] = aSrc[s * 8 * AP + 32 * i];
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) b[s][j] = bSrc[s * 8 * BP + 32 * j];
     }
-    // one to three tiles left
-    step(Buf0{}, Buf1{}, kt + 1 < ktEnd, kt + 2 < ktEnd);
-    if (kt + 1 < ktEnd) step(Buf1{}, Buf0{}, kt + 2 < ktEnd, false);
-    if (kt + 2 < ktEnd) step(Buf0{}, Buf1{}, false, false);
+    loadTiles();  // (one k-tile past the end at the last: inside the tensors or out of range)
+    mfmaSplit(a, b, acc, lo);
+    __syncthreads();
   }
 
-  // lane holds column (lane & 31), rows 8*(v/4) + 4*(lane/32) + v%4 of each 32x32 tile
-  float *dst = p.partial + (long)(TINY ? split * 4 + wave : split) * p.M * p.Ncols;
+  float bad = 0.f;  // NaN as soon as one sum is not finite
 #pragma unroll
-  for (int tj = 0; tj < TJ; ++tj) {
-    const int col = j0 + wn * 64 + tj * 32 + idx;
-    if (col >= p.Ncols) continue;
+  for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int ti = 0; ti < TI; ++ti)
+    for (int j = 0; j < TJ; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm * 64 + ti * 32 + 8 * (v >> 2) + grp * 4 + (v & 3);
-        if (row < p.M) dst[(long)row * p.Ncols + col] = acc[ti][tj][v];
+        acc[i][j][v] += lo[i][j][v];
+        bad = __builtin_fmaf(acc[i][j][v], 0.f, bad);
       }
+  if (__any(bad != bad)) {  // the wave's positions again with the fp32 instruction, straight from memory
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+      const unsigned off = (unsigned)columnOffset(j0 + j * 32 + idx);
+#pragma unroll
+      for (int i = 0; i < TI; ++i) {
+        const unsigned rOff = (unsigned)(min(m0 + i * 32 + idx, p.M - 1) * g.L * 4);
+        float16v c;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) c[v] = 0.f;
+#pragma unroll 1
+        for (int kt = ktBegin; kt < ktEnd; ++kt)
+#pragma unroll 1
+          for (int q = 0; q < 16; q += 2) {
+            int n, l;
+            locate((unsigned)kt * KP + wave * 16 + q + grp, n, l);
+            const unsigned at = n < g.N ? (unsigned)(n * imgStrideA + l * 4) : 0x7fffffffu;
+            const float av = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gr, (int)(at + rOff), 0, 0));
+            const float bv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, (int)((unsigned)positionOffset(n, l) + off), 0, 0));
+            c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
+          }
+        acc[i][j] = c;
+      }
+    }
+  }
+
+  // the four waves' sums; lane holds column (lane & 31), rows 8 * (v / 4) + 4 * (lane / 32) + v % 4 of each block
+  float4 *fold = reinterpret_cast<float4 *>(lds);
+#pragma unroll
+  for (int r = 0; r < RQ; ++r) {
+    const float16v &c = acc[r / (4 * TJ)][(r >> 2) % TJ];
+    fold[(wave * RQ + r) * dev::kWave + lane] = make_float4(c[4 * (r & 3)], c[4 * (r & 3) + 1], c[4 * (r & 3) + 2], c[4 * (r & 3) + 3]);
+  }
+  __syncthreads();
+  float *dst = p.partial + (long)split * p.M * p.Ncols;
+#pragma unroll
+  for (int u = 0; u < RQ / 4; ++u) {  // each wave folds and stores a quarter
+    const int r = wave * (RQ / 4) + u;
+    float4 v = fold[r * dev::kWave + lane];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) {
+      const float4 w = fold[(q * RQ + r) * dev::kWave + lane];
+      v.x += w.x, v.y += w.y, v.z += w.z, v.w += w.w;
+    }
+    const int row = m0 + r / (4 * TJ) * 32 + 8 * (r & 3) + 4 * grp, col = j0 + (r >> 2) % TJ * 32 + idx;
+    const float vals[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (row + e < p.M && col < p.Ncols) dst[(long)(row + e) * p.Ncols + col] = vals[e];
   }
   if (rowSums) {
-    // the 2 (WM = 2) or 4 (WM = 1) lanes that loaded parts of a row are neighbours inside a quad
-    rowSum = dev::dppAdd<0xB1>(rowSum);
-    if (WM == 1) rowSum = dev::dppAdd<0x4E>(rowSum);
-    if ((t & (WM == 2 ? 1 : 3)) == 0 && m0 + rowA < p.M && (t >> 2) < TBM) {
-      if (TINY) {  // four partial slots per workgroup: the row sums go to the first, the others add nothing
-        float *bp = p.biasPartial + (long)split * 4 * p.M + m0 + rowA;
-        bp[0] = rowSum, bp[p.M] = 0.f, bp[2 * (long)p.M] = 0.f, bp[3 * (long)p.M] = 0.f;
-      } else {
-        p.biasPartial[(long)split * p.M + m0 + rowA] = rowSum;
-      }
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      float v = rowSum[i];  // the 16 lanes that loaded parts of a row
+      v = dev::dppAdd<0xB1>(v), v = dev::dppAdd<0x4E>(v), v = dev::dppAdd<0x141>(v), v = dev::dppAdd<0x140>(v);
+      const int row = m0 + (t >> 4) + 16 * i;
+      if ((t & 15) == 0 && row < p.M) p.biasPartial[(long)split * p.M + row] = v;
     }
   }
 }
@@ -1845,11 +1778,10 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     nOffB = n * imgStrideB;
   }
   // byte offset of position l of the image at nOff (positions behind the image's last one exist when the gradOutput
-  // rows were padded to a multiple of 4: their gradOutput is zero, they read the image at position 0)
+  // rows were padded to a multiple of 4: zeros in gradOutput, and out of range here, which reads as 0 too)
   auto positionOffset = [&](int l, int nOff) {
-    const int lq = l < p.Lvalid ? l : 0;
-    const int oh = dev::fastDiv(lq, p.magicOW), ow = lq - oh * g.oW;
-    return nOff + oh * rowStepB + ow * colStepB;
+    const int oh = dev::fastDiv(l, p.magicOW), ow = l - oh * g.oW;
+    return l < p.Lvalid ? nOff + oh * rowStepB + ow * colStepB : kOob;
   };
 
   u32x4 ra[WM];
@@ -3200,7 +3132,6 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   const bool padGy = !forceGeneric() && (g.L % 4 != 0 || !launch::aligned16(gy)) && Lp >= BK;
   const int Lk = padGy ? Lp : g.L;  // positions per image as the kernel sees them
   if ((long)g.N * Lk >= 0x7fffffffL) error("spatial convolution: batch too large");
-  const int totalKt = launch::ceilDiv(g.N * Lk, BK);
   const int HpX = g.H + 2 * g.padH;
   // second-generation kernel: gradOutput rows loadable as float4 groups, 32-bit byte offsets into both operands
   const bool bordered = g.padH > 0 || g.padW > 0;
@@ -3212,17 +3143,20 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   const bool l16 = Lk % BK == 0;
   // tile shape: 64 x 256 where it covers gradWeight (Cout x K) with less padding than 128 x 128
   const bool wide = fast && tiles(g.Cout, 64) * 64 * tiles(g.K, 256) * 256 < tiles(g.Cout, BM) * BM * tiles(g.K, BN) * BN;
-  // Small tiles (the waves of a workgroup split the positions instead of the tile; blocks of 32 rows x 32 columns:
-  // 1x1, 1x2, 1x4, 2x1, 2x2) where the large shapes would mostly multiply padding. The shape is the one with
-  // the least tiles x cost per tile and k-tile; the costs are measured (first layers, 32- and 64-plane layers at
-  // 56x56 ... 149x149): the gather of the image patch weighs more than the matrix instructions, so a tile is not
-  // cheaper in proportion to its area.
+  // 16-byte gathers of the image: unit stride along a row, and groups of 4 positions that stay inside an output row
+  // (or output rows that follow each other in the image without a gap: kW = 1, no padding, unit stride down too)
+  const bool b4 = fast && !padGy && g.dW == 1 && (g.oW % 4 == 0 || (g.dH == 1 && g.W + 2 * g.padW == g.oW));
+  // Small tiles (32 x 32 blocks: 1x1, 1x2, 2x1, 2x2) where the large shapes would mostly multiply padding. The shape is
+  // the one with the least tiles x cost of a tile per position, in proportion to measured times: 64 x 147 over
+  // 32 x 112 x 112 positions, stride 2 (us, without the bordered copy): 10 tiles of 1x1 105, 6 of 1x2 107, 5 of 2x1 83,
+  // 3 of 2x2 80, one of 64 x 256 86; 64 x 576 over 32 x 56 x 56, stride 1: 86, 72, 72, 56, 51 (16-byte gathers). The
+  // first took 116 with the fp32 instruction (2x1), the second 81 (128 x 128).
   struct Shape {
     int ti, tj, cost;
   };
-  static const Shape kSmall[] = {{2, 2, 88}, {1, 4, 90}, {1, 2, 50}, {2, 1, 50}, {1, 1, 33}};
-  const int kBigCost = 260;  // a 128 x 128 or 64 x 256 tile
-  long bestCost = std::min(tiles(g.Cout, 64) * tiles(g.K, 256), tiles(g.Cout, BM) * tiles(g.K, BN)) * (long)kBigCost;
+  static const Shape kSmall[] = {{2, 2, 85}, {1, 2, 55}, {2, 1, 53}, {1, 1, 33}};
+  const int bigCost = b4 ? 240 : 270;  // a 128 x 128 or 64 x 256 tile
+  long bestCost = std::min(tiles(g.Cout, 64) * tiles(g.K, 256), tiles(g.Cout, BM) * tiles(g.K, BN)) * (long)bigCost;
   int tI = 0, tJ = 0;
   if (fast)
     for (const Shape &sh : kSmall) {
@@ -3231,41 +3165,29 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
     }
   const bool tiny = tI > 0;
   const int mT = (int)tiles(g.Cout, tiny ? 32 * tI : wide ? 64 : BM), nT = (int)tiles(g.K, tiny ? 32 * tJ : wide ? 256 : BN);
-  struct TinyKernel {
+  struct Kernel {
     const void *fn;
     void (*launch)(dim3, hipStream_t, const GradWeightArgs &, const ConvGeom &);
   };
-  auto tinyKernel = [&](auto l16c, auto tic, auto tjc) {
-    constexpr bool L = decltype(l16c)::value;
+  auto smallKernel = [](auto tic, auto tjc) {
     constexpr int I = decltype(tic)::value, J = decltype(tjc)::value;
-    return TinyKernel{(const void *)convGradWeightKernel<L, 0, I, J>,
-                      [](dim3 grid, hipStream_t st, const GradWeightArgs &q, const ConvGeom &gk) {
-                        convGradWeightKernel<L, 0, I, J><<<grid, dev::kBlock, 0, st>>>(q, gk);
-                      }};
+    return Kernel{(const void *)convGradWeightSmallKernel<I, J>,
+                  [](dim3 grid, hipStream_t st, const GradWeightArgs &q, const ConvGeom &gk) {
+                    convGradWeightSmallKernel<I, J><<<grid, dev::kBlock, 0, st>>>(q, gk);
+                  }};
   };
-  auto pickTiny = [&](auto l16c) {
+  auto pickSmall = [&]() {
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
-    using I4 = std::integral_constant<int, 4>;
-    if (tI == 1 && tJ == 1) return tinyKernel(l16c, I1{}, I1{});
-    if (tI == 1 && tJ == 2) return tinyKernel(l16c, I1{}, I2{});
-    if (tI == 1 && tJ == 4) return tinyKernel(l16c, I1{}, I4{});
-    if (tI == 2 && tJ == 1) return tinyKernel(l16c, I2{}, I1{});
-    return tinyKernel(l16c, I2{}, I2{});
-  };
-  const TinyKernel tk = l16 ? pickTiny(std::true_type{}) : pickTiny(std::false_type{});
-  // 16-byte gathers of the image: unit stride along a row, and groups of 4 positions that stay inside an output row
-  // (or output rows that follow each other in the image without a gap: kW = 1, no padding, unit stride down too)
-  const bool b4 = fast && !tiny && !padGy && g.dW == 1 &&
-                  (g.oW % 4 == 0 || (g.dH == 1 && g.W + 2 * g.padW == g.oW));
-  struct BigKernel {
-    const void *fn;
-    void (*launch)(dim3, hipStream_t, const GradWeightArgs &, const ConvGeom &);
+    if (tI == 1 && tJ == 1) return smallKernel(I1{}, I1{});
+    if (tI == 1 && tJ == 2) return smallKernel(I1{}, I2{});
+    if (tI == 2 && tJ == 1) return smallKernel(I2{}, I1{});
+    return smallKernel(I2{}, I2{});
   };
   auto bigKernel = [](auto l16c, auto wmc, auto b4c) {
     constexpr bool L = decltype(l16c)::value, B = decltype(b4c)::value;
     constexpr int W = decltype(wmc)::value;
-    return BigKernel{(const void *)convGradWeightSplitKernel<L, W, B>,
+    return Kernel{(const void *)convGradWeightSplitKernel<L, W, B>,
                      [](dim3 grid, hipStream_t st, const GradWeightArgs &q, const ConvGeom &gk) {
                        convGradWeightSplitKernel<L, W, B><<<grid, dev::kBlock, 0, st>>>(q, gk);
                      }};
@@ -3274,8 +3196,10 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   auto pickBigW = [&](auto l16c) {
     return wide ? pickBig(l16c, std::integral_constant<int, 1>{}) : pickBig(l16c, std::integral_constant<int, 2>{});
   };
-  const BigKernel bk = l16 ? pickBigW(std::true_type{}) : pickBigW(std::false_type{});
-  const void *kern = !fast ? (const void *)convGemmKernel<kGradWeight> : tiny ? tk.fn : bk.fn;
+  const Kernel gw = tiny ? pickSmall() : l16 ? pickBigW(std::true_type{}) : pickBigW(std::false_type{});
+  const void *kern = fast ? gw.fn : (const void *)convGemmKernel<kGradWeight>;
+  const int ktPositions = tiny ? kSmallPositions : BK;
+  const int totalKt = launch::ceilDiv(g.N * Lk, ktPositions);
   // Every split leaves a partial copy of gradWeight (64 KB per tile) for the fold: three workgroups per CU
   // measured better than the four that fit (less partial traffic for the same matrix-pipe load), two when
   // gradWeight is one or two tiles and the partials are most of the traffic. The small tiles stream: as many
@@ -3287,12 +3211,10 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
     const int slots = std::min(residentSlots(kern), residentSlots(nullptr) * wgPerCu);
     return std::max(1, std::min(totalKt, slots / (mT * nT)));
   };
-  while (perCu > 1 && totalKt / splitsAt(perCu) < 20) --perCu;
+  while (perCu > 1 && totalKt / splitsAt(perCu) < 20 * BK / ktPositions) --perCu;
   int splits = splitsAt(perCu);
   const int perSplit = launch::ceilDiv(totalKt, splits);
   splits = launch::ceilDiv(totalKt, perSplit);
-  const int wgSplits = splits;       // splits of the positions over workgroups
-  if (tiny) splits *= 4;             // partial copies of gradWeight: one per wave
   const long count = (long)g.Cout * g.K;
   // scratch: the splits' partial products, then (second-generation kernel) the images with their zero border
   const long partialFloats = (splits * count + 3) / 4 * 4;
@@ -3335,11 +3257,7 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
     q.magicOW = dev::magicOf(g.oW);
     q.magicKK = dev::magicOf(g.kH * g.kW), q.magicKW = dev::magicOf(g.kW);
     q.Lvalid = g.L;
-    const dim3 grid(mT * nT * wgSplits);
-    if (tiny)
-      tk.launch(grid, s, q, gk);
-    else
-      bk.launch(grid, s, q, gk);
+    gw.launch(dim3(mT * nT * splits), s, q, gk);
   } else {
     GemmArgs p{};
     p.a = gy;

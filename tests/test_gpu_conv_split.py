@@ -31,6 +31,12 @@ CASES = [
     (2, 28, 60, 16, 16, 3, 2, 1),
     (3, 28, 60, 9, 12, 3, 1, 1),
     (3, 28, 60, 13, 14, 3, 1, 1),
+    # the weight gradient's small tiles: 2x2, 2x1, 1x2 and 1x1 blocks, images shorter than a k-tile, padded rows of positions
+    (3, 3, 64, 30, 28, 7, 2, 3),
+    (2, 3, 50, 13, 11, 3, 1, 1),
+    (2, 6, 24, 16, 12, 3, 1, 1),
+    (5, 8, 32, 4, 4, 1, 1, 0),
+    (4, 6, 24, 5, 5, 3, 1, 1),
     # bordered copies in runs: planes of an odd size, larger than a run, smaller with several to a run, wide rows
     (2, 8, 24, 67, 61, 3, 1, 1),
     (33, 64, 8, 37, 35, 3, 1, 1),
@@ -96,7 +102,7 @@ def _check_non_finite(case, passes=3):
     N, Ci, Co, H, W, k, st, pad = case
     x, w, gy = _tensors(case, "normal", 6)
     w *= 1e-3
-    x[0, 1, 2, 3], x[1 % N, 0, 4 % H, 4], x[N - 1, Ci - 1, H - 1, W - 1], x[0, 2, H - 1, 0] = np.inf, np.nan, 3.4e38, -3.4e38
+    x[0, 1, 2, 3], x[1 % N, 0, 4 % H, 4 % W], x[N - 1, Ci - 1, H - 1, W - 1], x[0, 2, H - 1, 0] = np.inf, np.nan, 3.4e38, -3.4e38
     gy[0, 3, 1, 2], gy[1 % N, 0, 0, 0] = -np.inf, np.nan
     gyw = gy * np.float32(1e-3)          # times 3.4e38 still finite: no sum overflows in one order and not in another
     gy[N - 1, Co - 1, 2, 1] = 3.4e38
