@@ -385,20 +385,20 @@ __device__ __forceinline__ void splitColumn(const FwdArgs &p, const ConvGeom &g,
 }
 
 // biasDone: the accumulators started from the bias (whole tiles of the padded kernel)
-template <int TBN = BN, int TI = 2>
-__device__ __forceinline__ void fwdEpilogue(const FwdArgs &p, const ConvGeom &g, const float16v (&acc)[TI][2], int bx,
+template <int TBN = BN, int TI = 2, int TJ = 2>
+__device__ __forceinline__ void fwdEpilogue(const FwdArgs &p, const ConvGeom &g, const float16v (&acc)[TI][TJ], int bx,
                                             int by, int m0, int j0, int wm, int wn, int grp, int idx,
                                             const float *biasLds = nullptr, int toPartial = -1, bool biasDone = false) {
   const int rowHalf = grp * 4;
   if (toPartial < 0 ? p.nSplit > 1 : toPartial != 0) {
-    float *dst = p.partial + ((long)bx * p.nSplit + by) * (BM * BN);  // both tile shapes hold BM * BN elements
+    float *dst = p.partial + ((long)bx * p.nSplit + by) * (BM * BN);  // (no tile shape holds more than BM * BN elements)
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj)
+    for (int tj = 0; tj < TJ; ++tj)
 #pragma unroll
       for (int ti = 0; ti < TI; ++ti)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-          dst[(wm * 64 + ti * 32 + 8 * (v >> 2) + rowHalf + (v & 3)) * TBN + wn * 64 + tj * 32 + idx] = acc[ti][tj][v];
+          dst[(wm * 64 + ti * 32 + 8 * (v >> 2) + rowHalf + (v & 3)) * TBN + wn * 32 * TJ + tj * 32 + idx] = acc[ti][tj][v];
     return;
   }
   if (biasDone && p.outBytes > 0 && m0 + wm * 64 + TI * 32 <= p.M) {
@@ -407,8 +407,8 @@ __device__ __forceinline__ void fwdEpilogue(const FwdArgs &p, const ConvGeom &g,
     const __amdgpu_buffer_rsrc_t orr = dev::makeRsrc(p.out, p.outBytes);
     const int rowBase = __builtin_amdgcn_readfirstlane(m0 + wm * 64);
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      const unsigned col = (unsigned)j0 + wn * 64 + tj * 32 + idx;
+    for (int tj = 0; tj < TJ; ++tj) {
+      const unsigned col = (unsigned)j0 + wn * 32 * TJ + tj * 32 + idx;
       int n, oh, ow;
       splitColumn(p, g, min(col, (unsigned)p.Ncols - 1), n, oh, ow);
       const int voff = col < (unsigned)p.Ncols
@@ -458,8 +458,8 @@ __device__ __forceinline__ void fwdEpilogue(const FwdArgs &p, const ConvGeom &g,
         }
     }
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      const unsigned col = (unsigned)j0 + wn * 64 + tj * 32 + idx;  // Ncols < 2^31
+    for (int tj = 0; tj < TJ; ++tj) {
+      const unsigned col = (unsigned)j0 + wn * 32 * TJ + tj * 32 + idx;  // Ncols < 2^31
       if (col >= (unsigned)p.Ncols) continue;
       int n, oh, ow;
       splitColumn(p, g, col, n, oh, ow);
@@ -963,6 +963,7 @@ __device__ __forceinline__ void mfmaSplit(const u32x4 (&a)[3][TI], const u32x4 (
 // Rows past M and columns past the batch are clamped to valid ones and dropped in the epilogue.
 // WM = 2: 128 x 128 tiles, the four waves as 2 x 2; WM = 1: 64 x 256 tiles, the four waves side by side,
 // for row counts whose last 128-row tile would be at most half full; a wave multiplies 64 x 64 either way.
+// WM = 3: 96 x 128 tiles, the four waves side by side, a wave multiplies 96 x 32 (see tileShape).
 // WM = 0: 32 x 256 tiles, a wave multiplies 32 x 64, for 32 rows or fewer left over (32-plane layers).
 // (bx, by): position among the tiles that start at tile0 and split; whole: the workgroup reduces all of K
 // of tile bx and writes the output itself
@@ -970,11 +971,11 @@ __device__ __forceinline__ void mfmaSplit(const u32x4 (&a)[3][TI], const u32x4 (
 // read from the table
 template <int WM, bool LINEAR = false>
 __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &g, int bx, int by, bool whole) {
-  constexpr int TBM = WM == 0 ? 32 : 64 * WM, TBN = WM == 2 ? 128 : 256;
-  constexpr int TI = WM == 0 ? 1 : 2;         // 32-row blocks of a wave
-  constexpr int NA = WM == 2 ? 2 : 1;         // 16-byte groups of weights a lane loads per k-tile
+  constexpr int TBM = WM == 0 ? 32 : WM == 3 ? 96 : 64 * WM, TBN = WM >= 2 ? 128 : 256;
+  constexpr int TI = WM == 0 ? 1 : WM == 3 ? 3 : 2, TJ = WM == 3 ? 1 : 2;  // 32 x 32 blocks of a wave
+  constexpr int NA = WM >= 2 ? 2 : 1;         // 16-byte groups of weights a lane loads per k-tile
   constexpr int AP = TBM + 8, BP = TBN + 8;   // 16-byte groups (8 k of one part) per k-group row
-  constexpr int NB = WM == 2 ? 8 : 16;        // image elements a lane gathers per k-tile
+  constexpr int NB = WM >= 2 ? 8 : 16;        // image elements a lane gathers per k-tile
   __shared__ u32x4 As[2][3][2][AP];           // [buffer][part][k-group of 8][row]
   __shared__ u32x4 Bs[2][3][2][BP];
   __shared__ __attribute__((aligned(16))) float biasS[TBM];  // the tile's bias values: the epilogue reads them from here
@@ -989,12 +990,15 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, p.xBytes, 0x00020000);
   // weights: WM = 2 - a lane loads 8 consecutive k of row t / 2; WM = 1 - 4 consecutive k of row t / 4;
   //          WM = 0 - the same of row (t / 4) % 32: both halves of the workgroup fetch and park the same values
-  // image:   WM = 2 - a lane gathers 8 taps of column t % 128; WM < 2 - all 16 taps of column t
-  const int rowA = WM == 2 ? t >> 1 : WM == 1 ? t >> 2 : (t >> 2) & 31;
+  //          WM = 3 - 4 consecutive k of row t / 4, and of row 64 + (t / 4) % 32 (both halves the same)
+  // image:   WM >= 2 - a lane gathers 8 taps of column t % 128; WM < 2 - all 16 taps of column t
+  const int rowA = WM == 2 ? t >> 1 : WM == 0 ? (t >> 2) & 31 : t >> 2;
+  const int rowA2 = 64 + ((t >> 2) & 31);  // WM = 3
   const int kA = WM == 2 ? (t & 1) * 8 : (t & 3) * 4;
-  const int colB = WM == 2 ? t & 127 : t;
-  const int kgB = WM == 2 ? t >> 7 : 0;
+  const int colB = WM >= 2 ? t & 127 : t;
+  const int kgB = WM >= 2 ? t >> 7 : 0;
   const int aOff = (min(m0 + rowA, p.M - 1) * g.K + kA) * 4;
+  const int aOff2 = WM == 3 ? (min(m0 + rowA2, p.M - 1) * g.K + kA) * 4 : aOff + 16;  // the second group
   const int kB = __builtin_amdgcn_readfirstlane(kgB * 8);
   auto columnOffset = [&](unsigned col) {
     int n, oh, ow;
@@ -1025,7 +1029,7 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   auto loadTiles = [&](int kt) {
     const int k0 = __builtin_amdgcn_readfirstlane(kt * BK);
 #pragma unroll
-    for (int i = 0; i < NA; ++i) ra[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, aOff + 16 * i, k0 * 4, 0);
+    for (int i = 0; i < NA; ++i) ra[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, i ? aOff2 : aOff, k0 * 4, 0);
 #pragma unroll
     for (int i = 0; i < NB / 4; ++i) {
       rb[4 * i + 0] = __builtin_amdgcn_raw_buffer_load_b32(xr, posOff, e[i].x, 0);
@@ -1051,13 +1055,16 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
       aDst[b * BUFA + PA] = u32x4{m[0], m[1], m[2], m[3]};
       aDst[b * BUFA + 2 * PA] = u32x4{l[0], l[1], l[2], l[3]};
     } else {  // 4 k: half of a group
-      unsigned h[2], m[2], l[2];
-      splitPair(ra[0].x, ra[0].y, h[0], m[0], l[0]);
-      splitPair(ra[0].z, ra[0].w, h[1], m[1], l[1]);
-      u32x2 *d = reinterpret_cast<u32x2 *>(aDst + b * BUFA) + ((kA >> 2) & 1);
-      d[0] = u32x2{h[0], h[1]};
-      d[2 * PA] = u32x2{m[0], m[1]};
-      d[4 * PA] = u32x2{l[0], l[1]};
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        unsigned h[2], m[2], l[2];
+        splitPair(ra[i].x, ra[i].y, h[0], m[0], l[0]);
+        splitPair(ra[i].z, ra[i].w, h[1], m[1], l[1]);
+        u32x2 *d = reinterpret_cast<u32x2 *>(aDst + b * BUFA + (i ? rowA2 - rowA : 0)) + ((kA >> 2) & 1);
+        d[0] = u32x2{h[0], h[1]};
+        d[2 * PA] = u32x2{m[0], m[1]};
+        d[4 * PA] = u32x2{l[0], l[1]};
+      }
     }
 #pragma unroll
     for (int q = 0; q < NB / 8; ++q) {
@@ -1071,23 +1078,23 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   };
   const int grp = lane >> 5, idx = lane & 31;
   const u32x4 *aSrc = &As[0][0][grp][wm * 64 + idx];
-  const u32x4 *bSrc = &Bs[0][0][grp][wn * 64 + idx];
+  const u32x4 *bSrc = &Bs[0][0][grp][wn * 32 * TJ + idx];
   using Buf0 = std::integral_constant<int, 0>;
   using Buf1 = std::integral_constant<int, 1>;
 
-  float16v acc[TI][2], lo[TI][2];
+  float16v acc[TI][TJ], lo[TI][TJ];
 
   // Software pipeline. While tile kt is multiplied out of one LDS buffer, tile kt + 1 waits in registers - it is
   // split and parked in the other buffer under the matrix instructions - and tile kt + 2 is requested from memory.
   auto step = [&](auto cur, auto nxt, int kt, bool store, bool load) {
     constexpr int C = decltype(cur)::value;
-    u32x4 a[3][TI], b[3][2];
+    u32x4 a[3][TI], b[3][TJ];
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
 #pragma unroll
       for (int i = 0; i < TI; ++i) a[s][i] = aSrc[C * BUFA + s * PA + 32 * i];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) b[s][j] = bSrc[C * BUFB + s * PB + 32 * j];
+      for (int j = 0; j < TJ; ++j) b[s][j] = bSrc[C * BUFB + s * PB + 32 * j];
     }
     if (store) storeTiles(nxt);
     if (load) {
@@ -1120,11 +1127,12 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   };
 #pragma unroll
   for (int i = 0; i < TI; ++i) {
-    acc[i][0] = acc[i][1] = biasBlock(i);
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TJ; ++j) {
+      acc[i][j] = biasBlock(i);
 #pragma unroll
       for (int v = 0; v < 16; ++v) lo[i][j][v] = 0.f;
+    }
   }
   int kt = ktBegin;
   for (; kt + 3 < nkt; kt += 2) {  // tile kt sits in buffer 0, tile kt + 1 in registers
@@ -1140,7 +1148,7 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TJ; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
@@ -1149,8 +1157,8 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   if (__any(bad != bad)) {
     // the wave's blocks again in fp32, operands straight from memory
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int cOff = columnOffset((unsigned)j0 + wn * 64 + j * 32 + idx);
+    for (int j = 0; j < TJ; ++j) {
+      const int cOff = columnOffset((unsigned)j0 + wn * 32 * TJ + j * 32 + idx);
 #pragma unroll
       for (int i = 0; i < TI; ++i) {
         const int rOff = min(m0 + wm * 64 + i * 32 + idx, p.M - 1) * g.K;
@@ -1171,7 +1179,7 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
       }
     }
   }
-  fwdEpilogue<TBN, TI>(p, g, acc, bx, by, m0, j0, wm, wn, grp, idx, biasS, whole ? 0 : 1, whole);
+  fwdEpilogue<TBN, TI, TJ>(p, g, acc, bx, by, m0, j0, wm, wn, grp, idx, biasS, whole ? 0 : 1, whole);
 }
 
 // Forward kernel for short calls (planDirect): a workgroup computes a tile of 32 T x 32 T, its four waves a quarter of
@@ -2253,7 +2261,7 @@ bool forceGeneric() { return g_switches.convGeneric == 1; }
 // Whole tiles and splits are workgroups of one launch: the splits take the slots
 // that the last whole tiles free.
 struct FwdPlan {
-  int bm, bn;          // tile shape: 128 x 128, or 64 x 256 when that wastes fewer rows (padded kernel only)
+  int bm, bn;          // tile shape: 128 x 128, or one that wastes fewer rows (tileShape; padded kernel only)
   int direct;          // != 0: convFwdDirectKernel, tiles of 32 * direct rows and columns
   int mTiles, total, full, tail, nSplit, ktPerSplit;
   int tapEntries;      // > 0: the padded kernel applies; entries of the tap table at the start of the scratch
@@ -2261,13 +2269,24 @@ struct FwdPlan {
   long weightFloats;   // floats of the copy of the weights with rows padded to a multiple of BK (0: not needed)
   long scratchFloats;  // tap table, tail partials, padded images
 };
+// Shape of the output tiles for M rows (others: the padded kernel's shapes beside 128 x 128 may be used).
+void tileShape(int M, bool others, int &bm, int &bn) {
+  const long r128 = tiles(M, BM) * (long)BM, r64 = tiles(M, 64) * 64L, r96 = tiles(M, 96) * 96L, r32 = tiles(M, 32) * 32L;
+  bm = BM, bn = BN;
+  if (!others) return;
+  // 96 x 128 where that pads a sixth fewer rows (65 ... 96 rows; its waves read LDS a third more often per product): 80 rows,
+  // 3x3 of 192 planes over 32 x 71 x 71 positions 455 us in 32-row tiles, 348 in 96; 288 rows of 128 planes 24.6 in 64, 26.2
+  if (r96 * 6 < std::min(r64, r128) * 5)
+    bm = 96;
+  else if (r32 * 4 <= r64 * 3)  // 32 rows: a wave issues half the matrix instructions per element it gathers
+    bm = 32, bn = 256;
+  else if (r64 < r128)
+    bm = 64, bn = 256;
+}
+
 // Tiles of an M x Ncols output reduced over nkt k-tiles; wideOk: the 64 x 256 tile shape may be used.
 void planTiles(FwdPlan &pl, int M, long Ncols, int nkt, bool wideOk) {
-  const bool wide = wideOk && tiles(M, 64) * 64 < tiles(M, BM) * BM;
-  // 32-row tiles when they cut the padded rows by a quarter or more (a wave then issues half the MFMAs per
-  // element it gathers)
-  const bool low = wideOk && tiles(M, 32) * 32 * 4 <= tiles(M, 64) * 64 * 3;
-  pl.bm = low ? 32 : wide ? 64 : BM, pl.bn = low || wide ? 256 : BN;
+  tileShape(M, wideOk, pl.bm, pl.bn);
   pl.mTiles = (int)tiles(M, pl.bm);
   pl.total = pl.mTiles * (int)tiles(Ncols, pl.bn);
   const int cus = residentSlots(nullptr);
@@ -2378,12 +2397,16 @@ void launchFwdKernels(hipStream_t s, const FwdPlan &pl, FwdArgs p, float *partia
         convFwdPaddedKernel<0, true><<<grid, dev::kBlock, 0, s>>>(p, gk);
       else if (pl.bm == 64)
         convFwdPaddedKernel<1, true><<<grid, dev::kBlock, 0, s>>>(p, gk);
+      else if (pl.bm == 96)
+        convFwdPaddedKernel<3, true><<<grid, dev::kBlock, 0, s>>>(p, gk);
       else
         convFwdPaddedKernel<2, true><<<grid, dev::kBlock, 0, s>>>(p, gk);
     } else if (pl.bm == 32) {
       convFwdPaddedKernel<0><<<grid, dev::kBlock, 0, s>>>(p, gk);
     } else if (pl.bm == 64) {
       convFwdPaddedKernel<1><<<grid, dev::kBlock, 0, s>>>(p, gk);
+    } else if (pl.bm == 96) {
+      convFwdPaddedKernel<3><<<grid, dev::kBlock, 0, s>>>(p, gk);
     } else {
       convFwdPaddedKernel<2><<<grid, dev::kBlock, 0, s>>>(p, gk);
     }
@@ -2719,9 +2742,8 @@ bool gradInputByPhase(THCState *state, const ConvGeom &g, const float *gy, const
   // All phases of a group of images run as one batched launch. The phases differ in K; the heavier ones are
   // split along K so that a workgroup reduces about the same number of k-tiles whatever its phase and the
   // grid holds about two workgroups per CU. Split phases leave partial tiles for the batched fold.
-  const bool wide = tiles(g.Cin, 64) * 64 < tiles(g.Cin, BM) * BM;
-  const bool low = tiles(g.Cin, 32) * 32 * 4 <= tiles(g.Cin, 64) * 64 * 3;  // as in planTiles
-  const int bm = low ? 32 : wide ? 64 : BM, bn = low || wide ? 256 : BN;
+  int bm, bn;
+  tileShape(g.Cin, true, bm, bn);
   const int mTiles = (int)tiles(g.Cin, bm);
   struct Split {
     int tiles, tail, nSplit, ktPerSplit;  // the last `tail` of the item's tiles are split nSplit ways
@@ -2862,10 +2884,12 @@ bool gradInputByPhase(THCState *state, const ConvGeom &g, const float *gy, const
     }
     batch.wholeTotal = wholeTotal;
     const dim3 grid(wholeTotal + splitTotal);
-    if (low)
+    if (bm == 32)
       convFwdPaddedBatchKernel<0><<<grid, dev::kBlock, 0, s>>>(batch);
-    else if (wide)
+    else if (bm == 64)
       convFwdPaddedBatchKernel<1><<<grid, dev::kBlock, 0, s>>>(batch);
+    else if (bm == 96)
+      convFwdPaddedBatchKernel<3><<<grid, dev::kBlock, 0, s>>>(batch);
     else
       convFwdPaddedBatchKernel<2><<<grid, dev::kBlock, 0, s>>>(batch);
     THC_HIP_CHECK(hipGetLastError());

@@ -144,3 +144,25 @@ def test_short_calls(case, shape):
         _check_non_finite(case, passes=2)    # forward and gradInput
     finally:
         cunn_amd.set_switch("THCUNN_CONV_DIRECT", None)
+
+
+# ---- the tiled kernels also where the kernel for short calls would be taken, and their 96-row tiles (65 ... 96 rows, a
+#      strided gradInput by phases, split along K) ----
+ROWS96 = [
+    (2, 32, 80, 14, 13, 3, 1, 1),
+    (2, 80, 40, 13, 12, 3, 1, 1),
+    (2, 72, 16, 15, 14, 3, 2, 1),
+    (1, 32, 96, 9, 9, 1, 1, 0),
+    (2, 512, 96, 8, 8, 3, 1, 1),
+]
+
+
+@pytest.mark.parametrize("case", CASES + ROWS96)
+def test_tiled(case):
+    print("case", case, flush=True)
+    cunn_amd.set_switch("THCUNN_CONV_DIRECT", "0")
+    try:
+        _check_error(case, "normal")
+        _check_non_finite(case, passes=2)
+    finally:
+        cunn_amd.set_switch("THCUNN_CONV_DIRECT", None)
