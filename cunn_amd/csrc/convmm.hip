@@ -352,7 +352,7 @@ struct FwdArgs {
   const float *bias;  // M or null
   int M, Ncols;       // Ncols = nImages * L
   int mTiles;
-  int bm, bn;         // rows and columns of an output tile: 128 x 128, or 64 x 256 (padded kernel only)
+  int bm, bn;         // rows and columns of an output tile (tileShape)
   int xBytes;         // bytes of the nImages input images (< 2^31)
   int wBytes;         // padded kernel: bytes of the weights (< 2^31)
   bool vecA;
@@ -961,21 +961,18 @@ __device__ __forceinline__ void mfmaSplit(const u32x4 (&a)[3][TI], const u32x4 (
 // clock that power has pulled down to 2.05 GHz. 256 -> 256 planes 3x3 at 28 x 28, N = 64 (59.2 GFLOP):
 // 430 us with v_mfma_f32_32x32x2_f32, 307 us (193 TFLOP/s) on the parts.
 // Rows past M and columns past the batch are clamped to valid ones and dropped in the epilogue.
-// WM = 2: 128 x 128 tiles, the four waves as 2 x 2; WM = 1: 64 x 256 tiles, the four waves side by side,
-// for row counts whose last 128-row tile would be at most half full; a wave multiplies 64 x 64 either way.
-// WM = 3: 96 x 128 tiles, the four waves side by side, a wave multiplies 96 x 32 (see tileShape).
-// WM = 0: 32 x 256 tiles, a wave multiplies 32 x 64, for 32 rows or fewer left over (32-plane layers).
-// (bx, by): position among the tiles that start at tile0 and split; whole: the workgroup reduces all of K
-// of tile bx and writes the output itself
-// LINEAR: 1x1 windows - the tap offsets are an arithmetic sequence, computed by the scalar unit instead of
-// read from the table
+// WM = 2: 128 x 128 tiles, the four waves as 2 x 2, 64 x 64 each. For row counts that would leave much of a 128-row tile
+// empty (tileShape) the four waves sit side by side: WM = 1: 64 x 128 tiles, 64 x 32 a wave; WM = 3: 96 x 128, 96 x 32;
+// WM = 0: 32 x 256, 32 x 64. WM = 1 keeps three workgroups on a CU; with 64 x 256 tiles (64 x 64 a wave, two workgroups)
+// 64 -> 64 3x3 on 56x56 took, at N = 8 / 16 / 32, 33.7 / 49.0 / 65.9 us, now 32.5 / 42.1 / 61.6; 3 -> 64 7x7 stride 2 on
+// 224x224, N = 32: 83.9, now 75.0; 256 -> 64 1x1 on 56x56, N = 8: 21.0, now 12.5.
 template <int WM, bool LINEAR = false>
 __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &g, int bx, int by, bool whole) {
-  constexpr int TBM = WM == 0 ? 32 : WM == 3 ? 96 : 64 * WM, TBN = WM >= 2 ? 128 : 256;
-  constexpr int TI = WM == 0 ? 1 : WM == 3 ? 3 : 2, TJ = WM == 3 ? 1 : 2;  // 32 x 32 blocks of a wave
-  constexpr int NA = WM >= 2 ? 2 : 1;         // 16-byte groups of weights a lane loads per k-tile
+  constexpr int TBM = WM == 0 ? 32 : WM == 2 ? 128 : WM == 3 ? 96 : 64, TBN = WM == 0 ? 256 : 128;
+  constexpr int TI = WM == 0 ? 1 : WM == 3 ? 3 : 2, TJ = WM == 1 || WM == 3 ? 1 : 2;  // 32 x 32 blocks of a wave
+  constexpr int NA = WM == 2 || WM == 3 ? 2 : 1;         // 16-byte groups of weights a lane loads per k-tile
   constexpr int AP = TBM + 8, BP = TBN + 8;   // 16-byte groups (8 k of one part) per k-group row
-  constexpr int NB = WM >= 2 ? 8 : 16;        // image elements a lane gathers per k-tile
+  constexpr int NB = WM == 0 ? 16 : 8;        // image elements a lane gathers per k-tile
   __shared__ u32x4 As[2][3][2][AP];           // [buffer][part][k-group of 8][row]
   __shared__ u32x4 Bs[2][3][2][BP];
   __shared__ __attribute__((aligned(16))) float biasS[TBM];  // the tile's bias values: the epilogue reads them from here
@@ -991,12 +988,12 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   // weights: WM = 2 - a lane loads 8 consecutive k of row t / 2; WM = 1 - 4 consecutive k of row t / 4;
   //          WM = 0 - the same of row (t / 4) % 32: both halves of the workgroup fetch and park the same values
   //          WM = 3 - 4 consecutive k of row t / 4, and of row 64 + (t / 4) % 32 (both halves the same)
-  // image:   WM >= 2 - a lane gathers 8 taps of column t % 128; WM < 2 - all 16 taps of column t
+  // image:   a lane gathers 8 taps of column t % 128; WM = 0 - all 16 taps of column t
   const int rowA = WM == 2 ? t >> 1 : WM == 0 ? (t >> 2) & 31 : t >> 2;
   const int rowA2 = 64 + ((t >> 2) & 31);  // WM = 3
   const int kA = WM == 2 ? (t & 1) * 8 : (t & 3) * 4;
-  const int colB = WM >= 2 ? t & 127 : t;
-  const int kgB = WM >= 2 ? t >> 7 : 0;
+  const int colB = WM == 0 ? t : t & 127;
+  const int kgB = WM == 0 ? 0 : t >> 7;
   const int aOff = (min(m0 + rowA, p.M - 1) * g.K + kA) * 4;
   const int aOff2 = WM == 3 ? (min(m0 + rowA2, p.M - 1) * g.K + kA) * 4 : aOff + 16;  // the second group
   const int kB = __builtin_amdgcn_readfirstlane(kgB * 8);
@@ -1350,7 +1347,7 @@ convFwdDirectKernel(FwdArgs p, ConvGeom g) {
 }
 
 template <int WM, bool LINEAR = false>
-__global__ void __launch_bounds__(dev::kBlock, 2)
+__global__ void __launch_bounds__(dev::kBlock, WM == 1 ? 3 : 2)
 convFwdPaddedKernel(FwdArgs p, ConvGeom g) {
   int bx = blockIdx.x, by = 0;
   const bool whole = bx < p.full;
@@ -1379,7 +1376,7 @@ struct FwdBatch {
 static_assert(sizeof(FwdBatch) <= 4096, "kernel arguments are limited to 4 KB");
 
 template <int WM>
-__global__ void __launch_bounds__(dev::kBlock, 2)
+__global__ void __launch_bounds__(dev::kBlock, WM == 1 ? 3 : 2)
 convFwdPaddedBatchKernel(FwdBatch b) {
   int bx = blockIdx.x, by = 0, i = 0;
   const bool whole = bx < b.wholeTotal;
@@ -2280,11 +2277,11 @@ void tileShape(int M, bool others, int &bm, int &bn) {
     bm = 96;
   else if (r32 * 4 <= r64 * 3)  // 32 rows: a wave issues half the matrix instructions per element it gathers
     bm = 32, bn = 256;
-  else if (r64 < r128)
-    bm = 64, bn = 256;
+  else if (r64 < r128)  // (128 rows or more: 128 x 128 is better, 256 -> 256 3x3 on 28x28, N = 64: 334 against 357 us)
+    bm = 64;
 }
 
-// Tiles of an M x Ncols output reduced over nkt k-tiles; wideOk: the 64 x 256 tile shape may be used.
+// Tiles of an M x Ncols output reduced over nkt k-tiles; wideOk: tileShape has its choice.
 void planTiles(FwdPlan &pl, int M, long Ncols, int nkt, bool wideOk) {
   tileShape(M, wideOk, pl.bm, pl.bn);
   pl.mTiles = (int)tiles(M, pl.bm);
@@ -2293,16 +2290,17 @@ void planTiles(FwdPlan &pl, int M, long Ncols, int nkt, bool wideOk) {
   // Which tiles to split along K, and how finely: the workgroups go to the CUs in launch order (up to three
   // share a CU), so a CU's time is the sum over what it is dealt. In units of one k-tile of one workgroup alone
   // on its CU: a workgroup costs its k-tiles + 4 (prologue, epilogue), a split tile 0.006 more per partial
-  // (written, then read by the fold), and a CU that only ever holds one workgroup runs at 0.85 of the rate
+  // (written, then read by the fold), and a CU that only ever holds one workgroup runs at 0.85 of the rate (0.75 with 64-row tiles)
   // (nothing covers its barriers) - constants fitted to measured sweeps over S on 14x14 ... 56x56 layers.
   // Candidates: no split; the last, partial round split S ways; every tile split S ways (S <= 16, >= 4 k-tiles
   // per split). E.g. 196 tiles on 256 CUs: 5 splits (980 workgroups, 4 per CU at most) beat 2 (392: 136 CUs
   // carry two halves, 120 one) by 15 %; 136 tiles left over after a full round: 3 splits, not 1.
   const int maxS = std::max(1, std::min(nkt / 4, 16));
   const int q = pl.total / cus, r = pl.total % cus;
+  const double lone = pl.bm == 64 ? 0.75 : 0.85;
   auto perWg = [&](int S) { return (double)launch::ceilDiv(nkt, S) + 4.0; };
   // a split has to promise 5 % before it is taken: the model is coarse and the fold is one more launch
-  double best = 0.95 * launch::ceilDiv(pl.total, cus) * perWg(1) / (pl.total <= cus ? 0.85 : 1.0);
+  double best = 0.95 * launch::ceilDiv(pl.total, cus) * perWg(1) / (pl.total <= cus ? lone : 1.0);
   int nSplit = 1;
   pl.tail = 0;
   for (int S = 2; S <= maxS; ++S) {
@@ -2313,7 +2311,7 @@ void planTiles(FwdPlan &pl, int M, long Ncols, int nkt, bool wideOk) {
     }
     if (pl.total <= 2 * cus) {
       const int n = launch::ceilDiv(pl.total * S, cus);
-      const double t = n * perWg(S) / (n == 1 ? 0.85 : 1.0) + 0.006 * pl.total * S;
+      const double t = n * perWg(S) / (n == 1 ? lone : 1.0) + 0.006 * pl.total * S;
       if (t < best) best = t, nSplit = S, pl.tail = pl.total;
     }
   }
@@ -2326,7 +2324,7 @@ inline long partialFloats(const FwdPlan &pl) { return pl.tail ? (long)pl.tail * 
 // Whether a short call runs on convFwdDirectKernel: one launch, against workgroup tiles that would leave CUs idle or
 // have K split over workgroups, with partial tiles in memory and a second launch that folds them. Both times in us,
 // fitted to measured calls (tiled / direct): 512 -> 512 1x1 on 14x14, N = 1: 9.8 / 6.3; 256 -> 256 1x1 on 14x14, N = 8:
-// 12.8 / 7.7; 128 -> 128 3x3 on 28x28, N = 2: 20.4 / 14.6; 256 -> 64 1x1 on 56x56, N = 8: 19.5 / 15.6; 64 -> 128 1x1 on
+// 12.8 / 7.7; 128 -> 128 3x3 on 28x28, N = 2: 20.4 / 14.6; 256 -> 64 1x1 on 56x56, N = 8: 12.5 / 15.6; 64 -> 128 1x1 on
 // 28x28, N = 16: 9.4 / 10.6; 128 -> 512 1x1 on 28x28, N = 8: 13.7 / 20.7; 256 -> 256 3x3 on 14x14, N = 1: 18.0 / 21.8.
 // 32 x 32 tiles while those are few, then 64 x 64 (fewer loads per product; the line between them: 64 -> 64 3x3 on
 // 56x56, N = 4, 784 tiles of 32 x 32: 23.9 / 20.0; 256 -> 256 1x1 on 14x14, N = 8, 392 tiles: 7.7 / 9.8).
@@ -2337,7 +2335,7 @@ void planDirect(FwdPlan &pl, int M, long Ncols, int nkt) {
   const bool small = tiles32 <= 512;
   if (force < 0) {
     if (pl.total >= residentSlots(nullptr)) return;  // a workgroup tile for every CU: the tiled kernel is better at any size
-    const double tiled = 6.0 + 0.85 * pl.ktPerSplit + (pl.tail > 0 ? 5.0 + 0.02 * pl.tail * pl.nSplit : 0.0);
+    const double tiled = 6.0 + (pl.bm == 64 ? 0.55 : 0.85) * pl.ktPerSplit + (pl.tail > 0 ? 5.0 + 0.02 * pl.tail * pl.nSplit : 0.0);
     const double direct = 4.5 + 0.002 * tiles32 + std::max(0.13 * nkt, (small ? 0.65e-3 : 0.45e-3) * tiles32 * nkt);
     if (direct >= tiled) return;
   }
