@@ -2770,7 +2770,9 @@ bool gradInputByPhase(THCState *state, const ConvGeom &g, const float *gy, const
     // No phase is heavy enough to be split by that rule, and the whole tiles fill the CUs once or more with a
     // partial round left over (4 equal phases of a 4x4 stride-2 layer: 392 tiles on 256 CUs): the tiles of that
     // last round - the end of the launch order - are split along K like the tail of a single forward pass
-    // (planTiles: same cost model, the k-tiles of the heaviest phase in the tail).
+    // (planTiles: same cost model, the k-tiles of the heaviest phase in the tail), where that pays for the fold: its
+    // stores are every other float of a row, 17 us for 408 partial tiles. (256 -> 128 4x4 stride 2 on 14x14, N = 64,
+    // forward + backward: 336 us with the last round split three ways, 328 with whole tiles, two to a CU.)
     const int q = (int)(wgs / cus), r = (int)(wgs % cus);
     if (!anySplit && q > 0 && r > 0) {
       int first = set.count - 1;  // first item with tiles in the tail
@@ -2781,7 +2783,7 @@ bool gradInputByPhase(THCState *state, const ConvGeom &g, const float *gy, const
       int S = 1;
       for (int c = 2; c <= std::max(1, std::min(nktTail / 4, 16)); ++c) {
         if (launch::ceilDiv(nktTail, launch::ceilDiv(nktTail, c)) != c) continue;
-        const double t = q * perWg(nktHead, 1) + launch::ceilDiv(r * c, cus) * perWg(nktTail, c) + 0.006 * r * c;
+        const double t = q * perWg(nktHead, 1) + launch::ceilDiv(r * c, cus) * perWg(nktTail, c) + 0.05 * r * c;
         if (t < best) best = t, S = c;
       }
       if (S > 1) {
