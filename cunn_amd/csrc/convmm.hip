@@ -3224,13 +3224,12 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   const void *kern = fast ? gw.fn : (const void *)convGemmKernel<kGradWeight>;
   const int ktPositions = tiny ? kSmallPositions : BK;
   const int totalKt = launch::ceilDiv(g.N * Lk, ktPositions);
-  // Every split leaves a partial copy of gradWeight (64 KB per tile) for the fold: three workgroups per CU
-  // measured better than the four that fit (less partial traffic for the same matrix-pipe load), two when
-  // gradWeight is one or two tiles and the partials are most of the traffic. The small tiles stream: as many
-  // workgroups as fit, to have enough loads in flight.
-  // A split should keep at least about 20 k-tiles (short reductions at 14x14 and 7x7: with 8 k-tiles per split the
-  // partial copies and the pipeline fill cost more than the third workgroup per CU gains).
-  int perCu = mT * nT <= 2 ? 2 : tiny ? 4 : 3;
+  // Every split leaves a partial copy of gradWeight (64 KB per large tile) for the fold. The registers hold two workgroups
+  // of the large tiles on a CU, three or four of the small ones, which stream: as many as fit, to have enough loads in
+  // flight; two where gradWeight is one or two tiles and the partials are most of the traffic. A split should keep at
+  // least about 20 k-tiles of 16 positions (short reductions at 14x14 and 7x7: with 8 k-tiles per split the partial
+  // copies and the pipeline fill cost more than another workgroup per CU gains).
+  int perCu = mT * nT <= 2 ? 2 : tiny ? 4 : 3;  // (the large tiles' limit comes from the resident slots)
   auto splitsAt = [&](int wgPerCu) {
     const int slots = std::min(residentSlots(kern), residentSlots(nullptr) * wgPerCu);
     return std::max(1, std::min(totalKt, slots / (mT * nT)));
