@@ -909,6 +909,10 @@ convFwdImplicitKernel(FwdArgs p, ConvGeom g) {
 // (measured on registers alone: 300 TFLOP/s of fp32 products, held back by power, against 138 - 150).
 // An operand that is not finite (or rounds up to infinity as bf16) makes the result NaN or infinite; the kernels then
 // compute that block again with the fp32 instruction, so infinities, NaNs and overflows come out as they did.
+// The bf16 instruction reads subnormal parts as zero, so an operand below 2^-102 loses its last part or more: up to 2^-125
+// times the other operand per product. That is beneath the rounding of any sum that is not itself tiny; blocks with a
+// sum below 2^-80 (and not zero) are computed again with the fp32 instruction as well. (Left over: a sum all of whose
+// terms have a subnormal operand comes out as zero.)
 // (Splitting a float into bf16 parts: Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial intelligence
 // datatype for higher-precision computations", ARITH 2019.)
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -923,6 +927,13 @@ __device__ __forceinline__ void splitPair(unsigned x0, unsigned x1, unsigned &h,
   m = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
   r = f32x2{r.x - __uint_as_float(m << 16), r.y - __uint_as_float(m & 0xffff0000u)};
   l = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+}
+
+// a sum of split products that is not finite, or not zero and below 2^-80
+__device__ __forceinline__ bool redoInFp32(float v) {
+  constexpr unsigned kInf = 0x7f800000u, kLeast = (127u - 80u) << 23;
+  const unsigned u = __float_as_uint(v) & 0x7fffffffu;
+  return u != 0 && u - kLeast >= kInf - kLeast;
 }
 
 __device__ __forceinline__ bf16x8 asBf16(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
@@ -1141,7 +1152,7 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   if (kt + 1 < nkt) step(Buf1{}, Buf0{}, kt + 1, kt + 2 < nkt, false);
   if (kt + 2 < nkt) step(Buf0{}, Buf1{}, kt + 2, false, false);
 
-  float bad = 0.f;  // NaN as soon as one sum is not finite
+  bool bad = false;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1149,9 +1160,9 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
-        bad = __builtin_fmaf(acc[i][j][v], 0.f, bad);
+        bad |= redoInFp32(acc[i][j][v]);
       }
-  if (__any(bad != bad)) {
+  if (__any(bad)) {
     // the wave's blocks again in fp32, operands straight from memory
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
@@ -1282,7 +1293,7 @@ convFwdDirectKernel(FwdArgs p, ConvGeom g) {
 #pragma unroll 1
     for (int k = s0; k < s1; k += D) each([&](auto dc) { step(dc, k + D + decltype(dc)::value); });
   }
-  float bad = 0.f;  // NaN as soon as one sum is not finite
+  bool bad = false;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1290,9 +1301,9 @@ convFwdDirectKernel(FwdArgs p, ConvGeom g) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
-        bad = __builtin_fmaf(acc[i][j][v], 0.f, bad);
+        bad |= redoInFp32(acc[i][j][v]);
       }
-  if (__any(bad != bad)) {  // the slice again in fp32
+  if (__any(bad)) {  // the slice again in fp32
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1642,7 +1653,7 @@ convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
     __syncthreads();
   }
 
-  float bad = 0.f;  // NaN as soon as one sum is not finite
+  bool bad = false;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1650,9 +1661,9 @@ convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
-        bad = __builtin_fmaf(acc[i][j][v], 0.f, bad);
+        bad |= redoInFp32(acc[i][j][v]);
       }
-  if (__any(bad != bad)) {  // the wave's positions again with the fp32 instruction, straight from memory
+  if (__any(bad)) {  // the wave's positions again with the fp32 instruction, straight from memory
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
       const unsigned off = (unsigned)columnOffset(j0 + j * 32 + idx);
@@ -1910,7 +1921,7 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     if (kt + 2 < ktEnd) step(Buf0{}, Buf1{}, false, false);
   }
 
-  float bad = 0.f;  // NaN as soon as one sum is not finite
+  bool bad = false;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1918,9 +1929,9 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
-        bad = __builtin_fmaf(acc[i][j][v], 0.f, bad);
+        bad |= redoInFp32(acc[i][j][v]);
       }
-  if (__any(bad != bad)) {
+  if (__any(bad)) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const unsigned tap = (unsigned)columnOffset(j0 + wn * 64 + j * 32 + idx);

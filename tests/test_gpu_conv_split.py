@@ -56,6 +56,8 @@ def _tensors(case, kind, seed=5):
         gy *= np.exp2(np.round(rng.standard_normal(gy.shape) * 4))
     elif kind == "tiny":
         x, w = x * 1e-30, w * 1e-3
+    elif kind == "smallest":             # the parts of these would be subnormal as bf16
+        x, gy, w = x * 1e-35, gy * 1e-35, w + 2
     return tuple(v.astype(np.float32) for v in (x, w, gy))
 
 
@@ -71,7 +73,7 @@ def _passes(case, x, w, gy, gyw):
     return y.numpy(), gx.numpy(), gw.numpy()
 
 
-@pytest.mark.parametrize("kind", ["normal", "one-signed", "scaled", "tiny"])
+@pytest.mark.parametrize("kind", ["normal", "one-signed", "scaled", "tiny", "smallest"])
 @pytest.mark.parametrize("case", CASES)
 def test_error_against_64_bit_sums(case, kind):
     print("case", case, kind, flush=True)
@@ -86,7 +88,9 @@ def _check_error(case, kind):
     y = torch.nn.functional.conv2d(dx, dw, stride=st, padding=pad)
     y.backward(torch.from_numpy(gy).double())
     terms = (Ci * k * k, Co * k * k, N * gy.shape[2] * gy.shape[3])
-    for got, ref, n in zip(_passes(case, x, w, gy, gy), (y.detach(), dx.grad, dw.grad), terms):
+    gyw = gy if kind != "smallest" else (gy * np.float32(1e35)).astype(np.float32)
+    gw = torch.nn.grad.conv2d_weight(dx.detach(), dw.shape, torch.from_numpy(gyw).double(), stride=st, padding=pad)
+    for got, ref, n in zip(_passes(case, x, w, gy, gyw), (y.detach(), dx.grad, gw), terms):
         ref = ref.numpy().reshape(got.shape)
         err = np.linalg.norm(got.astype(np.float64) - ref) / np.linalg.norm(ref)
         assert err <= 2.0 ** -25 * np.sqrt(n) + 2.0 ** -24, (err, n)   # + one rounding of the result
@@ -139,7 +143,7 @@ def test_short_calls(case, shape):
     print("case", case, shape, flush=True)
     cunn_amd.set_switch("THCUNN_CONV_DIRECT", shape)
     try:
-        for kind in ("normal", "one-signed", "tiny"):
+        for kind in ("normal", "one-signed", "tiny", "smallest"):
             _check_error(case, kind)
         _check_non_finite(case, passes=2)    # forward and gradInput
     finally:
