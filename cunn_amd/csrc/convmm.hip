@@ -929,12 +929,16 @@ __device__ __forceinline__ void splitPair(unsigned x0, unsigned x1, unsigned &h,
   l = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
 }
 
-// a sum of split products that is not finite, or not zero and below 2^-80
-__device__ __forceinline__ bool redoInFp32(float v) {
-  constexpr unsigned kInf = 0x7f800000u, kLeast = (127u - 80u) << 23;
-  const unsigned u = __float_as_uint(v) & 0x7fffffffu;
-  return u != 0 && u - kLeast >= kInf - kLeast;
-}
+// Whether a wave has to compute its blocks again: any sum not finite, or not zero and below 2^-80.
+struct SumCheck {
+  float bad = 0.f;        // NaN as soon as one sum is not finite
+  unsigned least = ~0u;   // smallest magnitude seen, as the bits shifted left, minus 1: a zero counts as the largest
+  __device__ __forceinline__ void add(float v) {
+    bad = __builtin_fmaf(v, 0.f, bad);
+    least = min(least, (__float_as_uint(v) << 1) - 1u);
+  }
+  __device__ __forceinline__ bool redo() const { return __any(bad != bad || least < ((127u - 80u) << 24) - 1u); }
+};
 
 __device__ __forceinline__ bf16x8 asBf16(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
@@ -1152,7 +1156,7 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   if (kt + 1 < nkt) step(Buf1{}, Buf0{}, kt + 1, kt + 2 < nkt, false);
   if (kt + 2 < nkt) step(Buf0{}, Buf1{}, kt + 2, false, false);
 
-  bool bad = false;
+  SumCheck check;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1160,9 +1164,9 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
-        bad |= redoInFp32(acc[i][j][v]);
+        check.add(acc[i][j][v]);
       }
-  if (__any(bad)) {
+  if (check.redo()) {
     // the wave's blocks again in fp32, operands straight from memory
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
@@ -1293,7 +1297,7 @@ convFwdDirectKernel(FwdArgs p, ConvGeom g) {
 #pragma unroll 1
     for (int k = s0; k < s1; k += D) each([&](auto dc) { step(dc, k + D + decltype(dc)::value); });
   }
-  bool bad = false;
+  SumCheck check;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1301,9 +1305,9 @@ convFwdDirectKernel(FwdArgs p, ConvGeom g) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
-        bad |= redoInFp32(acc[i][j][v]);
+        check.add(acc[i][j][v]);
       }
-  if (__any(bad)) {  // the slice again in fp32
+  if (check.redo()) {  // the slice again in fp32
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1653,7 +1657,7 @@ convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
     __syncthreads();
   }
 
-  bool bad = false;
+  SumCheck check;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -1661,9 +1665,9 @@ convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
-        bad |= redoInFp32(acc[i][j][v]);
+        check.add(acc[i][j][v]);
       }
-  if (__any(bad)) {  // the wave's positions again with the fp32 instruction, straight from memory
+  if (check.redo()) {  // the wave's positions again with the fp32 instruction, straight from memory
 #pragma unroll
     for (int j = 0; j < TJ; ++j) {
       const unsigned off = (unsigned)columnOffset(j0 + j * 32 + idx);
@@ -1921,7 +1925,7 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     if (kt + 2 < ktEnd) step(Buf0{}, Buf1{}, false, false);
   }
 
-  bool bad = false;
+  SumCheck check;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1929,9 +1933,9 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         acc[i][j][v] += lo[i][j][v];
-        bad |= redoInFp32(acc[i][j][v]);
+        check.add(acc[i][j][v]);
       }
-  if (__any(bad)) {
+  if (check.redo()) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const unsigned tap = (unsigned)columnOffset(j0 + wn * 64 + j * 32 + idx);
