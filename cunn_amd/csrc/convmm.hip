@@ -907,21 +907,28 @@ convFwdImplicitKernel(FwdArgs p, ConvGeom g) {
 // 2.0e-7 / 8.6e-7 / 1.6e-6 (one-signed, badly scaled and 1e-30-sized terms: the same ratio or better).
 // The matrix pipe runs bf16 at 16 times its fp32 rate, so six products cost 6/16 of the fp32 instruction's time
 // (measured on registers alone: 300 TFLOP/s of fp32 products, held back by power, against 138 - 150).
-// An operand that is not finite (or rounds up to infinity as bf16) makes the result NaN or infinite; the kernels then
-// compute that block again with the fp32 instruction, so infinities, NaNs and overflows come out as they did.
-// The bf16 instruction reads subnormal parts as zero, so an operand below 2^-102 loses its last part or more: up to 2^-125
-// times the other operand per product. That is beneath the rounding of any sum that is not itself tiny; blocks with a
-// sum below 2^-80 (and not zero) are computed again with the fp32 instruction as well. (Left over: a sum all of whose
-// terms have a subnormal operand comes out as zero.)
+// The bf16 instruction reads subnormal parts as zero, and the last part of a float reaches 2^-23 below it. Every operand is
+// therefore multiplied by 2^24 as it is split: its parts are multiples of 2^-149 * 2^24 = 2^-125 then, none of them
+// subnormal, so the sums are as exact for the smallest floats as for any other, whatever the other operand is. The sums
+// carry 2^48, which is taken out of them at the end (their own underflow lies at 2^-174, below the smallest float). One
+// more multiplication per element: 256 -> 256 planes 3x3 at 28 x 28, N = 64, forward + backward 977 -> 990 us; 64-row tiles,
+// with half the products per element, 20.7 -> 21.6 us (64 -> 64 3x3 on 56 x 56, N = 8). (Taking the remainders with
+// v_dot2c_f32_bf16, nine instructions a pair instead of thirteen, is exact too but does not run at the full rate: 1101 us.)
+// An operand that is not finite or reaches 2^104, and a sum that reaches 2^80, make a block's results infinite or NaN; the
+// kernels then compute that block of 32 x 32 again with the fp32 instruction, so infinities, NaNs, overflows and numbers
+// of that size come out as they did.
 // (Splitting a float into bf16 parts: Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial intelligence
 // datatype for higher-precision computations", ARITH 2019.)
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// two neighbouring k -> the packed pairs of their three parts
+constexpr float kSplitScale = 0x1p24f;       // of each operand
+constexpr float kSumScale = 0x1p48f;         // of their products
+
+// two neighbouring k -> the packed pairs of the three parts of kSplitScale times them
 __device__ __forceinline__ void splitPair(unsigned x0, unsigned x1, unsigned &h, unsigned &m, unsigned &l) {
-  f32x2 r = {__uint_as_float(x0), __uint_as_float(x1)};
+  f32x2 r = {__uint_as_float(x0) * kSplitScale, __uint_as_float(x1) * kSplitScale};
   h = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
   r = f32x2{r.x - __uint_as_float(h << 16), r.y - __uint_as_float(h & 0xffff0000u)};
   m = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
@@ -929,16 +936,17 @@ __device__ __forceinline__ void splitPair(unsigned x0, unsigned x1, unsigned &h,
   l = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
 }
 
-// Whether a wave has to compute its blocks again: any sum not finite, or not zero and below 2^-80.
-struct SumCheck {
+// A block's sums from the large and the small products, without their scale. Returns (to the whole wave) whether one of
+// them is not finite, so that the block has to be computed again.
+__device__ __forceinline__ bool finishSums(float16v &acc, const float16v &lo) {
   float bad = 0.f;        // NaN as soon as one sum is not finite
-  unsigned least = ~0u;   // smallest magnitude seen, as the bits shifted left, minus 1: a zero counts as the largest
-  __device__ __forceinline__ void add(float v) {
-    bad = __builtin_fmaf(v, 0.f, bad);
-    least = min(least, (__float_as_uint(v) << 1) - 1u);
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    acc[v] = (acc[v] + lo[v]) * (1.f / kSumScale);
+    bad = __builtin_fmaf(acc[v], 0.f, bad);
   }
-  __device__ __forceinline__ bool redo() const { return __any(bad != bad || least < ((127u - 80u) << 24) - 1u); }
-};
+  return __any(bad != bad);
+}
 
 __device__ __forceinline__ bf16x8 asBf16(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
@@ -970,8 +978,8 @@ __device__ __forceinline__ void mfmaSplit(const u32x4 (&a)[3][TI], const u32x4 (
 //    scalar offset; every tap of every position is inside the padded image - no bounds test
 //  * weight rows are addressed as fixed VGPR offset + scalar k offset
 //  * the loop is unrolled over the two LDS buffers, so every LDS address is base + immediate
-//  * a k-step of a wave is 24 matrix instructions of 32 cycles, 88 vector-ALU instructions that split the next
-//    tile (they fit between the matrix instructions: leaving them out gains 5 %), 12 LDS reads and 6 LDS writes
+//  * a k-step of a wave is 24 matrix instructions of 32 cycles, 104 vector-ALU instructions that split the next
+//    tile (between the matrix instructions: leaving out all but the scaling gained 5 %), 12 LDS reads and 6 LDS writes
 // What bounds it: two workgroups per CU (128 accumulator registers per lane) keep the matrix pipe 55 % busy at a
 // clock that power has pulled down to 2.05 GHz. 256 -> 256 planes 3x3 at 28 x 28, N = 64 (59.2 GFLOP):
 // 430 us with v_mfma_f32_32x32x2_f32, 307 us (193 TFLOP/s) on the parts.
@@ -1143,7 +1151,7 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
     for (int j = 0; j < TJ; ++j) {
       acc[i][j] = biasBlock(i);
 #pragma unroll
-      for (int v = 0; v < 16; ++v) lo[i][j][v] = 0.f;
+      for (int v = 0; v < 16; ++v) acc[i][j][v] *= kSumScale, lo[i][j][v] = 0.f;
     }
   }
   int kt = ktBegin;
@@ -1156,41 +1164,29 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
   if (kt + 1 < nkt) step(Buf1{}, Buf0{}, kt + 1, kt + 2 < nkt, false);
   if (kt + 2 < nkt) step(Buf0{}, Buf1{}, kt + 2, false, false);
 
-  SumCheck check;
 #pragma unroll
-  for (int i = 0; i < TI; ++i)
+  for (int j = 0; j < TJ; ++j)
 #pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        acc[i][j][v] += lo[i][j][v];
-        check.add(acc[i][j][v]);
-      }
-  if (check.redo()) {
-    // the wave's blocks again in fp32, operands straight from memory
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) {
+    for (int i = 0; i < TI; ++i) {
+      if (!finishSums(acc[i][j], lo[i][j])) continue;
+      // the block again in fp32, operands straight from memory
       const int cOff = columnOffset((unsigned)j0 + wn * 32 * TJ + j * 32 + idx);
-#pragma unroll
-      for (int i = 0; i < TI; ++i) {
-        const int rOff = min(m0 + wm * 64 + i * 32 + idx, p.M - 1) * g.K;
-        float16v c = biasBlock(i);
+      const int rOff = min(m0 + wm * 64 + i * 32 + idx, p.M - 1) * g.K;
+      float16v c = biasBlock(i);
 #pragma unroll 1
-        for (int k = ktBegin * BK; k < nkt * BK; k += 8) {
-          float av[4], bv[4];
+      for (int k = ktBegin * BK; k < nkt * BK; k += 8) {
+        float av[4], bv[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int kk = k + 2 * u + grp;
-            av[u] = p.w[rOff + kk];
-            bv[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, cOff + (LINEAR ? kk * p.tapStride : p.taps[kk]), 0, 0));
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u], bv[u], c, 0, 0, 0);
+        for (int u = 0; u < 4; ++u) {
+          const int kk = k + 2 * u + grp;
+          av[u] = p.w[rOff + kk];
+          bv[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, cOff + (LINEAR ? kk * p.tapStride : p.taps[kk]), 0, 0));
         }
-        acc[i][j] = c;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u], bv[u], c, 0, 0, 0);
       }
+      acc[i][j] = c;
     }
-  }
   fwdEpilogue<TBN, TI, TJ>(p, g, acc, bx, by, m0, j0, wm, wn, grp, idx, biasS, whole ? 0 : 1, whole);
 }
 
@@ -1297,33 +1293,22 @@ convFwdDirectKernel(FwdArgs p, ConvGeom g) {
 #pragma unroll 1
     for (int k = s0; k < s1; k += D) each([&](auto dc) { step(dc, k + D + decltype(dc)::value); });
   }
-  SumCheck check;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int j = 0; j < TJ; ++j)
+    for (int j = 0; j < TJ; ++j) {
+      if (!finishSums(acc[i][j], lo[i][j])) continue;
+      float16v c;  // the block's share of the slice again in fp32
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        acc[i][j][v] += lo[i][j][v];
-        check.add(acc[i][j][v]);
-      }
-  if (check.redo()) {  // the slice again in fp32
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) {
-        float16v c;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) c[v] = 0.f;
+      for (int v = 0; v < 16; ++v) c[v] = 0.f;
 #pragma unroll 1
-        for (int k = s0 * 8; k < s1 * 8; ++k) {
-          const float av = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wr, rowOff[i], k * 4, 0));
-          const float bv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, posOff[j], LINEAR ? k * p.tapStride : p.taps[k], 0));
-          c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
-        }
-        acc[i][j] = c;
+      for (int k = s0 * 8; k < s1 * 8; ++k) {
+        const float av = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wr, rowOff[i], k * 4, 0));
+        const float bv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, posOff[j], LINEAR ? k * p.tapStride : p.taps[k], 0));
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
       }
-  }
+      acc[i][j] = c;
+    }
 
   // rows 8 * (r % 4) + 4 * (lane / 32) .. + 3 of block (r / 4 / TJ, r / 4 % TJ) at column lane % 32
   auto finish = [&](int r, float4 v) {
@@ -1657,41 +1642,30 @@ convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
     __syncthreads();
   }
 
-  SumCheck check;
 #pragma unroll
-  for (int i = 0; i < TI; ++i)
+  for (int j = 0; j < TJ; ++j)
 #pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        acc[i][j][v] += lo[i][j][v];
-        check.add(acc[i][j][v]);
-      }
-  if (check.redo()) {  // the wave's positions again with the fp32 instruction, straight from memory
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) {
+    for (int i = 0; i < TI; ++i) {
+      if (!finishSums(acc[i][j], lo[i][j])) continue;
+      // the block over the wave's positions again with the fp32 instruction, straight from memory
       const unsigned off = (unsigned)columnOffset(j0 + j * 32 + idx);
+      const unsigned rOff = (unsigned)(min(m0 + i * 32 + idx, p.M - 1) * g.L * 4);
+      float16v c;
 #pragma unroll
-      for (int i = 0; i < TI; ++i) {
-        const unsigned rOff = (unsigned)(min(m0 + i * 32 + idx, p.M - 1) * g.L * 4);
-        float16v c;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) c[v] = 0.f;
+      for (int v = 0; v < 16; ++v) c[v] = 0.f;
 #pragma unroll 1
-        for (int kt = ktBegin; kt < ktEnd; ++kt)
+      for (int kt = ktBegin; kt < ktEnd; ++kt)
 #pragma unroll 1
-          for (int q = 0; q < 16; q += 2) {
-            int n, l;
-            locate((unsigned)kt * KP + wave * 16 + q + grp, n, l);
-            const unsigned at = n < g.N ? (unsigned)(n * imgStrideA + l * 4) : 0x7fffffffu;
-            const float av = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gr, (int)(at + rOff), 0, 0));
-            const float bv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, (int)((unsigned)positionOffset(n, l) + off), 0, 0));
-            c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
-          }
-        acc[i][j] = c;
-      }
+        for (int q = 0; q < 16; q += 2) {
+          int n, l;
+          locate((unsigned)kt * KP + wave * 16 + q + grp, n, l);
+          const unsigned at = n < g.N ? (unsigned)(n * imgStrideA + l * 4) : 0x7fffffffu;
+          const float av = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gr, (int)(at + rOff), 0, 0));
+          const float bv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, (int)((unsigned)positionOffset(n, l) + off), 0, 0));
+          c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
+        }
+      acc[i][j] = c;
     }
-  }
 
   // the four waves' sums; lane holds column (lane & 31), rows 8 * (v / 4) + 4 * (lane / 32) + v % 4 of each block
   float4 *fold = reinterpret_cast<float4 *>(lds);
@@ -1737,7 +1711,7 @@ convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
 //  * image, else: a lane owns one position of the k-tile and gathers groups of 4 neighbouring columns (16 lanes read
 //    16 consecutive positions, 64-byte runs); the 4 lanes of a quad then transpose their 4 x 4 elements through DPP
 // WM = 2: 128 x 128 tiles of gradWeight (Cout x K), WM = 1: 64 x 256 tiles; a wave multiplies 64 x 64 either way.
-// A partial tile whose sums are not all finite is computed again with the fp32 instruction, straight from memory.
+// A block whose sums are not all finite is computed again with the fp32 instruction, straight from memory.
 // What bounds it: as the forward kernel, two workgroups per CU and a clock that power pulls down. Against the fp32
 // instruction: 256 x 2304 over 64 x 28 x 28 positions (59.2 GFLOP) 519 -> 334 us; 192 x 720 over 32 x 71 x 71 (64 x 256
 // tiles, gathers transposed) 462 -> 342 us; 256 x 2048, stride 2, over 64 x 14 x 14 142 -> 99 us.
@@ -1925,39 +1899,28 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     if (kt + 2 < ktEnd) step(Buf0{}, Buf1{}, false, false);
   }
 
-  SumCheck check;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        acc[i][j][v] += lo[i][j][v];
-        check.add(acc[i][j][v]);
-      }
-  if (check.redo()) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int i = 0; i < 2; ++i) {
+      if (!finishSums(acc[i][j], lo[i][j])) continue;
+      // the block again with the fp32 instruction, straight from memory
       const unsigned tap = (unsigned)columnOffset(j0 + wn * 64 + j * 32 + idx);
+      const int rOff = min(m0 + wm * 64 + i * 32 + idx, p.M - 1) * g.L * 4;
+      float16v c;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int rOff = min(m0 + wm * 64 + i * 32 + idx, p.M - 1) * g.L * 4;
-        float16v c;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) c[v] = 0.f;
+      for (int v = 0; v < 16; ++v) c[v] = 0.f;
 #pragma unroll 1
-        for (int r0 = ktBegin * BK; r0 < ktEnd * BK; r0 += 2) {
-          const int r = r0 + grp, n = (int)((unsigned)r / (unsigned)g.L), l = r - n * g.L;
-          const float av = __uint_as_float(
-              __builtin_amdgcn_raw_buffer_load_b32(gr, n < g.N ? n * imgStrideA + rOff + l * 4 : kOob, 0, 0));
-          const float bv = __uint_as_float(
-              __builtin_amdgcn_raw_buffer_load_b32(xr, (int)((unsigned)positionOffset(l, n * imgStrideB) + tap), 0, 0));
-          c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
-        }
-        acc[i][j] = c;
+      for (int r0 = ktBegin * BK; r0 < ktEnd * BK; r0 += 2) {
+        const int r = r0 + grp, n = (int)((unsigned)r / (unsigned)g.L), l = r - n * g.L;
+        const float av = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(gr, n < g.N ? n * imgStrideA + rOff + l * 4 : kOob, 0, 0));
+        const float bv = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(xr, (int)((unsigned)positionOffset(l, n * imgStrideB) + tap), 0, 0));
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, c, 0, 0, 0);
       }
+      acc[i][j] = c;
     }
-  }
 
   // lane holds column (lane & 31), rows 8*(v/4) + 4*(lane/32) + v%4 of each 32x32 tile
   float *dst = p.partial + (long)split * p.M * p.Ncols;

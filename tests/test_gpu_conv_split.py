@@ -124,6 +124,64 @@ def _check_non_finite(case, passes=3):
         np.testing.assert_allclose(got[fine], r[fine], rtol=1e-5, atol=max(1e-4, 1e-6 * np.abs(r[fine], dtype=np.float64).max()))
 
 
+# Sizes of x and w (of gradOutput and x in the weight gradient): operands so small that a bf16 part of theirs would be
+# subnormal, with partners large enough that the sums are ordinary numbers; and operands and sums above the range in which
+# products are formed from parts. The bound is the one above: no size of an operand may cost precision.
+SIZES = [(1e-33, 1e16), (1e-36, 1e19), (1e19, 1e-36), (1e-38, 1e21), (1e-39, 1e22), (1e30, 1e-39), (1e-39, 1e36), (1e15, 1e17)]
+
+
+def _check_sizes(case, a, b, passes=3):
+    import torch
+    N, Ci, Co, H, W, k, st, pad = case
+    x, w, gy = _tensors(case, "normal", 8)
+    f = lambda v, s: (v.astype(np.float64) * s).astype(np.float32)
+    x, w, gyw, gy = f(x, a), f(w, b), f(gy, b), f(gy, a)
+    d = lambda v, *s: torch.from_numpy(v.reshape(*s) if s else v).double()
+    dw = d(w, Co, Ci, k, k)
+    refs = (torch.nn.functional.conv2d(d(x), dw, stride=st, padding=pad),
+            torch.nn.grad.conv2d_input(x.shape, dw, d(gy), stride=st, padding=pad),
+            torch.nn.grad.conv2d_weight(d(x), dw.shape, d(gyw), stride=st, padding=pad))
+    terms = (Ci * k * k, Co * k * k, N * gy.shape[2] * gy.shape[3])
+    for name, got, ref, n in list(zip(("output", "gradInput", "gradWeight"), _passes(case, x, w, gy, gyw), refs, terms))[:passes]:
+        ref = ref.numpy().reshape(got.shape)
+        err = np.linalg.norm(got.astype(np.float64) - ref) / np.linalg.norm(ref)
+        assert err <= 2.0 ** -25 * np.sqrt(n) + 2.0 ** -24, (name, err, n)
+
+
+@pytest.mark.parametrize("sizes", SIZES)
+@pytest.mark.parametrize("case", CASES)
+def test_small_operands_with_large_partners(case, sizes):
+    print("case", case, sizes, flush=True)
+    _check_sizes(case, *sizes)
+
+
+@pytest.mark.parametrize("direct", ["0", "1", "2"])
+def test_bias_of_any_size(direct):
+    """The sums start from the bias in some kernels and meet it at the end in others: nothing of it may be lost or overflow."""
+    case = (2, 32, 40, 9, 8, 3, 1, 1)
+    print("direct", direct, flush=True)
+    N, Ci, Co, H, W, k, st, pad = case
+    x, w, _ = _tensors(case, "normal", 9)
+    size = np.array([0, 1e-44, 1e-38, 1e-3, 1, 1e20, 1e26, 3e38])[np.arange(Co) % 8]
+    bias = (size * np.where(np.arange(Co) % 3, 1, -1)).astype(np.float32)
+    x = (x.astype(np.float64) * np.array([1, 1e-38])[:N, None, None, None]).astype(np.float32)
+    cunn_amd.set_switch("THCUNN_CONV_DIRECT", direct)
+    try:
+        THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
+        y = CT()
+        THNN.SpatialConvolutionMM_updateOutput(CT.from_numpy(x), y, CT.from_numpy(w), CT.from_numpy(bias), CT(), CT(), k, k, st, st, pad, pad)
+        got = y.numpy()
+    finally:
+        cunn_amd.set_switch("THCUNN_CONV_DIRECT", None)
+    K = Ci * k * k
+    col = np.lib.stride_tricks.sliding_window_view(np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 1), (1, 1))), (k, k), axis=(2, 3))
+    W64 = w.astype(np.float64).reshape(Co, Ci, k, k)
+    ref = np.einsum("ncijkl,ockl->noij", col, W64) + bias.astype(np.float64)[None, :, None, None]
+    terms = np.einsum("ncijkl,ockl->noij", np.abs(col), np.abs(W64)) + np.abs(bias.astype(np.float64))[None, :, None, None]
+    # K fp32 additions of what the terms add up to in magnitude, and a rounding to the smallest float
+    assert (np.abs(got - ref) <= K * 2.0 ** -24 * terms + 2.0 ** -149).all()
+
+
 # ---- the kernel for short calls: every tile shape, ragged rows and columns, fewer k-steps than waves, uneven slices ----
 DIRECT = [
     (1, 16, 8, 5, 5, 1, 1, 0),       # one k-step: three of the four waves have none
@@ -145,6 +203,8 @@ def test_short_calls(case, shape):
     try:
         for kind in ("normal", "one-signed", "tiny", "smallest"):
             _check_error(case, kind)
+        for sizes in SIZES:
+            _check_sizes(case, *sizes, passes=2)
         _check_non_finite(case, passes=2)    # forward and gradInput
     finally:
         cunn_amd.set_switch("THCUNN_CONV_DIRECT", None)
