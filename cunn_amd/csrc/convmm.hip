@@ -355,6 +355,7 @@ struct FwdArgs {
   int bm, bn;         // rows and columns of an output tile (tileShape)
   int xBytes;         // bytes of the nImages input images (< 2^31)
   int wBytes;         // padded kernel: bytes of the weights (< 2^31)
+  int kReal;          // padded kernel: k of the convolution itself; from there to K the weights are zero and the taps any valid ones
   bool vecA;
   // tail launch: tiles tile0 .. are each reduced by nSplit workgroups over ktPerSplit k-tiles;
   // their 128x128 partial tiles go to `partial` and fwdTailFixupKernel folds them
@@ -490,7 +491,8 @@ __device__ __forceinline__ void fwdEpilogue(const FwdArgs &p, const ConvGeom &g,
 
 // taps[k] = ((c*H + kh*dilH)*W + kw*dilW) * 4 for k = (c*kH + kh)*kW + kw; g is the geometry of the padded images.
 // Entries beyond Cin*kH*kW (rows padded to a multiple of BK, spare entries) point at the position's own
-// first element: valid memory, and their weights are zero or they are never used.
+// first element: valid memory, and their weights are zero or they are never used. (If that element is not finite its
+// product with a zero weight is NaN, and the second pass over such a block leaves these k out: FwdArgs::kReal.)
 // byte offset of tap k = (c, kh, kw) inside a (zero-bordered) image of g.H x g.W; 0 beyond the last tap
 __device__ __forceinline__ int tapOffset(int k, const ConvGeom &g) {
   const int KK = g.kH * g.kW;
@@ -1181,6 +1183,7 @@ __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &
           const int kk = k + 2 * u + grp;
           av[u] = p.w[rOff + kk];
           bv[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, cOff + (LINEAR ? kk * p.tapStride : p.taps[kk]), 0, 0));
+          if (kk >= p.kReal) bv[u] = 0.f;  // (times a weight of zero an infinity there would be NaN)
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u], bv[u], c, 0, 0, 0);
@@ -2480,6 +2483,7 @@ void launchFwdImplicit(hipStream_t s, const FwdPlan &pl, float *scratch, const f
   }
   p.xBytes = (int)((long)nImages * gk.Cin * gk.H * gk.W * sizeof(float));
   p.wBytes = (int)((long)M * gk.K * sizeof(float));
+  p.kReal = g.K;
   p.vecA = (gk.K % 4 == 0) && launch::aligned16(w);
   launchFwdKernels(s, pl, p, partial, gk, fast);
 }
@@ -2849,6 +2853,7 @@ bool gradInputByPhase(THCState *state, const ConvGeom &g, const float *gy, const
       }
       a.xBytes = (int)(cnt * imgFloats * 4);
       a.wBytes = (int)((long)g.Cin * P.Kp * 4);
+      a.kReal = P.K;
       a.vecA = true;
       a.mTiles = mTiles, a.bm = bm, a.bn = bn;
       a.tail = split[i].tail, a.full = split[i].tiles - split[i].tail;

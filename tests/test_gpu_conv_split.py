@@ -124,6 +124,58 @@ def _check_non_finite(case, passes=3):
         np.testing.assert_allclose(got[fine], r[fine], rtol=1e-5, atol=max(1e-4, 1e-6 * np.abs(r[fine], dtype=np.float64).max()))
 
 
+def _same_special(got, ref):
+    for f in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(f(got), f(ref)), f.__name__
+    fine = np.isfinite(ref)
+    np.testing.assert_allclose(got[fine], ref[fine], rtol=1e-5, atol=1e-4)
+
+
+# A sum whose length is no multiple of the k-tile is filled up with zero weights, and what those are multiplied with is
+# some element of the image: an infinity there must not reach outputs that it is no term of, nor turn into NaN where it is.
+@pytest.mark.parametrize("direct", ["0", None])
+@pytest.mark.parametrize("case", [(2, 8, 40, 13, 12, 3, 2, 0), (2, 6, 36, 11, 15, 5, 3, 1), (1, 8, 24, 9, 9, 2, 3, 0)])
+def test_infinities_beside_filled_up_sums(case, direct):
+    """Strided gradInput (phases of Cout x taps terms) and the transposed convolution's forward pass: infinities in the first
+    plane, which the zero weights meet."""
+    print("case", case, direct, flush=True)
+    N, Ci, Co, H, W, k, st, pad = case
+    _, w, gy = _tensors(case, "normal", 12)
+    gy[0, 0, 1, 1], gy[N - 1, 0, 0, 2], gy[0, 0, gy.shape[2] - 1, 0] = np.inf, -np.inf, np.inf
+    THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
+    g = (k, k, st, st, pad, pad)
+    cunn_amd.set_switch("THCUNN_CONV_DIRECT", direct)
+    try:
+        gx, y = CT(), CT()
+        THNN.SpatialConvolutionMM_updateGradInput(CT.from_numpy(np.zeros((N, Ci, H, W), np.float32)), CT.from_numpy(gy), gx,
+                                                  CT.from_numpy(w), CT(), CT(), *g)
+        wf, bias = w.reshape(Co, Ci, k, k), np.arange(Ci, dtype=np.float32)
+        THNN.SpatialFullConvolution_updateOutput(CT.from_numpy(gy), y, CT.from_numpy(wf), CT.from_numpy(bias), CT(), CT(), *g, 0, 0)
+    finally:
+        cunn_amd.set_switch("THCUNN_CONV_DIRECT", None)
+    with np.errstate(all="ignore"):
+        _same_special(gx.numpy(), O.convmm_updateGradInput((N, Ci, H, W), gy, w, *g))
+        _same_special(y.numpy(), O.fullconv_updateOutput(gy, wf, bias, *g))
+
+
+@pytest.mark.parametrize("relu", [False, True])
+@pytest.mark.parametrize("case", [(2, 3, 24, 21, 19, 3, 1, 1), (2, 3, 40, 15, 14, 7, 2, 3), (1, 3, 70, 9, 9, 1, 1, 0), (2, 5, 136, 10, 9, 3, 1, 0)])
+def test_infinities_beside_filled_up_sums_forward(case, relu):
+    print("case", case, relu, flush=True)
+    N, Ci, Co, H, W, k, st, pad = case
+    x, w, _ = _tensors(case, "normal", 13)
+    x[0, 0, 3, 3], x[N - 1, 0, 0, 4], x[0, 0, H - 1, W - 1] = np.inf, -np.inf, np.inf
+    THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
+    y, g = CT(), (k, k, st, st, pad, pad)
+    f = THNN.SpatialConvolutionMMReLU_updateOutput if relu else THNN.SpatialConvolutionMM_updateOutput
+    f(CT.from_numpy(x), y, CT.from_numpy(w), None, CT(), CT(), *g)
+    with np.errstate(all="ignore"):
+        ref = O.convmm_updateOutput(x, w, None, *g)
+        if relu:
+            ref = np.where(ref > 0, ref, np.float32(0))
+    _same_special(y.numpy(), ref)
+
+
 # Sizes of x and w (of gradOutput and x in the weight gradient): operands so small that a bf16 part of theirs would be
 # subnormal, with partners large enough that the sums are ordinary numbers; and operands and sums above the range in which
 # products are formed from parts. The bound is the one above: no size of an operand may cost precision.
