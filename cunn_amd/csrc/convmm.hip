@@ -3191,6 +3191,12 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
       const long c = (long)tiles(g.Cout, 32 * sh.ti) * tiles(g.K, 32 * sh.tj) * sh.cost;
       if (c < bestCost) bestCost = c, tI = sh.ti, tJ = sh.tj;
     }
+  // Short reductions: up to 16 blocks of 32 x 32 x 64 positions per CU, every larger tile leaves CUs idle, and its start and
+  // end (16 KB of sums per block folded through LDS) are most of the time. us, the shape by cost / 1x1: 136 x 64 over 64
+  // positions 10.4 / 7.5; 64 x 64 over 6480 13.0 / 9.8; 456 x 200 over 484 18.2 / 12.4; 144 x 432 over 2312 (10 per CU) 24.2 /
+  // 20.5; 240 x 2600 over 486 (20 per CU) 26.9 / 27.1; 368 x 288 over 5184 (34 per CU) 33.1 / 32.9.
+  if (fast && tiles(g.Cout, 32) * tiles(g.K, 32) * (long)launch::ceilDiv(g.N * Lk, kSmallPositions) <= 16L * residentSlots(nullptr))
+    tI = tJ = 1;
   const bool tiny = tI > 0;
   const int mT = (int)tiles(g.Cout, tiny ? 32 * tI : wide ? 64 : BM), nT = (int)tiles(g.K, tiny ? 32 * tJ : wide ? 256 : BN);
   struct Kernel {
