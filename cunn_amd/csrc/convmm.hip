@@ -2580,11 +2580,13 @@ bool convPointwise(THCState *state, const ConvGeom &g, const float *x, const flo
   if (g.L % 4 != 0 || g.Cout % 8 != 0 || P < 32 || !pwShape(g.Cout, g.K, &sh)) return false;
   // The shortest forward calls (an image or two of 14x14 and smaller planes) go to the direct kernel; those with the
   // transposed weights stay (direct needs a launch that transposes). us, this one / direct: 64 -> 64, N = 1, 56x56:
-  // 7.8 / 5.6, transposed 7.5 / 8.4; 128 -> 128: 7.2 / 6.5. The 256-row shape has a long start (14 us): on mid-sized
-  // calls it loses to the other kernels in both directions (64 -> 256, N = 1 on 56x56: 14.4 / 7.5; N = 8: 17.7 / 13.9;
-  // N = 16: 21.6 / 23.3).
+  // 7.8 / 5.6, transposed 7.5 / 8.4; 128 -> 128: 7.2 / 6.5. The 256-row shape has a long start (14 us for K = 64, 20 for 32):
+  // up to 560 million products the other kernels are better. us, this one / those (forward; gradInput), at 1024 ... 75264
+  // positions: 64 -> 256, 31360 positions 19.6 / 15.7 (18.6 / 18.1), 37632: 20.2 / 22.5 (19.3 / 24.1); 64 -> 512, 12544: 18.4 /
+  // 14.8 (18.0 / 17.4), 18816: 19.9 / 22.0 (19.4 / 24.2); 64 -> 1024, 6272: 18.3 / 14.7 (18.2 / 17.8), 9408: 19.6 / 22.4 (19.1 /
+  // 24.2); 32 -> 512, 31360: 25.6 / 21.2 (25.5 / 23.4), 37632: 25.6 / 26.5 (25.5 / 29.1).
   if (g_switches.convPointwise == 1 && g_switches.convDirect < 0 &&
-      ((sh.mr == 2 && P >= 1024 && P < 40000) || (!transW && P <= 512)))
+      ((sh.mr == 2 && P >= 1024 && P * g.Cout * g.K < 560000000L) || (!transW && P <= 512)))
     return false;
   // Short runs: with fewer than three chunks per workgroup the pipeline (chunk c multiplied, c + 1 in registers,
   // c + 2 in flight) never fills; chunks of half the size do better there (128 -> 128 at 28 x 28, N = 64, 7 column
