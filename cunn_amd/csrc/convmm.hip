@@ -18,6 +18,7 @@
 //                      of images into `gradColumns`, then the col2im gather of
 //                      lib/THCUNN/im2col.h:63-102 over the group.
 #include <atomic>
+#include <climits>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -2269,10 +2270,20 @@ struct FwdPlan {
   long scratchFloats;  // tap table, tail partials, padded images
 };
 // Shape of the output tiles for M rows (others: the padded kernel's shapes beside 128 x 128 may be used).
-void tileShape(int M, bool others, int &bm, int &bn) {
+// tiles64, kTiles64: the output in 64 x 128 tiles, and the k-tiles of all of them together.
+void tileShape(int M, bool others, long tiles64, long kTiles64, int &bm, int &bn) {
   const long r128 = tiles(M, BM) * (long)BM, r64 = tiles(M, 64) * 64L, r96 = tiles(M, 96) * 96L, r32 = tiles(M, 32) * 32L;
   bm = BM, bn = BN;
   if (!others) return;
+  // Short calls - one round of 64 x 128 tiles with short sums, or little work altogether - are bound by the start and end of
+  // a workgroup, which the 64 x 128 shape has the shortest of. us, 64 rows / 96 (72 -> 96 rows): 3136 positions, 4 k-tiles 7.1 /
+  // 8.9; 12544, 12: 12.3 / 16.5; 2178, 21: 16.5 / 17.7; beyond: 50176, 4: 15.9 / 12.9; 3362, 54: 24.8 / 22.6. 64 rows / 32 (16
+  // rows): 3136, 6: 7.6 / 9.7; 12544, 12: 12.9 / 12.5; beyond: 200704, 2: 15.7 / 13.8; 9600, 29 (32 rows): 21.4 / 19.4.
+  const bool brief = (tiles64 <= residentSlots(nullptr) && kTiles64 <= 12 * tiles64) || kTiles64 < 1200;
+  if (brief && M <= 96) {
+    bm = 64;
+    return;
+  }
   // 96 x 128 where that pads a sixth fewer rows (65 ... 96 rows; its waves read LDS a third more often per product): 80 rows,
   // 3x3 of 192 planes over 32 x 71 x 71 positions 455 us in 32-row tiles, 348 in 96; 288 rows of 128 planes 24.6 in 64, 26.2
   if (r96 * 6 < std::min(r64, r128) * 5)
@@ -2285,7 +2296,8 @@ void tileShape(int M, bool others, int &bm, int &bn) {
 
 // Tiles of an M x Ncols output reduced over nkt k-tiles; wideOk: tileShape has its choice.
 void planTiles(FwdPlan &pl, int M, long Ncols, int nkt, bool wideOk) {
-  tileShape(M, wideOk, pl.bm, pl.bn);
+  const long tiles64 = tiles(M, 64) * (long)tiles(Ncols, 128);
+  tileShape(M, wideOk, tiles64, tiles64 * nkt, pl.bm, pl.bn);
   pl.mTiles = (int)tiles(M, pl.bm);
   pl.total = pl.mTiles * (int)tiles(Ncols, pl.bn);
   const int cus = residentSlots(nullptr);
@@ -2746,7 +2758,12 @@ bool gradInputByPhase(THCState *state, const ConvGeom &g, const float *gy, const
   // split along K so that a workgroup reduces about the same number of k-tiles whatever its phase and the
   // grid holds about two workgroups per CU. Split phases leave partial tiles for the batched fold.
   int bm, bn;
-  tileShape(g.Cin, true, bm, bn);
+  long tiles64 = 0, kTiles64 = 0;  // (up to 32 rows: the splits below make up for few tiles better than 64-row tiles do, so those
+  for (int i = 0; i < set.count && g.Cin > 32; ++i) {  // never count as a short call: 192 -> 8 4x4 stride 4, N = 33: 20.6 against 26.3 us)
+    const long t = tiles(g.Cin, 64) * (long)tiles((long)std::min(group, g.N) * set.ph[i].h.n * set.ph[i].w.n, 128);
+    tiles64 += t, kTiles64 += t * (set.ph[i].Kp / BK);
+  }
+  tileShape(g.Cin, true, tiles64, g.Cin > 32 ? kTiles64 : LONG_MAX, bm, bn);
   const int mTiles = (int)tiles(g.Cin, bm);
   struct Split {
     int tiles, tail, nSplit, ktPerSplit;  // the last `tail` of the item's tiles are split nSplit ways
