@@ -2336,21 +2336,28 @@ void planTiles(FwdPlan &pl, int M, long Ncols, int nkt, bool wideOk) {
 inline long partialFloats(const FwdPlan &pl) { return pl.tail ? (long)pl.tail * pl.nSplit * BM * BN : 0; }
 
 // Whether a short call runs on convFwdDirectKernel: one launch, against workgroup tiles that would leave CUs idle or
-// have K split over workgroups, with partial tiles in memory and a second launch that folds them. Both times in us,
-// fitted to measured calls (tiled / direct): 512 -> 512 1x1 on 14x14, N = 1: 9.8 / 6.3; 256 -> 256 1x1 on 14x14, N = 8:
-// 12.8 / 7.7; 128 -> 128 3x3 on 28x28, N = 2: 20.4 / 14.6; 256 -> 64 1x1 on 56x56, N = 8: 12.5 / 15.6; 64 -> 128 1x1 on
-// 28x28, N = 16: 9.4 / 10.6; 128 -> 512 1x1 on 28x28, N = 8: 13.7 / 20.7; 256 -> 256 3x3 on 14x14, N = 1: 18.0 / 21.8.
+// have K split over workgroups, with partial tiles in memory and a second launch that folds them. Both times in us, without
+// the copies that both need, fitted to 320 calls of 1x1 ... 5x5 windows, strides 1, 2 and 4, up to 4 GFLOP (taking the estimated
+// better one costs 0.5 % over the better one). E.g. (tiled / direct): 512 -> 512 1x1 on 14x14, N = 1: 9.8 / 6.3; 256 -> 256 1x1 on
+// 14x14, N = 8: 12.8 / 7.7; 128 -> 128 3x3 on 28x28, N = 2: 20.4 / 14.6; 256 -> 64 1x1 on 56x56, N = 8: 12.5 / 15.6; 128 -> 512 1x1
+// on 28x28, N = 8: 13.7 / 20.7; 256 -> 32 1x1 on 28x28, N = 48: 21.5 / 19.2. With a stride the lanes' loads touch more cache lines:
+// 64 -> 620 4x4 stride 4, 160 positions: 20.6 / 32.0.
 // 32 x 32 tiles while those are few, then 64 x 64 (fewer loads per product; the line between them: 64 -> 64 3x3 on
-// 56x56, N = 4, 784 tiles of 32 x 32: 23.9 / 20.0; 256 -> 256 1x1 on 14x14, N = 8, 392 tiles: 7.7 / 9.8).
-void planDirect(FwdPlan &pl, int M, long Ncols, int nkt) {
+// 56x56, N = 4, 784 tiles of 32 x 32: 23.9 / 20.0; 256 -> 256 1x1 on 14x14, N = 8, 392 tiles: 7.7 / 9.8), which 32 rows cannot
+// fill (the last call above with 64 x 64: 25.5).
+void planDirect(FwdPlan &pl, int M, long Ncols, int nkt, bool window, bool strided) {
   const int force = g_switches.convDirect;
   if (force == 0) return;
   const long tiles32 = (long)tiles(M, 32) * tiles(Ncols, 32);
-  const bool small = tiles32 <= 512;
+  const bool small = tiles32 <= 512 || M <= 32;
   if (force < 0) {
     if (pl.total >= residentSlots(nullptr)) return;  // a workgroup tile for every CU: the tiled kernel is better at any size
-    const double tiled = 6.0 + (pl.bm == 64 ? 0.55 : 0.85) * pl.ktPerSplit + (pl.tail > 0 ? 5.0 + 0.02 * pl.tail * pl.nSplit : 0.0);
-    const double direct = 4.5 + 0.002 * tiles32 + std::max(0.13 * nkt, (small ? 0.65e-3 : 0.45e-3) * tiles32 * nkt);
+    const double tiled = pl.tail > 0 ? (pl.bm == BM ? 6.3 : 4.6) + 0.85 * pl.ktPerSplit + 0.025 * pl.tail * pl.nSplit
+                         : pl.bm == BM ? 4.7 + 1.15 * pl.ktPerSplit
+                                       : 3.4 + 0.66 * pl.ktPerSplit;
+    const double perStep = !small ? 0.25 : strided ? 0.13 : window ? 0.11 : 0.08;   // bound by latency
+    const double perTile = !small ? 0.4e-3 : strided ? 0.72e-3 : 0.45e-3;           // bound by loads
+    const double direct = 4.3 + 0.002 * tiles32 + std::max(perStep * nkt, perTile * tiles32 * nkt);
     if (direct >= tiled) return;
   }
   pl.direct = force > 0 ? force : small ? 1 : 2;
@@ -2370,7 +2377,7 @@ FwdPlan planFwdImplicit(int M, int nImages, const ConvGeom &g, bool wAligned = t
   const int Kp = nkt * BK;
   const bool fast = !forceGeneric() && padded * 4 < 0x7fffffffL && (long)M * Kp * 4 < 0x7fffffffL;
   planTiles(pl, M, (long)nImages * g.L, nkt, fast);
-  if (fast && direct && g.K % BK == 0 && g.Cin % 2 == 0) planDirect(pl, M, (long)nImages * g.L, nkt);
+  if (fast && direct && g.K % BK == 0 && g.Cin % 2 == 0) planDirect(pl, M, (long)nImages * g.L, nkt, g.kH * g.kW > 1, g.dW > 1);
   pl.tapEntries = fast ? Kp + 2 * BK : 0;  // spare entries: the kernel reads tap offsets up to two k-tiles ahead
   pl.paddedFloats = fast && (g.padH > 0 || g.padW > 0) ? padded : 0;
   pl.weightFloats = fast && (Kp != g.K || !wAligned) ? (long)M * Kp : 0;
