@@ -540,12 +540,13 @@ __device__ __forceinline__ void flipWeights(const FlipJob &f, int block, int blo
 }
 
 // xp(nc, Hp, Wp) = x(nc, H, W) at row padTop, column padLeft inside zeros, for any plane size and count: a workgroup
-// writes one run of kPadRun floats of the destination with 16-byte stores, wherever planes begin and end in it. One
+// writes one run of 1024 U floats of the destination with 16-byte stores, wherever planes begin and end in it. One
 // scalar division per workgroup locates the run; inside it a lane's offsets are small, so the reciprocal divisions
-// are exact (a dividend below d + kPadRun with d < kPadRun; a larger d is passed at most once). The four elements of
+// are exact (a dividend below d + the run with d below the run; a larger d is passed at most once). The four elements of
 // a group are found by stepping. Bound by memory: 6144 planes 71 x 71 -> 75 x 75 (262 MB) 103 us with a lane per
 // element and a workgroup per 256 elements of a plane, 48 us (5.4 TB/s) in this form.
-constexpr int kPadRun = 4096;
+// U = 1: runs of 1024 for destinations that would leave CUs without one of 4096 (64 planes 33 x 33: 4.2 us with U = 4, 2.9 so).
+template <int U>
 __global__ void __launch_bounds__(dev::kBlock)
 padPlanesRunKernel(const float *__restrict__ x, float *__restrict__ xp, int H, int W, int padTop, int padLeft, int Hp, int Wp,
                    long total, int copyBlocks, bool vec, int *taps, int tapEntries, ConvGeom tg, int tapBlocks, FlipJob flip) {
@@ -558,15 +559,16 @@ padPlanesRunKernel(const float *__restrict__ x, float *__restrict__ xp, int H, i
       taps[k] = tapOffset(k, tg);
     return;
   }
+  constexpr int kPadRun = 4 * U * dev::kBlock;
   const int plane = Hp * Wp;
   const unsigned magicPlane = dev::magicOf(plane), magicW = dev::magicOf(Wp);
   const long e0 = (long)blockIdx.x * kPadRun;
   const long pl0 = e0 / plane;
   const int r0 = (int)(e0 - pl0 * plane), h0 = r0 / Wp, c0 = r0 - h0 * Wp;
   const float *src = x + pl0 * H * W;
-  float v[4][4];
+  float v[U][4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int o = (u * dev::kBlock + threadIdx.x) * 4;
     const int r = r0 + o;
     int pl = plane < kPadRun ? dev::fastDiv(r, magicPlane) : r >= plane;
@@ -587,7 +589,7 @@ padPlanesRunKernel(const float *__restrict__ x, float *__restrict__ xp, int H, i
     }
   }
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < U; ++u) {
     const long e = e0 + (u * dev::kBlock + threadIdx.x) * 4;
     if (vec && e + 4 <= total) {
       *reinterpret_cast<float4 *>(xp + e) = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
@@ -660,6 +662,8 @@ padPlanesFlatKernel(const float *__restrict__ x, float *__restrict__ xp, int H, 
   padFlatVecBody(x, xp, H, W, padTop, padLeft, Hp, Wp, total4, copyBlocks);
 }
 
+int residentSlots(const void *kernel);
+
 // taps != nullptr: the same launch also builds the tap table (tapEntries entries) of geometry tg
 // flip != nullptr: and flips the weights of *flip (the flat kernels take the job along; otherwise a launch of its own)
 void launchPadPlanes(hipStream_t s, const float *x, float *xp, long planes, int H, int W, int padTop, int padLeft, int Hp,
@@ -683,9 +687,11 @@ void launchPadPlanes(hipStream_t s, const float *x, float *xp, long planes, int 
     padPlanesFlatKernel<true><<<copyBlocks + tapBlocks + flipBlocks, dev::kBlock, 0, s>>>(
         x, xp, H, W, padTop, padLeft, Hp, Wp, total, copyBlocks, taps, tapEntries, g, tapBlocks, fj);
   } else {
-    const long total = planes * plane, copyBlocks = (total + kPadRun - 1) / kPadRun;
+    const long total = planes * plane;
+    const int run = total <= 4096L * residentSlots(nullptr) ? 1024 : 4096;
+    const long copyBlocks = (total + run - 1) / run;
     if (copyBlocks + tapBlocks + flipBlocks > 0x7fffffffL) error("SpatialConvolutionMM: batch too large");
-    padPlanesRunKernel<<<(unsigned)copyBlocks + tapBlocks + flipBlocks, dev::kBlock, 0, s>>>(
+    (run == 1024 ? padPlanesRunKernel<1> : padPlanesRunKernel<4>)<<<(unsigned)copyBlocks + tapBlocks + flipBlocks, dev::kBlock, 0, s>>>(
         x, xp, H, W, padTop, padLeft, Hp, Wp, total, (int)copyBlocks, launch::aligned16(xp), taps, tapEntries, g, tapBlocks, fj);
   }
   THC_HIP_CHECK(hipGetLastError());

@@ -41,6 +41,8 @@ CASES = [
     (2, 8, 24, 67, 61, 3, 1, 1),
     (33, 64, 8, 37, 35, 3, 1, 1),
     (1, 8, 16, 3, 4500, 3, 1, 1),
+    (9, 32, 8, 67, 61, 3, 1, 1),      # the same in longer runs
+    (2, 32, 8, 3, 4500, 3, 1, 1),
 ]
 
 
