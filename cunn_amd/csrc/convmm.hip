@@ -1,21 +1,26 @@
-// SpatialConvolutionMM for gfx950: im2col/col2im + fp32 MFMA GEMM.
+// SpatialConvolutionMM for gfx950: implicit im2col GEMM on the matrix cores, fp32 in and out.
 //
 // The reference loops over the batch and per image launches im2col, an SGEMM
 // and (for the bias) a k=1 SGEMM, writing a (Cin*kH*kW) x (oH*oW) column
 // buffer to memory and reading it back
 // (lib/THCUNN/generic/SpatialConvolutionMM.cu:129-194, 272-308, 396-470).
-// Here each entry point is one batched GEMM over the whole mini-batch built on
-// v_mfma_f32_32x32x2_f32 with LDS-staged 128x128x16 tiles:
+// Here each entry point is one batched GEMM over the whole mini-batch. Most kernels
+// multiply fp32 operands as products of three bf16 parts each, accumulated in fp32
+// (v_mfma_f32_32x32x16_bf16; "fp32 products on the bf16 matrix pipe" below); the 1x1
+// kernel of 32 / 64 / 128 planes, the few-plane gradInput and the general fallbacks use the
+// fp32 matrix instruction.
 //   updateOutput       C[o][n,l]  = bias[o] + sum_k W[o][k] * col[k][n,l]
-//                      col is never stored: the B-tile loader gathers it from
-//                      the NCHW input on the fly (implicit im2col, zero padded)
+//                      col is never stored: the B-tile loader gathers it from a
+//                      zero-bordered copy of the input on the fly (implicit im2col)
 //   accGradParameters  gW[o][k]  += scale * sum_{n,l} gy[n][o][l] * col[k][n,l]
-//                      split over groups of images; partial products go to the
+//                      split over groups of positions; partial products go to the
 //                      caller's `columns` scratch and are folded in a fixed
-//                      order (deterministic, no atomics); gradBias is a
-//                      separate 64-lane shuffle reduction
-//   updateGradInput    gradCol[k][n,l] = sum_o W[o][k] * gy[n][o][l] for a group
-//                      of images into `gradColumns`, then the col2im gather of
+//                      order (deterministic, no atomics); gradBias rides along
+//                      where the fold can take it, else it is a pass of its own
+//   updateGradInput    stride 1: the forward kernels on gradOutput with flipped
+//                      weights; other strides: the same phase by phase; what neither
+//                      takes: gradCol[k][n,l] = sum_o W[o][k] * gy[n][o][l] for a group of
+//                      images into `gradColumns`, then the col2im gather of
 //                      lib/THCUNN/im2col.h:63-102 over the group.
 #include <atomic>
 #include <climits>
@@ -601,10 +606,6 @@ padPlanesRunKernel(const float *__restrict__ x, float *__restrict__ xp, int H, i
   }
 }
 
-// The same for small planes (7x7 ... 28x28 stages: a workgroup per plane would leave most lanes idle): a lane per
-// 16-byte group of the whole destination. Workgroups past copyBlocks build the tap table.
-// ANY: planes of any size (9x9 = a bordered 7x7 plane): a group may straddle two planes and the last elements of
-// the destination may not fill a group.
 // The copy of padPlanesFlatKernel for planes of a multiple of 4 floats: workgroups 0 .. copyBlocks - 1 of a launch, a
 // lane per 16-byte group of the bordered planes.
 __device__ __forceinline__ void padFlatVecBody(const float *__restrict__ x, float *__restrict__ xp, int H, int W, int padTop,
@@ -625,6 +626,10 @@ __device__ __forceinline__ void padFlatVecBody(const float *__restrict__ x, floa
   }
 }
 
+// The bordered copy for small planes (7x7 ... 28x28 stages): a lane per 16-byte group of the whole destination. Workgroups
+// past copyBlocks build the tap table, those behind them flip the weights.
+// ANY: planes of any size (9x9 = a bordered 7x7 plane): a group may straddle two planes and the last elements of
+// the destination may not fill a group.
 template <bool ANY>
 __global__ void __launch_bounds__(dev::kBlock)
 padPlanesFlatKernel(const float *__restrict__ x, float *__restrict__ xp, int H, int W, int padTop, int padLeft, int Hp, int Wp,
@@ -665,7 +670,7 @@ padPlanesFlatKernel(const float *__restrict__ x, float *__restrict__ xp, int H, 
 int residentSlots(const void *kernel);
 
 // taps != nullptr: the same launch also builds the tap table (tapEntries entries) of geometry tg
-// flip != nullptr: and flips the weights of *flip (the flat kernels take the job along; otherwise a launch of its own)
+// flip != nullptr: and flips the weights of *flip
 void launchPadPlanes(hipStream_t s, const float *x, float *xp, long planes, int H, int W, int padTop, int padLeft, int Hp,
                      int Wp, int *taps = nullptr, int tapEntries = 0, const ConvGeom *tg = nullptr, const FlipJob *flip = nullptr) {
   const int plane = Hp * Wp;
@@ -1018,6 +1023,9 @@ __device__ __forceinline__ void put4(float *dst, u32x4 v) {
 // clock that power has pulled down to 2.05 GHz. 256 -> 256 planes 3x3 at 28 x 28, N = 64 (59.2 GFLOP):
 // 430 us with v_mfma_f32_32x32x2_f32, 307 us (193 TFLOP/s) on the parts.
 // Rows past M and columns past the batch are clamped to valid ones and dropped in the epilogue.
+// (bx, by): position among the tiles that start at tile0, and split; whole: the workgroup reduces all of K of tile bx and
+// writes the output itself, else it leaves a partial tile. LINEAR: 1x1 windows - the tap offsets are an arithmetic sequence,
+// computed by the scalar unit instead of read from the table.
 // WM = 2: 128 x 128 tiles, the four waves as 2 x 2, 64 x 64 each. For row counts that would leave much of a 128-row tile
 // empty (tileShape) the four waves sit side by side: WM = 1: 64 x 128 tiles, 64 x 32 a wave; WM = 3: 96 x 128, 96 x 32;
 // WM = 0: 32 x 256, 32 x 64. WM = 1 keeps three workgroups on a CU; with 64 x 256 tiles (64 x 64 a wave, two workgroups)
@@ -3186,8 +3194,8 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   // kernel.
   // The second-generation kernel loads 4 consecutive positions of a gradOutput row as one 16-byte group. Rows
   // whose length is not a multiple of 4 (7x7, 13x13, 27x27 ... planes) or that start off a 16-byte boundary are
-  // first copied into rows padded with zeros to a multiple of 4: the added positions contribute nothing (the
-  // kernel lets them read position 0 of the image).
+  // first copied into rows padded with zeros to a multiple of 4: the added positions contribute nothing (on the image's
+  // side they are out of range, which reads as 0 too).
   const int Lp = launch::roundUp(g.L, 4);
   const bool padGy = !forceGeneric() && (g.L % 4 != 0 || !launch::aligned16(gy)) && Lp >= BK;
   const int Lk = padGy ? Lp : g.L;  // positions per image as the kernel sees them

@@ -1,8 +1,8 @@
 """Convolutions multiply fp32 operands as six products of bf16 parts (SpatialConvolutionMM,
 lib/THCUNN/generic/SpatialConvolutionMM.cu:58-486). Checked here: the error against a 64-bit sum stays below what
-fp32 additions alone would give, also for one-signed and badly scaled operands, and infinities, NaNs and values that
-would round up to infinity as bf16 come out exactly as an fp32 convolution gives them (an operand that is not finite
-must not spread to outputs it does not reach).
+fp32 additions alone would give, also for one-signed and badly scaled operands and for the smallest floats beside the
+largest, and infinities, NaNs and values that would round up to infinity as bf16 come out exactly as an fp32 convolution
+gives them (an operand that is not finite must not spread to outputs it does not reach).
 
 Bound of the error: a chain of K fp32 additions rounds K times, each by at most 2^-24 of the partial sum, with random
 sign: about 2^-24 sqrt(K) / 2 of the result's norm for operands of mixed sign, and for one-signed operands (partial
