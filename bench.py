@@ -41,7 +41,10 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0        # MI355X HBM3E
-FP32_MFMA_PEAK_TFLOPS = 157.3
+# fp32 products of the convolutions: most kernels form one as six products of bf16 parts (dense bf16: 2.5 PFLOP/s), so this is
+# what bounds them; the fp32 matrix instruction (157.3), which the 1x1 kernel of 32 / 64 / 128 planes and the few-plane
+# gradInput use, is below it
+MFMA_PEAK_TFLOPS = 2500.0 / 6
 METRIC = "DW-conv fwd+bwd images/s + achieved HBM GB/s (% of peak), 1 MI355X"
 
 # HBM bytes per entry-point call, measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (KiB per dispatch) and kept
@@ -779,7 +782,7 @@ def run_workload(name, steps, warmup, hip, stream, nsets, cpu_seconds, ceiling=F
             if kind == "bytes":
                 scale, peak, unit = 1e9, HBM_PEAK_GBS, "GB/s"
             else:
-                scale, peak, unit = 1e12, FP32_MFMA_PEAK_TFLOPS, "TFLOP/s"
+                scale, peak, unit = 1e12, MFMA_PEAK_TFLOPS, "TFLOP/s"
             amount = max(amount, 1)       # entry points with no algorithmic traffic of their own (the unfused ReLU steps)
             kern[n] = dict(avg_ms=avg, median_ms=med, min_ms=float(np.min(per_kernel[n])), samples=len(per_kernel[n]),
                            achieved=amount / (avg * 1e-3) / scale, achieved_median=amount / (med * 1e-3) / scale,
@@ -788,7 +791,7 @@ def run_workload(name, steps, warmup, hip, stream, nsets, cpu_seconds, ceiling=F
         return kern
 
     step_work = sum(wl["work"][n][0] for n in names)
-    step_scale, step_peak = (1e9, HBM_PEAK_GBS) if wl["bound"] == "hbm" else (1e12, FP32_MFMA_PEAK_TFLOPS)
+    step_scale, step_peak = (1e9, HBM_PEAK_GBS) if wl["bound"] == "hbm" else (1e12, MFMA_PEAK_TFLOPS)
 
     def step_frac(ms):
         return round(step_work / (ms * 1e-3) / step_scale / step_peak, 4)
