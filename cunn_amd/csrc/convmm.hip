@@ -1019,9 +1019,9 @@ __device__ __forceinline__ void put4(float *dst, u32x4 v) {
 //  * the loop is unrolled over the two LDS buffers, so every LDS address is base + immediate
 //  * a k-step of a wave is 24 matrix instructions of 32 cycles, 104 vector-ALU instructions that split the next
 //    tile (between the matrix instructions: leaving out all but the scaling gained 5 %), 12 LDS reads and 6 LDS writes
-// What bounds it: two workgroups per CU (128 accumulator registers per lane) keep the matrix pipe 55 % busy at a
-// clock that power has pulled down to 2.05 GHz. 256 -> 256 planes 3x3 at 28 x 28, N = 64 (59.2 GFLOP):
-// 430 us with v_mfma_f32_32x32x2_f32, 307 us (193 TFLOP/s) on the parts.
+// What bounds it: two workgroups per CU (128 accumulator registers per lane) keep the matrix pipe 53 % busy at a
+// clock that power has pulled down to about 2 GHz. 256 -> 256 planes 3x3 at 28 x 28, N = 64 (59.2 GFLOP):
+// 430 us with v_mfma_f32_32x32x2_f32, 315 us (188 TFLOP/s) on the parts.
 // Rows past M and columns past the batch are clamped to valid ones and dropped in the epilogue.
 // (bx, by): position among the tiles that start at tile0, and split; whole: the workgroup reduces all of K of tile bx and
 // writes the output itself, else it leaves a partial tile. LINEAR: 1x1 windows - the tap offsets are an arithmetic sequence,
@@ -1029,8 +1029,9 @@ __device__ __forceinline__ void put4(float *dst, u32x4 v) {
 // WM = 2: 128 x 128 tiles, the four waves as 2 x 2, 64 x 64 each. For row counts that would leave much of a 128-row tile
 // empty (tileShape) the four waves sit side by side: WM = 1: 64 x 128 tiles, 64 x 32 a wave; WM = 3: 96 x 128, 96 x 32;
 // WM = 0: 32 x 256, 32 x 64. WM = 1 keeps three workgroups on a CU; with 64 x 256 tiles (64 x 64 a wave, two workgroups)
-// 64 -> 64 3x3 on 56x56 took, at N = 8 / 16 / 32, 33.7 / 49.0 / 65.9 us, now 32.5 / 42.1 / 61.6; 3 -> 64 7x7 stride 2 on
-// 224x224, N = 32: 83.9, now 75.0; 256 -> 64 1x1 on 56x56, N = 8: 21.0, now 12.5.
+// 64 -> 64 3x3 on 56x56 took, at N = 8 / 16 / 32, 33.7 / 49.0 / 65.9 us, with these 32.5 / 42.1 / 61.6; 3 -> 64 7x7 stride 2 on
+// 224x224, N = 32: 83.9 and 75.0; 256 -> 64 1x1 on 56x56, N = 8: 21.0 and 12.5. (Both before operands were scaled as they are
+// split, which costs 3 - 6 % here: 14.3 us now for the last kernel, 70 for the 7x7 one.)
 template <int WM, bool LINEAR = false>
 __device__ __forceinline__ void fwdPaddedBody(const FwdArgs &p, const ConvGeom &g, int bx, int by, bool whole) {
   constexpr int TBM = WM == 0 ? 32 : WM == 2 ? 128 : WM == 3 ? 96 : 64, TBN = WM == 0 ? 256 : 128;
@@ -3218,7 +3219,8 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   // the one with the least tiles x cost of a tile per position, in proportion to measured times: 64 x 147 over
   // 32 x 112 x 112 positions, stride 2 (us, without the bordered copy): 10 tiles of 1x1 105, 6 of 1x2 107, 5 of 2x1 83,
   // 3 of 2x2 80, one of 64 x 256 86; 64 x 576 over 32 x 56 x 56, stride 1: 86, 72, 72, 56, 51 (16-byte gathers). The
-  // first took 116 with the fp32 instruction (2x1), the second 81 (128 x 128).
+  // first took 116 with the fp32 instruction (2x1), the second 81 (128 x 128). (All of the split ones are 2 - 3 % longer now
+  // that operands are scaled as they are split: the 2x2 kernel of the first 98 -> 100 us in a whole pass.)
   struct Shape {
     int ti, tj, cost;
   };
