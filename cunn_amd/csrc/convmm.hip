@@ -2604,9 +2604,16 @@ void launchPointwiseShape(hipStream_t s, PwArgs p, int device) {
 }
 
 // out(N, M, L) = bias + W(M x K) x(N, K, L) on the weight-stationary kernel; false: the shape is not one of its.
+// Whether the library may give the caller's buffer the size it needs.
+bool growable(const THCudaTensor *buffer) {
+  const Storage *s = buffer ? erase(buffer)->storage : nullptr;
+  return buffer && (!s || ((s->flag & TH_STORAGE_RESIZABLE) && !s->allocator));
+}
+
 // transW: w holds (K x M) and its transpose is what multiplies (the gradInput pass hands over the layer's weights).
+// scratchBuf: the buffer that the other kernels would take their scratch from (this one needs none).
 bool convPointwise(THCState *state, const ConvGeom &g, const float *x, const float *w, const float *bias, float *out,
-                   bool relu = false, bool transW = false) {
+                   const THCudaTensor *scratchBuf, bool relu = false, bool transW = false) {
   if (forceGeneric() || g_switches.convPointwise == 0) return false;
   if (g.kH != 1 || g.kW != 1 || g.dH != 1 || g.dW != 1 || g.padH != 0 || g.padW != 0) return false;
   const long P = (long)g.N * g.L;
@@ -2619,7 +2626,8 @@ bool convPointwise(THCState *state, const ConvGeom &g, const float *x, const flo
   // positions: 64 -> 256, 31360 positions 19.6 / 15.7 (18.6 / 18.1), 37632: 20.2 / 22.5 (19.3 / 24.1); 64 -> 512, 12544: 18.4 /
   // 14.8 (18.0 / 17.4), 18816: 19.9 / 22.0 (19.4 / 24.2); 64 -> 1024, 6272: 18.3 / 14.7 (18.2 / 17.8), 9408: 19.6 / 22.4 (19.1 /
   // 24.2); 32 -> 512, 31360: 25.6 / 21.2 (25.5 / 23.4), 37632: 25.6 / 26.5 (25.5 / 29.1).
-  if (g_switches.convPointwise == 1 && g_switches.convDirect < 0 &&
+  // (Calls whose buffer has a fixed size, or none, stay: they need no scratch here.)
+  if (g_switches.convPointwise == 1 && g_switches.convDirect < 0 && growable(scratchBuf) &&
       ((sh.mr == 2 && P >= 1024 && P * g.Cout * g.K < 560000000L) || (!transW && P <= 512)))
     return false;
   // Short runs: with fewer than three chunks per workgroup the pipeline (chunk c multiplied, c + 1 in registers,
@@ -2670,7 +2678,7 @@ bool convPointwise(THCState *state, const ConvGeom &g, const float *x, const flo
 void convForward(THCState *state, const ConvGeom &g, const float *x, const float *w, const float *bias, float *out,
                  THCudaTensor *scratchBuf, const char *bufName, bool relu = false) {
   if ((long)g.N * g.Cout == 0) return;
-  if (convPointwise(state, g, x, w, bias, out, relu)) return;
+  if (convPointwise(state, g, x, w, bias, out, scratchBuf, relu)) return;
   hipStream_t s = state->stream;
   // images per launch so that the flat column index n*L + l fits an int
   int group = (int)std::min<long>(g.N, std::max<long>(1, 0x7fffffffL / 2 / g.L));
@@ -3097,7 +3105,7 @@ void convGradInput(THCState *state, const ConvGeom &g, const float *gy, const fl
     long need = pl.scratchFloats;
     if (g.N % group != 0) need = std::max(need, planFwdImplicit(t.Cout, g.N % group, t).scratchFloats);
     // 1x1: gradInput = W^T gradOutput, a pointwise pass itself, which reads the weights as they are
-    if (convPointwise(state, t, gy, w, bias, gi, false, true)) return;
+    if (convPointwise(state, t, gy, w, bias, gi, scratchBuf, false, true)) return;
     const long wfFloats = ((long)g.Cout * g.K + 3) / 4 * 4;
     Temp tmp;
     float *buf = scratchFloats(state, scratchBuf, wfFloats + need, tmp, bufName);

@@ -83,3 +83,27 @@ def test_pointwise_long_runs_of_tiles(case, cap):
 def test_pointwise_mobilenet_layer_full_size():
     """128 -> 128 at 56 x 56, N = 64 (the pointwise layer behind the benchmark's depthwise layer)."""
     _run((64, 128, 128, 56, 56), True, seed=72)
+
+
+@pytest.mark.parametrize("case", [(2, 64, 64, 8, 8), (1, 128, 96, 14, 14), (1, 64, 256, 36, 36), (2, 256, 64, 28, 28), (1, 512, 32, 40, 40)])
+@pytest.mark.parametrize("buffer", ["fixed", "none"])
+def test_pointwise_needs_no_scratch(case, buffer):
+    """1x1 convolutions that this kernel can take need no scratch, so a buffer tensor that cannot grow is no obstacle, also
+    where another kernel would be the faster one."""
+    import torch
+    N, Ci, Co, H, W = case
+    print("case", case, buffer, flush=True)
+    THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
+    rng = np.random.default_rng(74)
+    x, gy = rng.standard_normal((N, Ci, H, W)).astype(np.float32), rng.standard_normal((N, Co, H, W)).astype(np.float32)
+    w = (rng.standard_normal((Co, Ci)) * np.sqrt(2.0 / Ci)).astype(np.float32)
+    g = (1, 1, 1, 1, 0, 0)
+    cols = CT.from_torch(torch.zeros(1, device="cuda")) if buffer == "fixed" else None
+    if Ci in (32, 64, 128):
+        out = CT()
+        THNN.SpatialConvolutionMM_updateOutput(CT.from_numpy(x), out, CT.from_numpy(w), None, cols, CT(), *g)
+        np.testing.assert_allclose(out.numpy(), O.convmm_updateOutput(x, w, None, *g), rtol=1e-5, atol=1e-4)
+    if Co in (32, 64, 128):
+        gx = CT()
+        THNN.SpatialConvolutionMM_updateGradInput(CT.from_numpy(x), CT.from_numpy(gy), gx, CT.from_numpy(w), cols, CT(), *g)
+        np.testing.assert_allclose(gx.numpy(), O.convmm_updateGradInput(x.shape, gy, w, *g), rtol=1e-5, atol=1e-4)
