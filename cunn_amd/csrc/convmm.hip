@@ -2774,7 +2774,8 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
     const HalvesGemm &G = gemm[i];
     const long taps = (long)G.h.n * G.v.n;
     if (taps < 1 || G.nH < 1 || G.nW < 1) return false;
-    if (C * taps > (1 << 20)) return false;
+    // items (group, tap) are taken apart by dev::fastDiv: exact while their number, with what fills the last stages, times taps < 2^32
+    if (C * taps > (1 << 20) || (groups * taps + 8L * kStageItems) * taps >= 1L << 32) return false;
     maxTaps = std::max(maxTaps, taps);
     auto span = [](const SplitAxis &a, int n, int stride, int &low, int &high) {
       const int first = a.q0, last = a.q0 - (a.n - 1) * a.qStep;

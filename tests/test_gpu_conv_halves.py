@@ -88,6 +88,28 @@ def test_very_different_sizes(where, dil):
     assert (np.abs(y.numpy() - ref) <= Ci * k * k * 2.0 ** -24 * terms + 2.0 ** -149).all()
 
 
+@pytest.mark.parametrize("Ci, k", [(16, 224), (16, 215), (9, 200)])
+def test_windows_beyond_the_index_arithmetic(Ci, k):
+    """(groups of channels) x taps x taps at and beyond 2^32, where the division that takes (group, tap) apart is no longer exact:
+    every weight of such a window counts. One channel of large weights and elements, so a wrong one would show."""
+    print("case", Ci, k, flush=True)
+    rng = np.random.default_rng(k)
+    Co = 2
+    x = rng.standard_normal((1, Ci, k + 1, k + 1)).astype(np.float32)
+    w = np.zeros((Co, Ci, k, k), np.float32)
+    w[:, :, -1, -3:] = rng.standard_normal((Co, Ci, 3))   # the last taps of every channel
+    w[:, :, 0, :3] = rng.standard_normal((Co, Ci, 3))
+    ref = np.zeros((1, Co, 2, 2))
+    for i in range(2):
+        for j in range(2):
+            ref[0, :, i, j] = (w.astype(np.float64) * x[0, :, i:i + k, j:j + k]).sum((1, 2, 3))
+    CT, y = cunn_amd.CudaTensor, cunn_amd.CudaTensor()
+    cunn_amd.THNN.SpatialConvolutionMM_updateOutput(CT.from_numpy(x), y, CT.from_numpy(w.reshape(Co, -1)), None, CT(), CT(),
+                                                    k, k, 1, 1, 0, 0)
+    # at most 96 terms of size 1 that are not zero
+    assert np.abs(y.numpy() - ref).max() <= 96 * 2.0 ** -24 * 96
+
+
 @pytest.mark.parametrize("relu", [False, True])
 def test_bias_relu_and_buffers(relu):
     """Bias and clamp in the epilogue; a buffer tensor that is too small and cannot grow leaves the call to the other kernels."""
