@@ -2802,7 +2802,7 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   if (group < N && force < 0) return false;
   group = std::min(group, N);
 
-  // scratch: exponents, maxima and marks of the images, items, row exponents, split weights, split images, partial tiles
+  // scratch: ranges and forms of images and rows, items, split weights, split images, partial tiles
   long at = 0;
   auto take = [&](long bytes) {
     const long o = at;
@@ -2811,13 +2811,15 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   };
   int bm = 0, bn = 0;
   FwdPlan pl[kMaxHalvesJobs];
-  long partial[kMaxHalvesJobs], items[kMaxHalvesJobs], rowExp[kMaxHalvesJobs], split[kMaxHalvesJobs], splitBytes[kMaxHalvesJobs];
+  long partial[kMaxHalvesJobs], items[kMaxHalvesJobs], rowForm[kMaxHalvesJobs], split[kMaxHalvesJobs], split3[kMaxHalvesJobs];
   int itemsPad[kMaxHalvesJobs], rows = 0;
   const int chunks = launch::ceilDiv((int)(Hp * Wp), kSplitRun * dev::kBlock);
-  // slices of an image that absMaxKernel reads: enough workgroups to fill the chip, at least 4096 floats each
+  // slices of an image that rangesKernel reads, a power of two: enough workgroups to fill the chip, at least 4096 floats each
   const long perImg = (long)C * H * W;
-  const int nSlots = (int)std::max<long>(1, std::min<long>(kMaxSlots, std::min<long>(perImg / 4096, launch::ceilDiv(2048, group))));
-  const long slots = take((long)group * nSlots * 4), imgExp = take((long)group * 4), marks = take((long)group * groups * chunks * 4);
+  int nSlots = 1;
+  while (nSlots < kMaxSlots && 2 * nSlots <= perImg / 4096 && nSlots < launch::ceilDiv(2048, group)) nSlots *= 2;
+  const long slots = take((long)group * nSlots * sizeof(uint2)), imgForm = take((long)group * 4), rowRanges = take(M * (long)sizeof(uint2));
+  long minL = LONG_MAX;
   for (int i = 0; i < count; ++i) {
     const HalvesGemm &G = gemm[i];
     itemsPad[i] = launch::roundUp(groups * G.h.n * G.v.n, kStageItems);
@@ -2825,11 +2827,15 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
     planTiles(pl[i], M, (long)group * G.nH * G.nW, itemsPad[i] / kStageItems, true, 5.0, false);
     bm = pl[i].bm, bn = pl[i].bn;
     rows = launch::roundUp(M, bm);
-    splitBytes[i] = (long)rows * itemsPad[i] * 32;
-    if (splitBytes[i] >= 0x7fffffffL) return false;
-    items[i] = take((itemsPad[i] + 4 * kStageItems) * 4L), rowExp[i] = take(rows * 4L), split[i] = take(splitBytes[i]);
+    const long splitBytes = (long)rows * itemsPad[i] * 32;
+    if (splitBytes / 2 * 3 >= 0x7fffffffL) return false;
+    items[i] = take(2 * (itemsPad[i] + 4 * kStageItems) * 4L), rowForm[i] = take(rows * 4L);
+    split[i] = take(splitBytes), split3[i] = take(splitBytes / 2 * 3);
+    minL = std::min(minL, (long)G.nH * G.nW);
   }
-  const long images = take(group * imgBytes);
+  const int reach = (int)((bn - 2) / minL) + 1;  // images of a tile lie at most that far from each other
+  if ((reach + 1) * (imgBytes / 2 * 3) >= 0x7fffffffL) return false;
+  const long images = take(group * imgBytes), images3 = take(group * (imgBytes / 2 * 3));
   // several GEMMs (phases) in one launch: their tiles fill each other's last rounds, no tile is split
   if (count > 1)
     for (int i = 0; i < count; ++i)
@@ -2843,16 +2849,18 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   for (int first = 0; first < N; first += group) {
     const int cnt = std::min(group, N - first);
     const float *xg = x + (long)first * perImg;
-    const int perSlice = (int)((perImg + nSlots - 1) / nSlots + 3) / 4 * 4;
-    absMaxKernel<<<dim3(nSlots, cnt), dev::kBlock, 0, s>>>(xg, (unsigned *)(buf + slots), perImg, perSlice,
-                                                          perImg % 4 == 0 && launch::aligned16(xg));
+    RangeArgs ra{};
+    ra.x = xg, ra.slots = (uint2 *)(buf + slots), ra.perImg = perImg, ra.perSlice = (int)((perImg + nSlots - 1) / nSlots + 3) / 4 * 4;
+    ra.nSlots = nSlots, ra.vec = perImg % 4 == 0 && launch::aligned16(xg);
+    ra.w = w, ra.rows = (uint2 *)(buf + rowRanges), ra.M = M, ra.rs = rs, ra.cs = cs, ra.C = C, ra.taps = std::min(rs, cs);
+    rangesKernel<<<(unsigned)(M + cnt * nSlots), dev::kBlock, 0, s>>>(ra);
     THC_HIP_CHECK(hipGetLastError());
     SplitJobs J{};
     SplitImages &I = J.im;
-    I.x = xg, I.dst = (u32x4 *)(buf + images), I.slots = (unsigned *)(buf + slots);
-    I.exps = (int *)(buf + imgExp), I.marks = (int *)(buf + marks);
-    I.nSlots = nSlots, I.C = C, I.H = H, I.W = W, I.top = -lowH, I.left = -lowW, I.Hp = (int)Hp, I.Wp = (int)Wp;
-    I.groups = groups, I.chunks = chunks, I.oneScale = 1, I.blocks = cnt * groups * chunks, I.magicW = dev::magicOf((int)Wp);
+    I.x = xg, I.dst = (u32x4 *)(buf + images), I.dst3 = (u32x4 *)(buf + images3), I.slots = (uint2 *)(buf + slots);
+    I.forms = (int *)(buf + imgForm);
+    I.nSlots = nSlots, I.N = cnt, I.C = C, I.H = H, I.W = W, I.top = -lowH, I.left = -lowW, I.Hp = (int)Hp, I.Wp = (int)Wp;
+    I.groups = groups, I.chunks = chunks, I.reach = reach, I.blocks = cnt * groups * chunks, I.magicW = dev::magicOf((int)Wp);
     J.count = count;
     long blocks = I.blocks;
     HalvesBatch<kMaxHalvesJobs> batch{};
@@ -2861,15 +2869,17 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
     for (int i = 0; i < count; ++i) {
       const HalvesGemm &G = gemm[i];
       SplitRows &R = J.rows[i];
-      R.w = w, R.dst = (u32x4 *)(buf + split[i]), R.exps = (int *)(buf + rowExp[i]), R.items = (int *)(buf + items[i]);
+      R.w = w, R.dst = (u32x4 *)(buf + split[i]), R.dst3 = (u32x4 *)(buf + split3[i]);
+      R.ranges = (uint2 *)(buf + rowRanges), R.forms = (int *)(buf + rowForm[i]);
+      R.items = (int *)(buf + items[i]), R.items3 = R.items + itemsPad[i] + 4 * kStageItems;
       R.rs = rs, R.cs = cs, R.kW = kW, R.M = M, R.rows = rows, R.C = C, R.tileRows = bm, R.itemsPad = itemsPad[i];
       R.h = G.h, R.v = G.v;
       blocks += rows + 1;
       HalvesItem &it = batch.item[i];
       HalvesArgs &q = it.q;
-      q.a = R.dst, q.b = I.dst, q.items = R.items, q.rowExp = R.exps, q.imgExp = I.exps, q.marks = I.marks;
-      q.aBytes = (int)splitBytes[i], q.bBytes = (int)(cnt * imgBytes), q.imgBytes = (int)imgBytes, q.planeBytes = (int)(Hp * Wp * 16);
-      q.marksPerImg = groups * chunks, q.nItems = groups * G.h.n * G.v.n, q.itemsPad = itemsPad[i];
+      q.a = R.dst, q.b = I.dst, q.a3 = R.dst3, q.b3 = I.dst3, q.items = R.items, q.items3 = R.items3;
+      q.rowForm = R.forms, q.imgForm = I.forms, q.imgBytes = imgBytes, q.planeBytes = (int)(Hp * Wp * 16);
+      q.nItems = groups * G.h.n * G.v.n, q.itemsPad = itemsPad[i];
       q.w = w, q.x = xg, q.wBytes = (int)(wFloats * 4), q.xBytes = (int)(cnt * xImgBytes);
       q.rs = rs, q.cs = cs, q.kW = kW, q.C = C, q.H = H, q.W = W, q.h = G.h, q.v = G.v;
       q.magicT = dev::magicOf(G.h.n * G.v.n), q.magicV = dev::magicOf(G.v.n);

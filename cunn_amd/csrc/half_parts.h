@@ -1,30 +1,110 @@
 // fp32 products on the fp16 matrix pipe, three instructions per product, for long convolutions (included by convmm.hip).
 //
 // A float x is taken times a power of two 2^e and written as h + l / 2^12 with h = fp16(x 2^e) and l = fp16 of 2^12 times
-// what h leaves. For |x 2^e| from 2^-13 to 2^15 that is x to one unit in its last place (the remainder has up to 12
-// significant bits and a sign, l keeps 11 bits); below, the sum is exact to 2^-37. The product of two floats is
-// h h' + (h l' + l h') / 2^12; what is left out, l l' / 2^24, is 2^-24 of the product at the very most. hh' and the two
-// small products are summed in fp32 accumulators of their own. Either split costs 6e-8 of the result's norm, which a fourth
+// what h leaves (after Ootomo and Yokota, "Recovering single precision accuracy from Tensor Cores while surpassing the FP32
+// theoretical peak performance", IJHPCA 36, 2022). For |x 2^e| from 2^-14 to 2^15 that is x to one unit in its last place: the
+// remainder has up to 12 significant bits and a sign, l keeps 11 bits. The product of two floats is
+// h h' + (h l' + l h') / 2^12; what is left out, l l' / 2^24, is 2^-22 of the product at the very most, so a product is held to
+// 2^-21 of itself at worst. hh' and the two small products are summed in fp32 accumulators of their own. Either split costs 6e-8 of the result's norm, which a fourth
 // product (l l') does not change (8.6e-8 at 48 terms with three and with four), so short sums are left to the six products
 // of bf16 parts (convmm.hip), whose error starts at 4e-8 but grows with the root of the number of terms. The GEMM of
-// conv_halves.h therefore also moves the sum of the large products to a third accumulator every kFoldStages stages, so
+// conv_halves.h therefore also moves the sum of the large products to a third accumulator every kFoldTerms terms, so
 // that a sum of 2304 terms is rounded some 25 times at its full size and not 144 times, and the weight gradient takes
 // shorter partial sums. Error against 64 bits, normally distributed terms, K = 576 / 1152 / 2304 / 8192: 1.2e-7 / 1.3e-7 /
 // 1.4e-7 / 1.8e-7 in conv_halves.h; six bf16 products 1.4e-7 / 2.0e-7 / 2.9e-7 / 5.7e-7; the fp32 instruction three times that.
 //
-// The exponent e comes from the largest finite element of an image, of a weight row, or (weight gradient) of the tensor
-// (absMaxKernel: a pass of its own). Nothing overflows, and elements down to 2^-31 of the largest keep 21 bits or more.
-// What lies below is looked for, and computed again with the fp32 instruction as are sums that are not finite:
-//  * conv_halves.h: an image with such elements in numbers (more than a sixteenth of a channel's non-zero ones among 64
-//    neighbouring positions), or with one whose neighbours in its group of 8 channels are all small as well
-//  * weight gradient: blocks of rows or columns that are small throughout, all of it where a slice of a tensor is
+// The exponent e comes from the largest finite element of what shares one - an image, a weight row, the images of a partial
+// weight gradient - so nothing overflows; and the parts are only used where the smallest non-zero element of it, times 2^e, is
+// 2^-14 or more too (fitsHalves: within 2^28 of the largest). What spans more goes to the six products of bf16 parts, which
+// are exact for elements of every size. Either kernel family looks both numbers up (rangesKernel: a pass of its own over the
+// operands) before it starts. Sums that are not finite are computed again with the fp32 instruction.
 #pragma once
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 
-constexpr int kMaxSlots = 64;          // partial maxima of an image
+constexpr int kMaxSlots = 64;          // slices of an image
 constexpr int kTensorSlots = 1024;     // of a whole tensor
+
+// x: the largest finite |x|, as its bits; y: the smallest non-zero |x|, as its bits less one (all ones: there is none)
+__device__ __forceinline__ uint2 noRange() { return make_uint2(0u, 0xffffffffu); }
+__device__ __forceinline__ uint2 joinRanges(uint2 a, uint2 b) { return make_uint2(max(a.x, b.x), min(a.y, b.y)); }
+__device__ __forceinline__ uint2 addToRange(uint2 r, float x) {
+  const unsigned u = __float_as_uint(x) & 0x7fffffffu;
+  return make_uint2(u < 0x7f800000u ? max(r.x, u) : r.x, min(r.y, u - 1u));
+}
+// of `lanes` neighbouring lanes (a power of two)
+__device__ __forceinline__ uint2 lanesRange(uint2 r, int lanes) {
+  for (int d = lanes >> 1; d > 0; d >>= 1)
+    r = joinRanges(r, make_uint2((unsigned)__shfl_xor((int)r.x, d), (unsigned)__shfl_xor((int)r.y, d)));
+  return r;
+}
+__device__ __forceinline__ uint2 blockRange(uint2 r, uint2 *red) {
+  r = lanesRange(r, dev::kWave);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = r;
+  __syncthreads();
+  return joinRanges(joinRanges(red[0], red[1]), joinRanges(red[2], red[3]));
+}
+// e with 2^14 <= |x| 2^e < 2^15 for the largest |x| (its bits; a subnormal one counts as 2^-127)
+__device__ __forceinline__ int exponentFor(unsigned mostBits) { return mostBits ? 14 + 127 - (int)(mostBits >> 23) : 0; }
+__device__ __forceinline__ bool fitsHalves(uint2 r, int e) {
+  return r.y == 0xffffffffu || __builtin_amdgcn_ldexpf(__uint_as_float(r.y + 1u), e) >= 0x1p-14f;
+}
+
+// rows[row] = range of a weight row (the first workgroups: the longest), slots[image * nSlots + slice] = range of a slice of the
+// image. Bound by memory: the split behind it finds what still fits the Infinity Cache there.
+struct RangeArgs {
+  const float *x;          // images of perImg floats, nSlots slices of perSlice each
+  uint2 *slots;
+  long perImg;
+  int perSlice, nSlots;
+  bool vec;                // perImg % 4 == 0, perSlice % 4 == 0, aligned base
+  const float *w;          // element (row, channel, tap) at row * rs + channel * cs + tap
+  uint2 *rows;
+  int M, rs, cs, C, taps;
+};
+__global__ void __launch_bounds__(dev::kBlock) rangesKernel(RangeArgs a) {
+  __shared__ uint2 red[4];
+  uint2 r = noRange();
+  const int t = threadIdx.x;
+  if ((int)blockIdx.x < a.M) {
+    const float *src = a.w + (long)blockIdx.x * a.rs;
+    const int n = a.C * a.taps;
+    for (int i0 = t; i0 < n; i0 += 8 * dev::kBlock) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {  // (elements past the last repeat it)
+        const int i = min(i0 + u * dev::kBlock, n - 1), c = i / a.taps;
+        v[u] = src[(long)c * a.cs + (i - c * a.taps)];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) r = addToRange(r, v[u]);
+    }
+    r = blockRange(r, red);
+    if (t == 0) a.rows[blockIdx.x] = r;
+    return;
+  }
+  const int slot = blockIdx.x - a.M, img = slot / a.nSlots, slice = slot - img * a.nSlots;
+  const long b = (long)slice * a.perSlice, e = min(a.perImg, b + a.perSlice);
+  const float *src = a.x + img * a.perImg;
+  if (a.vec) {
+    const float4 *s4 = reinterpret_cast<const float4 *>(src);
+    auto add = [&](const float4 &v) { r = addToRange(addToRange(addToRange(addToRange(r, v.x), v.y), v.z), v.w); };
+    long i = (b >> 2) + t;
+    for (; i + 3 * dev::kBlock < e >> 2; i += 4 * dev::kBlock) {
+      float4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = s4[i + u * dev::kBlock];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) add(v[u]);
+    }
+    for (; i < e >> 2; i += dev::kBlock) add(s4[i]);
+  } else {
+    for (long i = b + t; i < e; i += dev::kBlock) r = addToRange(r, src[i]);
+  }
+  r = blockRange(r, red);
+  if (t == 0) a.slots[slot] = r;
+}
 
 // largest finite |x|, as its bits
 __device__ __forceinline__ unsigned finiteMax(unsigned m, float x) {
@@ -38,9 +118,6 @@ __device__ __forceinline__ unsigned blockMax(unsigned m, unsigned *red) {
   __syncthreads();
   return max(max(red[0], red[1]), max(red[2], red[3]));
 }
-// e with 2^14 <= |x| 2^e < 2^15 for the largest |x| (its bits; a subnormal one counts as 2^-127)
-__device__ __forceinline__ int exponentFor(unsigned maxBits) { return maxBits ? 14 + 127 - (int)(maxBits >> 23) : 0; }
-
 // slots[image][slice] = largest finite |x| of a slice of the image (its bits). grid (slices, images). Bound by memory: the
 // split behind it finds what still fits the Infinity Cache there.
 __global__ void __launch_bounds__(dev::kBlock)

@@ -1,7 +1,7 @@
 """Convolution passes on half-precision parts (three fp16 products per fp32 product, half_parts.h) wherever
 they can be forced: tile shapes and their edges, ragged channels, strides (phases), dilation, K split over workgroups, a
 smaller last group of positions; operands of all sizes, infinities and NaNs, images, channels and corners of very
-different size. Bounds: those of test_gpu_conv_split.py (a chain of K fp32 additions); element by element, K fp32
+different size, on fp16 parts, on bf16 parts where those do not hold an image or a weight row, and both in one call. Bounds: those of test_gpu_conv_split.py (a chain of K fp32 additions); element by element, K fp32
 additions of what the terms of the element add up to in magnitude."""
 import numpy as np
 import pytest
@@ -108,6 +108,94 @@ def test_windows_beyond_the_index_arithmetic(Ci, k):
                                                     k, k, 1, 1, 0, 0)
     # at most 96 terms of size 1 that are not zero
     assert np.abs(y.numpy() - ref).max() <= 96 * 2.0 ** -24 * 96
+
+
+def _grad_input(gy, w, dil, stride, H, W):
+    """gradInput of a convolution without padding in 64 bits, and the sum of the magnitudes of its terms"""
+    import torch
+    f = lambda a, b: torch.nn.functional.conv_transpose2d(torch.from_numpy(a).double(), torch.from_numpy(b).double(), stride=stride,
+                                                          dilation=dil).numpy()
+    out = []
+    for a, b in ((gy, w), (np.abs(gy), np.abs(w))):
+        full, padded = f(a, b), np.zeros(gy.shape[:1] + w.shape[1:2] + (H, W))
+        padded[:, :, :full.shape[2], :full.shape[3]] = full
+        out.append(padded)
+    return out
+
+
+def _forward_and_grad_input(x, gy, w, dil, stride):
+    """Both passes without padding against 64 bits, element by element: K fp32 additions of the element's own terms."""
+    CT, y, gx = cunn_amd.CudaTensor, cunn_amd.CudaTensor(), cunn_amd.CudaTensor()
+    Co, Ci, k, _ = w.shape
+    a = (k, k, stride, stride, 0, 0, dil, dil)
+    cunn_amd.THNN.SpatialDilatedConvolution_updateOutput(CT.from_numpy(x), y, CT.from_numpy(w), None, CT(), CT(), *a)
+    ref, terms = _terms(x, w, dil)
+    ref, terms = ref[:, :, ::stride, ::stride], terms[:, :, ::stride, ::stride]
+    worst = np.abs(y.numpy() - ref) / (Ci * k * k * 2.0 ** -24 * terms + 2.0 ** -149)
+    print("forward: worst element at %.3g of its bound" % worst.max(), flush=True)
+    assert worst.max() <= 1
+    cunn_amd.THNN.SpatialDilatedConvolution_updateGradInput(CT.from_numpy(x), CT.from_numpy(gy), gx, CT.from_numpy(w), CT(), *a)
+    ref, terms = _grad_input(gy, w, dil, stride, x.shape[2], x.shape[3])
+    worst = np.abs(gx.numpy() - ref) / (Co * k * k * 2.0 ** -24 * terms + 2.0 ** -149)
+    print("gradInput: worst element at %.3g of its bound" % worst.max(), flush=True)
+    assert worst.max() <= 1
+
+
+# 2^power apart: within reach of two parts, at the edge of it, at half the bits, lost altogether
+POWERS = [20, 27, 28, 29, 40, 44, 48, 52, 60]
+
+
+@pytest.mark.parametrize("dil, stride", [(1, 1), (2, 1), (1, 2)])
+@pytest.mark.parametrize("power", POWERS)
+def test_large_weights_that_meet_zeros(power, dil, stride):
+    """The rest of a weight row decides the output where the plane that its large weights meet is zero."""
+    print("case", power, dil, stride, flush=True)
+    rng = np.random.default_rng(power)
+    N, Ci, Co, H, W, k = 3, 40, 48, 15, 18, 3
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    span = dil * (k - 1) + 1
+    x, w, gy = f(N, Ci, H, W), f(Co, Ci, k, k), f(N, Co, (H - span) // stride + 1, (W - span) // stride + 1)
+    wx = w.copy()
+    x[:, 5] = 0
+    wx[:, 5] *= np.float32(2.0 ** power)
+    gy[:, 7] = 0
+    wx[7] *= np.float32(2.0 ** power)
+    wx[7, 5] = w[7, 5]
+    _forward_and_grad_input(x, gy, wx, dil, stride)
+
+
+@pytest.mark.parametrize("dil, stride", [(1, 1), (2, 1), (1, 2)])
+@pytest.mark.parametrize("power", POWERS)
+def test_small_elements_that_weights_pick_out(power, dil, stride):
+    """Rows of one weight each: an output is one element of the image, also one that is small beside all its neighbours."""
+    print("case", power, dil, stride, flush=True)
+    rng = np.random.default_rng(power)
+    N, Ci, Co, H, W, k = 3, 40, 40, 15, 18, 3
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    span = dil * (k - 1) + 1
+    x, gy = f(N, Ci, H, W), f(N, Co, (H - span) // stride + 1, (W - span) // stride + 1)
+    for t in (x, gy):
+        few = rng.random(t.shape) < 0.02
+        few[1] = False                              # an image that is ordinary throughout
+        t[few] *= np.float32(2.0 ** -power)
+    w = np.zeros((Co, Ci, k, k), np.float32)
+    for o in range(Co):
+        w[o, o, o % 3, o // 3 % 3] = rng.standard_normal()
+    _forward_and_grad_input(x, gy, w, dil, stride)
+
+
+@pytest.mark.parametrize("case", [(40, 24, 40, 3, 3, 3), (9, 24, 136, 5, 4, 3), (300, 20, 30, 1, 2, 1), (2, 16, 70, 40, 39, 2)])
+def test_images_of_both_kinds_in_a_tile(case):
+    """Every third image holds elements far below its largest: tiles of many images, tiles inside one, 1x1 planes."""
+    print("case", case, flush=True)
+    N, Ci, Co, H, W, k = case
+    rng = np.random.default_rng(N)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    x, w, gy = f(N, Ci, H, W), f(Co, Ci, k, k) * np.float32(0.1), f(N, Co, H - k + 1, W - k + 1) if k <= min(H, W) else None
+    for t in (x, gy):
+        t[::3, ::5] *= np.float32(2.0 ** -50)
+    w[:3] *= (rng.random((3, Ci, k, k)) < 0.1).astype(np.float32)
+    _forward_and_grad_input(x, gy, w, 1, 1)
 
 
 @pytest.mark.parametrize("relu", [False, True])
