@@ -1555,8 +1555,8 @@ struct GradWeightArgs {
   unsigned magicOW;
   unsigned magicKK, magicKW;  // reciprocals of kH * kW and kW (dev::magicOf)
   int Lvalid;               // positions of an image (g.L may count the padding of the gradOutput rows)
-  const unsigned *gySlots, *xSlots;  // HALVES: `slots` partial maxima of either tensor (absMaxKernel)
-  int slots;
+  const uint2 *gySlots, *xSlots;  // HALVES: ranges of gyNSlots / xNSlots slices of every image (rangesKernel)
+  int gyNSlots, xNSlots;
 };
 
 // Small gradWeights (first layers, narrow 1x1 convolutions), where the large tiles would spend most of their
@@ -1757,35 +1757,34 @@ convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
 //    16 consecutive positions, 64-byte runs); the 4 lanes of a quad then transpose their 4 x 4 elements through DPP
 // WM = 2: 128 x 128 tiles of gradWeight (Cout x K), WM = 1: 64 x 256 tiles; a wave multiplies 64 x 64 either way.
 // A block whose sums are not all finite is computed again with the fp32 instruction, straight from memory.
-// HALVES: the operands as two fp16 parts and three products (half_parts.h), scaled by the largest element of either tensor,
-// for long reductions; twice as many splits keep the sums as exact as the six products do. 256 x 2304 over 64 x 28 x 28
-// positions 333 -> 219 us (and 20 us for the largest elements, 5 for the longer fold), 192 x 720 over 32 x 71 x 71 396 -> 288.
+// HALVES: for long reductions. A split whose images are held by two fp16 parts (half_parts.h), scaled by the largest element
+// of either operand among them, takes these and three products, any other split the three bf16 parts; twice as many splits
+// keep the sums as exact as six products do. Whole pass, ranges (20 / 38 us) and a longer fold (5) included, us: 256 x 2304 over
+// 64 x 28 x 28 positions 339 -> 250 (374 where no split can), 192 x 720 over 32 x 71 x 71 372 -> 320 (419; 382 before).
 // What bounds it: as the forward kernel, two workgroups per CU and a clock that power pulls down. Against the fp32
 // instruction: 256 x 2304 over 64 x 28 x 28 positions (59.2 GFLOP) 519 -> 334 us; 192 x 720 over 32 x 71 x 71 (64 x 256
 // tiles, gathers transposed) 462 -> 342 us; 256 x 2048, stride 2, over 64 x 14 x 14 142 -> 99 us.
-template <bool L16, int WM, bool B4, bool HALVES>
-__global__ void __launch_bounds__(dev::kBlock, 2)
-convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
+// NP: parts; split: of the reduction; sc: scale of the fp16 parts (NP = 2).
+template <int WM, int NP>
+struct GradWeightLds {
+  static constexpr int AP = 64 * WM + 8, BP = 256 / WM + 8;  // 16-byte groups (8 positions of one part) per position-group row
+  u32x4 a[2][NP][2][AP];                        // [buffer][part][group of 8 positions][row]
+  u32x4 b[2][NP][2][BP];
+};
+template <bool L16, int WM, bool B4, int NP>
+__device__ __forceinline__ void gradWeightSplitBody(const GradWeightArgs &p, const ConvGeom &g, int split, int tileIdx,
+                                                    GradWeightLds<WM, NP> &lds, const HalvesScale &sc) {
   constexpr int TBM = 64 * WM, TBN = 256 / WM;
-  constexpr int AP = TBM + 8, BP = TBN + 8;     // 16-byte groups (8 positions of one part) per position-group row
+  constexpr int AP = GradWeightLds<WM, NP>::AP, BP = GradWeightLds<WM, NP>::BP;
   constexpr int NQ = TBN / 64;                  // groups of 4 positions a lane parks per k-tile
   constexpr int NT = B4 ? NQ : 4 * NQ;          // columns a lane fetches
-  constexpr int NP = HALVES ? 2 : 3;            // parts
-  __shared__ u32x4 As[2][NP][2][AP];            // [buffer][part][group of 8 positions][row]
-  __shared__ u32x4 Bs[2][NP][2][BP];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = WM == 2 ? wave >> 1 : 0, wn = WM == 2 ? wave & 1 : wave;
-  // workgroups that reduce the same positions (one split) are neighbours in the remapped order: same XCD, same L2
-  const int tilesPerSplit = p.mTiles * p.nTiles;
-  const int bid = dev::xcdRemap(blockIdx.x, gridDim.x);
-  const int split = bid / tilesPerSplit, tileIdx = bid - split * tilesPerSplit;
   const int mTile = tileIdx % p.mTiles, nTile = tileIdx / p.mTiles;
   const int m0 = mTile * TBM, j0 = nTile * TBN;
   const int ktBegin = split * p.ktPerSplit;
   const int ktEnd = min(p.totalKt, ktBegin + p.ktPerSplit);
   const int kOob = 0x7fffffff;
-  HalvesScale sc{};
-  if constexpr (HALVES) sc = halvesScale(p.gySlots, p.xSlots, p.slots);
 
   // ---- gradOutput. WM = 2: row t >> 1, positions 8 * (t & 1) .. + 7 of the k-tile; WM = 1: row t >> 2, positions
   //      4 * (t & 3) .. + 3
@@ -1862,24 +1861,20 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
   };
   constexpr int PA = 2 * AP, PB = 2 * BP;      // 16-byte groups of one part in one buffer
   constexpr int BUFA = NP * PA, BUFB = NP * PB;  // of one buffer
-  u32x4 *aDst = &As[0][0][pgA >> 1][rowA];
+  u32x4 *aDst = &lds.a[0][0][pgA >> 1][rowA];
   const int pgB = B4 ? t & 3 : (t & 15) >> 2, colB = B4 ? t >> 2 : (t >> 4) * 4 + (t & 3);
-  u32x2 *bDst = reinterpret_cast<u32x2 *>(&Bs[0][0][pgB >> 1][colB]) + (pgB & 1);
+  u32x2 *bDst = reinterpret_cast<u32x2 *>(&lds.b[0][0][pgB >> 1][colB]) + (pgB & 1);
   // The workgroups of the first column tile also sum the gradOutput elements they pass on (each element of a
   // row is loaded by exactly one lane of exactly one of them): the bias gradient without a second pass over gy.
   const bool rowSums = nTile == 0 && p.biasPartial != nullptr;
   float rowSum = 0.f;
-  float mostA = 0.f, mostB[NQ] = {};            // HALVES: largest element of the lane's row and columns
-  // scale, most: HALVES
-  auto split4 = [](const u32x4 &v, u32x2 (&part)[NP], float scale, float &most) {
+  auto split4 = [](const u32x4 &v, u32x2 (&part)[NP], float scale) {  // scale: of fp16 parts
     unsigned h[2], m[2], l[2];
-    if constexpr (HALVES) {
+    if constexpr (NP == 2) {
       const unsigned ux = v.x, uy = v.y, uz = v.z, uw = v.w;
       const float x = __uint_as_float(ux), y = __uint_as_float(uy), z = __uint_as_float(uz), w = __uint_as_float(uw);
       splitHalves(x * scale, y * scale, h[0], m[0]);
       splitHalves(z * scale, w * scale, h[1], m[1]);
-      most = fmaxf(fmaxf(most, __builtin_fabsf(x)), __builtin_fabsf(y));
-      most = fmaxf(fmaxf(most, __builtin_fabsf(z)), __builtin_fabsf(w));
       part[0] = u32x2{h[0], h[1]}, part[1] = u32x2{m[0], m[1]};
     } else {
       splitPair(v.x, v.y, h[0], m[0], l[0]);
@@ -1891,7 +1886,7 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     constexpr int buf = decltype(bufc)::value;
     u32x2 pa[WM][NP];
 #pragma unroll
-    for (int i = 0; i < WM; ++i) split4(ra[i], pa[i], sc.gy, mostA);
+    for (int i = 0; i < WM; ++i) split4(ra[i], pa[i], sc.gy);
 #pragma unroll
     for (int s = 0; s < NP; ++s) {
       if constexpr (WM == 2)
@@ -1911,14 +1906,14 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     for (int i = 0; i < NQ; ++i) {
       if constexpr (!B4) rb[i] = dev::quadTranspose(re[4 * i], re[4 * i + 1], re[4 * i + 2], re[4 * i + 3]);
       u32x2 pb[NP];
-      split4(rb[i], pb, sc.x, mostB[i]);
+      split4(rb[i], pb, sc.x);
 #pragma unroll
       for (int s = 0; s < NP; ++s) bDst[2 * (buf * BUFB + s * PB + 64 * i)] = pb[s];
     }
   };
   const int grp = lane >> 5, idx = lane & 31;
-  const u32x4 *aSrc = &As[0][0][grp][wm * 64 + idx];
-  const u32x4 *bSrc = &Bs[0][0][grp][wn * 64 + idx];
+  const u32x4 *aSrc = &lds.a[0][0][grp][wm * 64 + idx];
+  const u32x4 *bSrc = &lds.b[0][0][grp][wn * 64 + idx];
   using Buf0 = std::integral_constant<int, 0>;
   using Buf1 = std::integral_constant<int, 1>;
 
@@ -1943,7 +1938,7 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     }
     if (store) storeTiles(nxt);
     if (load) loadTiles();
-    if constexpr (HALVES)
+    if constexpr (NP == 2)
       mfmaHalves(a, b, acc, lo);
     else
       mfmaSplit(a, b, acc, lo);
@@ -1965,29 +1960,12 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     if (kt + 2 < ktEnd) step(Buf0{}, Buf1{}, false, false);
   }
 
-  // HALVES: rows and columns whose elements are all small beside the tensor's largest are not held exactly enough
-  float *rowMost = reinterpret_cast<float *>(&As[0][0][0][0]), *colMost = reinterpret_cast<float *>(&Bs[0][0][0][0]);
-  if constexpr (HALVES) {
-    mostA = fmaxf(mostA, __shfl_xor(mostA, 1));      // the 2 or 4 lanes of a row
-    if (WM == 1) mostA = fmaxf(mostA, __shfl_xor(mostA, 2));
-    rowMost[rowA] = mostA;
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      float m = mostB[i];                            // the 4 lanes of a column: neighbours (B4), or the quads of 16
-      m = fmaxf(m, __shfl_xor(m, B4 ? 1 : 4));
-      m = fmaxf(m, __shfl_xor(m, B4 ? 2 : 8));
-      colMost[colB + 64 * i] = m;
-    }
-    __syncthreads();
-  }
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      if constexpr (HALVES) {
-        const float r = rowMost[wm * 64 + i * 32 + idx] * sc.gy, c = colMost[wn * 64 + j * 32 + idx] * sc.x;
-        const bool coarse = sc.wide || (r > 0.f && r < 0x1p-10f) || (c > 0.f && c < 0x1p-10f);
-        if (!finishHalves(acc[i][j], lo[i][j], -(sc.gyExp + sc.xExp)) && !__any(coarse)) continue;
+      if constexpr (NP == 2) {
+        if (!finishHalves(acc[i][j], lo[i][j], -(sc.gyExp + sc.xExp))) continue;
       } else {
         if (!finishSums(acc[i][j], lo[i][j])) continue;
       }
@@ -2027,6 +2005,31 @@ convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
     rowSum = dev::dppAdd<0xB1>(rowSum);
     if (WM == 1) rowSum = dev::dppAdd<0x4E>(rowSum);
     if ((t & (WM == 2 ? 1 : 3)) == 0 && m0 + rowA < p.M) p.biasPartial[(long)split * p.M + m0 + rowA] = rowSum;
+  }
+}
+
+template <bool L16, int WM, bool B4, bool HALVES>
+__global__ void __launch_bounds__(dev::kBlock, 2)
+convGradWeightSplitKernel(GradWeightArgs p, ConvGeom g) {
+  // workgroups that reduce the same positions (one split) are neighbours in the remapped order: same XCD, same L2
+  const int tilesPerSplit = p.mTiles * p.nTiles;
+  const int bid = dev::xcdRemap(blockIdx.x, gridDim.x);
+  const int split = bid / tilesPerSplit, tileIdx = bid - split * tilesPerSplit;
+  if constexpr (HALVES) {
+    __shared__ union {
+      GradWeightLds<WM, 2> two;
+      GradWeightLds<WM, 3> three;
+    } lds;
+    const long r0 = (long)split * p.ktPerSplit * BK, r1 = min((long)p.totalKt, (long)(split + 1) * p.ktPerSplit) * BK;
+    const int n0 = (int)(r0 / g.L), n1 = min(g.N, (int)((r1 - 1) / g.L) + 1);
+    const HalvesScale sc = halvesScale(p.gySlots, p.gyNSlots, p.xSlots, p.xNSlots, n0, n1);
+    if (sc.fits)
+      gradWeightSplitBody<L16, WM, B4, 2>(p, g, split, tileIdx, lds.two, sc);
+    else
+      gradWeightSplitBody<L16, WM, B4, 3>(p, g, split, tileIdx, lds.three, sc);
+  } else {
+    __shared__ GradWeightLds<WM, 3> lds;
+    gradWeightSplitBody<L16, WM, B4, 3>(p, g, split, tileIdx, lds, HalvesScale{});
   }
 }
 
@@ -3637,13 +3640,17 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   };
   while (perCu > 1 && totalKt / splitsAt(perCu) < 20 * BK / ktPositions) --perCu;
   int splits = splitsAt(perCu);
+  // slices of an image that rangesKernel reads: about 1024 workgroups, at least 4096 floats each
+  auto slices = [&](long perImg) { return (int)std::max<long>(1, std::min<long>(perImg / 4096, launch::ceilDiv(1024, g.N))); };
+  const int gySlots = slices((long)g.Cout * g.L), xSlots = slices((long)g.Cin * g.H * g.W);
+  const long rangeFloats = 2L * g.N * (gySlots + xSlots);
   // Long reductions on half-precision parts, with twice the splits: their sums are then as exact as those of the six products
   // (3.6e-7 of the norm at 3584 positions a split; on three products 2.9e-7 at 1792) from about 1100 positions a split on.
   const int perSplitSix = launch::ceilDiv(totalKt, splits) * BK;
   // (They need more scratch: not with a buffer that cannot grow.)
   if (fast && !tiny && g_switches.convHalves != 0 && (perSplitSix >= 1100 || g_switches.convHalves == 1) &&
       (!scratchBuf || (growable(scratchBuf) && roomFor(state, scratchBuf, 2 * splits * ((long)g.Cout * g.K + g.Cout) + xpFloats + gypFloats +
-                                                                          2 * kTensorSlots + 16)))) {
+                                                                          rangeFloats + 16)))) {
     halves = true;
     gw = pick();
     kern = gw.fn;
@@ -3660,7 +3667,7 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   const long biasFloats = fusedBias ? ((long)splits * g.Cout + 3) / 4 * 4 : 0;
   Temp tmp;
   const long xpScratch = fast && bordered ? (xpFloats + 3) / 4 * 4 : 0;
-  const long slotFloats = halves ? 2 * kTensorSlots : 0;
+  const long slotFloats = halves ? rangeFloats : 0;
   float *partial = scratchFloats(state, scratchBuf, partialFloats + biasFloats + xpScratch + (fast ? (gypFloats + 3) / 4 * 4 : 0) + slotFloats, tmp,
                                  "columns");
   float *biasPartial = fusedBias ? partial + partialFloats : nullptr;
@@ -3696,15 +3703,17 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
     q.magicKK = dev::magicOf(g.kH * g.kW), q.magicKW = dev::magicOf(g.kW);
     q.Lvalid = g.L;
     if (halves) {
-      unsigned *slots = reinterpret_cast<unsigned *>(partial + partialFloats + biasFloats + xpScratch + (gypFloats + 3) / 4 * 4);
-      auto largest = [&](const float *t, long count, unsigned *dst) {
-        const long per = ((count + kTensorSlots - 1) / kTensorSlots + 3) / 4 * 4;
-        absMaxKernel<<<dim3(kTensorSlots, 1), dev::kBlock, 0, s>>>(t, dst, count, (int)per, count % 4 == 0 && launch::aligned16(t));
+      uint2 *slots = reinterpret_cast<uint2 *>(partial + partialFloats + biasFloats + xpScratch + (gypFloats + 3) / 4 * 4);
+      auto ranges = [&](const float *t, long perImg, int nSlots, uint2 *dst) {
+        RangeArgs ra{};
+        ra.x = t, ra.slots = dst, ra.perImg = perImg, ra.perSlice = (int)((perImg + nSlots - 1) / nSlots + 3) / 4 * 4, ra.nSlots = nSlots;
+        ra.vec = perImg % 4 == 0 && launch::aligned16(t);
+        rangesKernel<<<(unsigned)(g.N * nSlots), dev::kBlock, 0, s>>>(ra);
         THC_HIP_CHECK(hipGetLastError());
+        return dst;
       };
-      largest(gy, (long)g.N * g.Cout * g.L, slots);
-      largest(x, (long)g.N * g.Cin * g.H * g.W, slots + kTensorSlots);
-      q.gySlots = slots, q.xSlots = slots + kTensorSlots, q.slots = kTensorSlots;
+      q.gyNSlots = gySlots, q.gySlots = ranges(gy, (long)g.Cout * g.L, gySlots, slots);
+      q.xNSlots = xSlots, q.xSlots = ranges(x, (long)g.Cin * g.H * g.W, xSlots, slots + (long)g.N * gySlots);
     }
     gw.launch(dim3(mT * nT * splits), s, q, gk);
   } else {

@@ -24,7 +24,6 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 
 constexpr int kMaxSlots = 64;          // slices of an image
-constexpr int kTensorSlots = 1024;     // of a whole tensor
 
 // x: the largest finite |x|, as its bits; y: the smallest non-zero |x|, as its bits less one (all ones: there is none)
 __device__ __forceinline__ uint2 noRange() { return make_uint2(0u, 0xffffffffu); }
@@ -106,47 +105,6 @@ __global__ void __launch_bounds__(dev::kBlock) rangesKernel(RangeArgs a) {
   if (t == 0) a.slots[slot] = r;
 }
 
-// largest finite |x|, as its bits
-__device__ __forceinline__ unsigned finiteMax(unsigned m, float x) {
-  const unsigned u = __float_as_uint(x) & 0x7fffffffu;
-  return u < 0x7f800000u && u > m ? u : m;
-}
-__device__ __forceinline__ unsigned blockMax(unsigned m, unsigned *red) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, d));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  return max(max(red[0], red[1]), max(red[2], red[3]));
-}
-// slots[image][slice] = largest finite |x| of a slice of the image (its bits). grid (slices, images). Bound by memory: the
-// split behind it finds what still fits the Infinity Cache there.
-__global__ void __launch_bounds__(dev::kBlock)
-absMaxKernel(const float *__restrict__ x, unsigned *__restrict__ slots, long perImg, int perSlice, bool vec) {
-  __shared__ unsigned red[4];
-  const long b = (long)blockIdx.x * perSlice, e = min(perImg, b + perSlice);
-  const float *src = x + blockIdx.y * perImg;
-  unsigned m = 0;
-  if (vec) {  // perImg % 4 == 0, perSlice % 4 == 0, aligned base
-    const float4 *s4 = reinterpret_cast<const float4 *>(src);
-    long i = (b >> 2) + threadIdx.x;
-    for (; i + 3 * dev::kBlock < e >> 2; i += 4 * dev::kBlock) {
-      float4 v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = s4[i + u * dev::kBlock];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) m = finiteMax(finiteMax(finiteMax(finiteMax(m, v[u].x), v[u].y), v[u].z), v[u].w);
-    }
-    for (; i < e >> 2; i += dev::kBlock) {
-      const float4 v = s4[i];
-      m = finiteMax(finiteMax(finiteMax(finiteMax(m, v.x), v.y), v.z), v.w);
-    }
-  } else {
-    for (long i = b + threadIdx.x; i < e; i += dev::kBlock) m = finiteMax(m, src[i]);
-  }
-  m = blockMax(m, red);
-  if (threadIdx.x == 0) slots[blockIdx.y * gridDim.x + blockIdx.x] = m;
-}
-
 // y0, y1: already scaled
 __device__ __forceinline__ void splitHalves(float y0, float y1, unsigned &h, unsigned &l) {
   const f32x2 r = {y0, y1};
@@ -185,34 +143,25 @@ __device__ __forceinline__ bool finishHalves(float16v &acc, const float16v &lo, 
   return __any(bad != bad);
 }
 
-// Scales of the two operands of a weight gradient, from partial maxima of slices of the whole tensors. wide: a slice lies so
-// far below the largest element (2^-25) that its elements may not be held exactly enough.
+// Scales of the two operands of a split of a weight gradient over images [n0, n1), from the ranges of gyN and xN slices of
+// every image. fits: the fp16 parts hold all of their elements.
 struct HalvesScale {
   float gy, x;
   int gyExp, xExp;
-  bool wide;
+  bool fits;
 };
-__device__ __forceinline__ HalvesScale halvesScale(const unsigned *gySlots, const unsigned *xSlots, int slots) {
-  __shared__ unsigned red[4][4];
-  unsigned m[2] = {0, 0}, least[2] = {0, 0};     // least: of the slices that are not all zero, as its complement
-  for (int i = threadIdx.x; i < slots; i += dev::kBlock) {
-    const unsigned v[2] = {gySlots[i], xSlots[i]};
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      m[q] = max(m[q], v[q]);
-      if (v[q]) least[q] = max(least[q], ~v[q]);
-    }
-  }
+__device__ __forceinline__ HalvesScale halvesScale(const uint2 *gySlots, int gyN, const uint2 *xSlots, int xN, int n0, int n1) {
+  __shared__ uint2 red[2][4];
+  auto range = [&](const uint2 *slots, int n, uint2 *r4) {
+    uint2 r = noRange();
+    for (long i = (long)n0 * n + threadIdx.x; i < (long)n1 * n; i += dev::kBlock) r = joinRanges(r, slots[i]);
+    r = blockRange(r, r4);
+    return make_uint2(__builtin_amdgcn_readfirstlane(r.x), __builtin_amdgcn_readfirstlane(r.y));
+  };
+  const uint2 a = range(gySlots, gyN, red[0]), b = range(xSlots, xN, red[1]);
   HalvesScale s{};
-  int e[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const unsigned most = __builtin_amdgcn_readfirstlane(blockMax(m[q], red[q]));
-    const unsigned low = ~__builtin_amdgcn_readfirstlane(blockMax(least[q], red[2 + q]));
-    e[q] = min(exponentFor(most), 127);
-    s.wide |= most && (low >> 23) + 25 < most >> 23;
-  }
-  s.gyExp = e[0], s.xExp = e[1];
-  s.gy = __uint_as_float((unsigned)(e[0] + 127) << 23), s.x = __uint_as_float((unsigned)(e[1] + 127) << 23);  // (-113 <= e <= 127)
+  s.gyExp = min(exponentFor(a.x), 127), s.xExp = min(exponentFor(b.x), 127);
+  s.gy = __uint_as_float((unsigned)(s.gyExp + 127) << 23), s.x = __uint_as_float((unsigned)(s.xExp + 127) << 23);  // (-113 <= e <= 127)
+  s.fits = fitsHalves(a, s.gyExp) && fitsHalves(b, s.xExp);
   return s;
 }

@@ -22,7 +22,7 @@ CASES = [
     (9, 256, 96, 13, 15, 3, 1, 1),    # K split over workgroups
     (2, 40, 64, 9, 10, 2, 2, 0),
     (1, 16, 33, 5, 4, 4, 1, 2),       # fewer positions than a tile
-    # the weight gradient's large tiles: 128 x 128 and 64 x 256, k-tiles inside an image or not, 16-byte or transposed gathers
+    # 16-byte and transposed gathers, k-tiles inside an image or not (the weight gradient's large tiles: LARGE)
     (2, 64, 120, 16, 16, 3, 2, 1),
     (3, 64, 120, 9, 12, 3, 1, 1),
     (2, 64, 128, 25, 25, 3, 2, 1),
@@ -260,6 +260,87 @@ def test_weight_gradient_of_very_different_sizes(case, which):
                                                  stride=st, padding=pad).numpy().reshape(Co, -1)
     terms = f(np.abs(x), np.abs(gy))
     assert (np.abs(gw.numpy() - f(x, gy)) <= N * H * W * 2.0 ** -24 * terms + 2.0 ** -149).all()
+
+
+# Layers whose weight gradient runs on large tiles (the short reductions above take small ones): every instance of the kernel - 128 x 128
+# and 64 x 256 tiles, k-tiles inside an image or not, 16-byte or transposed gathers.
+LARGE = [
+    (16, 64, 128, 24, 24, 3, 1, 1),
+    (18, 64, 128, 48, 48, 3, 2, 1),
+    (20, 64, 128, 23, 24, 3, 1, 1),
+    (20, 64, 128, 23, 23, 3, 1, 1),
+    (32, 28, 60, 24, 24, 3, 1, 1),
+    (36, 28, 60, 47, 47, 3, 2, 1),
+    (33, 28, 60, 23, 24, 3, 1, 1),
+    (36, 28, 60, 23, 23, 3, 1, 1),
+]
+
+
+def _weight_gradient(x, gy, k, st, pad):
+    THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
+    gw = CT.from_numpy(np.zeros((gy.shape[1], x.shape[1] * k * k), np.float32))
+    THNN.SpatialConvolutionMM_accGradParameters(CT.from_numpy(x), CT.from_numpy(gy), gw, None, CT(), CT(), k, k, st, st, pad, pad, 1.0)
+    return gw.numpy()
+
+
+def _weight_gradient_exact(x, gy, k, st, pad):
+    """in 64 bits; and the sum of the magnitudes of the terms"""
+    import torch
+    out = []
+    for a, b in ((x, gy), (np.abs(x), np.abs(gy))):
+        col = torch.nn.functional.unfold(torch.from_numpy(a).cuda().double(), k, padding=pad, stride=st)   # N, K, L
+        rows = torch.from_numpy(b).cuda().double().flatten(2).transpose(0, 1).flatten(1)                   # Co, N * L
+        out.append((rows @ col.transpose(1, 2).flatten(0, 1)).cpu().numpy())
+    return out
+
+
+@pytest.mark.parametrize("case", LARGE)
+def test_weight_gradient_on_large_tiles(case):
+    """Within the bound of sums of the positions of a split, and not what the other kernels give: these ran."""
+    print("case", case, flush=True)
+    N, Ci, Co, H, W, k, st, pad = case
+    oH, oW = (H + 2 * pad - k) // st + 1, (W + 2 * pad - k) // st + 1
+    rng = np.random.default_rng(8)
+    x, gy = rng.standard_normal((N, Ci, H, W)).astype(np.float32), rng.standard_normal((N, Co, oH, oW)).astype(np.float32)
+    got = _weight_gradient(x, gy, k, st, pad)
+    ref, _ = _weight_gradient_exact(x, gy, k, st, pad)
+    cunn_amd.set_switch("THCUNN_CONV_HALVES", "0")
+    other = _weight_gradient(x, gy, k, st, pad)
+    assert not np.array_equal(got, other)
+    error, before = (np.linalg.norm(v - ref) / np.linalg.norm(ref) for v in (got, other))
+    print("error %.3g, six products %.3g" % (error, before), flush=True)
+    assert error <= 2.0 ** -25 * np.sqrt(N * oH * oW) + 2.0 ** -24
+
+
+@pytest.mark.parametrize("which", ["row", "column", "images", "few"])
+@pytest.mark.parametrize("power", [27, 40, 60])
+@pytest.mark.parametrize("case", LARGE)
+def test_weight_gradient_of_mixed_rows(case, power, which):
+    """Rows and columns that hold both sizes, the large elements against zeros: the small ones are the whole sum."""
+    print("case", case, power, which, flush=True)
+    N, Ci, Co, H, W, k, st, pad = case
+    rng = np.random.default_rng(power)
+    oH, oW = (H + 2 * pad - k) // st + 1, (W + 2 * pad - k) // st + 1
+    x, gy = rng.standard_normal((N, Ci, H, W)), rng.standard_normal((N, Co, oH, oW))
+    big = 2.0 ** power
+    if which == "row":                    # half of every gradOutput plane is large, no image under its windows
+        gy[..., oW // 2:] *= big
+        x[..., oW // 2 * st - pad:] = 0
+    elif which == "column":               # half of every image plane is large, no gradOutput where windows touch it
+        x[..., W // 2:] *= big
+        gy[..., max(0, (W // 2 + pad - k) // st + 1):] = 0
+    elif which == "images":               # images that only the other operand's zeros keep apart
+        x[0], gy[0] = 0, gy[0] * big
+        x[3], gy[3] = x[3] * big, 0
+    else:                                 # small elements everywhere, and rows of nothing else
+        gy[rng.random(gy.shape) < 0.02] /= big
+        x[rng.random(x.shape) < 0.02] /= big
+        gy[:, :3] /= big
+    x, gy = x.astype(np.float32), gy.astype(np.float32)
+    ref, terms = _weight_gradient_exact(x, gy, k, st, pad)
+    worst = np.abs(_weight_gradient(x, gy, k, st, pad) - ref) / (N * oH * oW * 2.0 ** -24 * terms + 2.0 ** -149)
+    print("worst element at %.3g of its bound" % worst.max(), flush=True)
+    assert worst.max() <= 1
 
 
 def test_captured_calls_do_not_allocate():
