@@ -876,9 +876,10 @@ inline bool overlap(const float *a, const float *b, long n) { return a < b + n &
 
 // How a team of workgroups takes a channel's backward pass (bn_teams.h).
 // us, chunked two-pass kernels / teams: 32 x 64 x 112 x 112 85.2 / 63.1; 64 x 96 x 56 x 56 69.5 / 48.8; 64 x 128 x 27 x 27
-// 29.7 / 17.9; 8 x 32 x 28 x 28 8.0 / 6.7; and for large channels that would leave a quarter of the compute units without one,
-// 64 x 128 x 28 x 28 18.4 / 16.2 (small ones not, 64 x 150 x 14 x 14: 9.4 / 11.0). Large planes off the 16-byte boundaries stay
-// with the chunked kernels, which load 16 bytes there all the same: 32 x 64 x 111 x 111 89.3 / 78.7, 128 x 16 x 149 x 149 160 / 165.
+// 29.7 / 17.9; 8 x 32 x 28 x 28 8.0 / 6.7. Large planes off the 16-byte boundaries stay with the chunked kernels, which load 16
+// bytes there all the same: 32 x 64 x 111 x 111 89.3 / 78.7, 128 x 16 x 149 x 149 160 / 165. Channels that a kernel without
+// scratch holds stay with that one, also where a team is faster (64 x 128 x 28 x 28 18.4 / 16.2): a captured call must not share
+// scratch with others where it never did, and gives the bits of an eager one.
 // V: floats of a unit, R: units per lane, as many as still make two workgroups per compute unit; R == 0: not a shape for teams.
 struct TeamPlan {
   int V, R, pieces, units;
@@ -888,12 +889,7 @@ TeamPlan teamsBackward(const BnView &v) {
   if (g_switches.bnTeams == 0 || g_switches.bnChunked == 1 || g.C > kTeamChannels || (long)g.N * g.C * g.L * 4 >= 0x7fffffffL - 65536)
     return TeamPlan{};
   if (g_switches.bnTeams < 0) {
-    const int R = residentR(v, 13);
-    if (R || smallR(v).rs) {
-      if (R <= 8 || g.C > 192) return TeamPlan{};
-    } else if (!v.vec && g.L >= 16384) {
-      return TeamPlan{};
-    }
+    if (residentR(v, 13) || smallR(v).rs || (!v.vec && g.L >= 16384)) return TeamPlan{};
   }
   TeamPlan p{};
   p.V = v.vec ? 4 : 1;
@@ -1027,14 +1023,10 @@ void bnBackward(THCState *state, THCudaTensor *input_, THCudaTensor *gradOutput_
   const bool needSums = (train && gradInput_) || gradWeight_ || gradBias_;
   const long elems = (long)g.N * g.C * g.L;
   const bool over = gradInput_ && (overlap(in.ptr(), data(gradInput_), elems) || overlap(go.ptr(), data(gradInput_), elems));
-  // Under capture a call that has a kernel without scratch takes that one: its graph may be replayed on any stream, next to
-  // others that were captured on this one.
   const TeamPlan t = train && needSums && !over ? teamsBackward(v) : TeamPlan{};
-  void *teamBlock = nullptr;
-  if (t.R && !((residentR(v, 13) || smallR(v).rs) && capturing(state))) teamBlock = keptScratch(state, teamBytes(kTeamChannels));
-  if (teamBlock) {
-    TeamArgs ta{};
-    ta.block = (char *)teamBlock;
+  TeamArgs ta{};
+  if (t.pieces > 1) ta.block = (char *)taggedScratch(state, g.C * teamStride(t.pieces), &ta.tag);
+  if (t.pieces == 1 || ta.block) {
     ta.pieces = t.pieces, ta.units = t.units, ta.spin = g_switches.bnTeams == 2 ? 0 : 1 << 15;
     ta.N = g.N, ta.C = g.C, ta.L = g.L;
 #define BN_BWD_TEAM(VV, RR)                                                                                           \

@@ -1,17 +1,14 @@
 // Backward pass of BatchNormalization in training with a team of workgroups per channel (included by batchnorm.hip).
 //
-// A channel that does not fit the registers of one compute unit used to be read twice (sums, then gradInput), and one
-// that does leaves half the chip idle when there are only a hundred channels. Here
-// the channel is cut into pieces, one workgroup each: it loads its piece once into registers, publishes the piece's two
-// sums, waits for those of the others, merges all of them in the same order and writes its results. Every byte
-// crosses HBM once. Bound by memory; 64 x 112 x 112, N = 32 (with ReLU): 85.2 -> 63.1 us (53 at the rate of a large copy).
+// A channel that does not fit the registers of one compute unit used to be read twice (sums, then gradInput). Here the channel
+// is cut into pieces, one workgroup each: it loads its piece once into registers, publishes the piece's two sums, waits for
+// those of the others, merges all of them in the same order and writes its results. Every byte crosses HBM once. Bound by memory; 64 x 112 x 112, N = 32 (with ReLU): 85.2 -> 63.1 us (53 at the rate of a large copy).
 // Two workgroups of 121 registers share a compute unit, so that one loads while the other waits or stores.
 // (The forward pass stays with the kernels it had: the sign of a normalised element within rounding of zero decides a fused
 // ReLU's gradient, so its statistics keep their order of summation.)
 //
-// The sums travel as 64-bit values (number, tag of the launch), so that a slot proves itself and no fence is
-// needed. The tag is one more than the number of launches that have ended on this scratch block; the last
-// workgroup of a launch to pass its wait moves it on, so replays of a captured graph need no clearing between them.
+// The sums travel as 64-bit values (number, tag of the launch), so that a slot proves itself and no fence is needed. The tag is
+// the host's (taggedScratch): no slot of the scratch holds it when the launch begins.
 //
 // The wait is bounded: pieces start in the order of their numbers and a team is far smaller than what the chip holds, so the
 // others are running or done; should one not answer in time (another program's kernels hold the compute units), the
@@ -23,21 +20,13 @@ constexpr int kTeamLanes = 512;
 constexpr int kTeamWaves = kTeamLanes / dev::kWave;
 constexpr int kTeamMax = 256;            // pieces of a channel
 constexpr int kTeamChannels = 2048;      // a call has at most
-constexpr int kTeamLine = 128;           // bytes between counters: a cache line each
 
-// The scratch block: launches that have ended on it, finished teams of the present one, and per channel the finished
-// workgroups of its team and the slots - at the same place for every shape, so that a word never changes its meaning, and
-// allocated for kTeamChannels at once, so that it never moves.
-constexpr size_t kTeamStride = kTeamLine + kTeamMax * 16;
-constexpr size_t teamBytes(int C) { return 2 * kTeamLine + C * kTeamStride; }
+// The scratch: per channel two slots a piece, on cache lines of the channel's own.
+__host__ __device__ constexpr size_t teamStride(int pieces) { return (pieces * 16 + 127) / 128 * 128; }
 struct TeamArgs {
   char *block;
-  __device__ unsigned *epoch() const { return reinterpret_cast<unsigned *>(block); }
-  __device__ unsigned *done() const { return reinterpret_cast<unsigned *>(block + kTeamLine); }
-  __device__ unsigned *doneOf(int ch) const { return reinterpret_cast<unsigned *>(block + 2 * kTeamLine + ch * kTeamStride); }
-  __device__ unsigned long *slots(int ch) const {
-    return reinterpret_cast<unsigned long *>(block + 3 * kTeamLine + ch * kTeamStride);
-  }
+  __device__ unsigned long *slots(int ch) const { return reinterpret_cast<unsigned long *>(block + ch * teamStride(pieces)); }
+  unsigned tag;
   int pieces, units;                     // of a channel; units of a piece
   int spin;                              // polls before a workgroup helps itself
   int N, C, L;
@@ -104,7 +93,6 @@ struct TeamShared {
   float red[kTeamWaves];
   float stat[kTeamMax][2];
   double out[2];
-  unsigned tag;
 };
 
 // Publishes (a, b) of piece `piece` and gathers those of all pieces into sh.stat. Returns false when some have not
@@ -117,7 +105,7 @@ __device__ __forceinline__ bool teamExchange(const TeamArgs &t, int ch, int piec
   }
   unsigned long *slot = t.slots(ch);
   const int k = threadIdx.x;
-  const unsigned tag = sh.tag;
+  const unsigned tag = t.tag;
   if (k < kTeamMax / 32) missing[k] = 0;
   if (k == 0) {
     __hip_atomic_store(slot + 2 * piece, (unsigned long)tag << 32 | __float_as_uint(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -148,22 +136,6 @@ __device__ __forceinline__ bool teamExchange(const TeamArgs &t, int ch, int piec
   return __syncthreads_or(late) == 0;
 }
 
-// The launch's tag; every workgroup reads it before the last one can move it on.
-__device__ __forceinline__ void teamBegin(const TeamArgs &t, TeamShared &sh) {
-  if (threadIdx.x == 0 && t.pieces > 1) sh.tag = __hip_atomic_load(t.epoch(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-}
-// Called when a workgroup has read its team's slots. Two levels of counters (the last of a team counts the team): a single
-// one that a thousand workgroups add to costs 30 ns each.
-__device__ __forceinline__ void teamEnd(const TeamArgs &t, const TeamShared &sh, int ch) {
-  if (threadIdx.x != 0 || t.pieces == 1) return;
-  unsigned *of = t.doneOf(ch);
-  if (__hip_atomic_fetch_add(of, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != (unsigned)t.pieces) return;
-  __hip_atomic_store(of, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (__hip_atomic_fetch_add(t.done(), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != (unsigned)t.C) return;
-  __hip_atomic_store(t.done(), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(t.epoch(), sh.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // The backward pass: pieces of up to kTeamLanes * R units of V floats, R per lane, x and gradOutput of each.
 template <int V, int R>
 __global__ void __launch_bounds__(kTeamLanes, 4)
@@ -173,7 +145,6 @@ bnBwdTeam(const float *__restrict__ x, const float *__restrict__ gy, float *__re
   __shared__ TeamShared sh;
   __shared__ unsigned missing[kTeamMax / 32];
   const int ch = blockIdx.x / t.pieces, piece = blockIdx.x - ch * t.pieces;
-  teamBegin(t, sh);
   const float mean = meanSrc[ch], stdVal = stdSrc[ch], weightVal = weight ? weight[ch] : 1.f;
   const ChannelMask m(rm, ch, mean);
   const int total = t.N * (t.L / V);
@@ -208,7 +179,10 @@ bnBwdTeam(const float *__restrict__ x, const float *__restrict__ gy, float *__re
   load(piece);
   float s0, s1;
   statistics(s0, s1);
-  if (!teamExchange(t, ch, piece, s0, s1, sh, missing)) {
+  int late = !teamExchange(t, ch, piece, s0, s1, sh, missing);
+  // (opaque: compiled into two copies, with and without an exchange, the kernel keeps x and gradOutput twice and spills)
+  asm volatile("" : "+v"(late));
+  if (__builtin_amdgcn_readfirstlane(late)) {
 #pragma unroll 1
     for (int k = 0; k < t.pieces; ++k)
       if (missing[k >> 5] >> (k & 31) & 1) {
@@ -247,5 +221,4 @@ bnBwdTeam(const float *__restrict__ x, const float *__restrict__ gy, float *__re
     if (gradWeight) gradWeight[ch] += scale * dotP * stdVal;
     if (gradBias) gradBias[ch] += scale * gradOutputSum;
   }
-  teamEnd(t, sh, ch);
 }

@@ -14,11 +14,17 @@
 
 // Per stream: a block of device memory that entry points without a buffer argument use for their partial results
 // (cutorch keeps such a scratch space per device and stream as well). It grows on demand and lives as long as the state.
+enum {
+  kScratchCall,    // contents belong to the call at hand
+  kScratchTagged,  // taggedScratch
+  kScratchOutgrown // was kScratchTagged, held until the state ends: a captured graph may still use it
+};
 struct StreamScratch {
   hipStream_t stream;
-  int kind;     // 0: contents belong to the call at hand; 1: cleared when it is made, then kept from call to call
+  int kind;     // kScratch...
   void *ptr;
   size_t bytes;
+  unsigned tag; // kScratchTagged: the last one handed out
 };
 
 struct THCState {
@@ -132,12 +138,12 @@ void stridedCopy(hipStream_t stream, const Tensor *t, void *contig, size_t elemS
 // At least `bytes` of device memory that belongs to (state, current stream) and is reused by every call on that
 // stream: work that uses it is ordered by the stream. Allocates only when a call needs more than any earlier call
 // on the stream did (then the stream is drained before the smaller block is freed).
-// kind 1: a block of its own that is all zeros when it is made (and made anew when it grows) and keeps what kernels leave in it.
 void *streamScratch(THCState *state, size_t bytes);
-// A block of one size that is cleared when it is made and keeps its contents from call to call. It never moves, so a captured
-// graph may hold its address. nullptr (the caller takes a path without it) when there is none yet and the stream is being
-// captured or the memory is not to be had.
-void *keptScratch(THCState *state, size_t bytes);
+// `bytes` of device memory of (state, current stream) in which no 64-bit word has *tag in its upper half, for words that prove
+// themselves by it. A call under capture gets memory of its own, which a kernel in the graph clears before every replay: replays
+// leave nothing behind for eager calls, nor these for them, on whatever stream the graph is replayed. nullptr (the caller takes a path
+// without it) when memory is not to be had, or would have to be allocated while the stream is being captured.
+void *taggedScratch(THCState *state, size_t bytes, unsigned *tag);
 bool capturing(THCState *state);
 
 // Stream-ordered temporary: memory is returned to the pool after the work

@@ -102,13 +102,13 @@ static StreamScratch *scratchSlot(THCState *state, int kind) {
   for (StreamScratch &sc : state->scratch)
     if (sc.stream == state->stream && sc.kind == kind) slot = &sc;
   if (!slot) {
-    state->scratch.push_back(StreamScratch{state->stream, kind, nullptr, 0});
+    state->scratch.push_back(StreamScratch{state->stream, kind, nullptr, 0, 0});
     slot = &state->scratch.back();
   }
   return slot;
 }
 void *streamScratch(THCState *state, size_t bytes) {
-  StreamScratch *slot = scratchSlot(state, 0);
+  StreamScratch *slot = scratchSlot(state, kScratchCall);
   if (slot->bytes < bytes) {
     if (slot->ptr) {
       THC_HIP_CHECK(hipStreamSynchronize(state->stream));
@@ -127,23 +127,42 @@ bool capturing(THCState *state) {
   THC_HIP_CHECK(hipStreamIsCapturing(state->stream, &st));
   return st != hipStreamCaptureStatusNone;
 }
-void *keptScratch(THCState *state, size_t bytes) {
-  StreamScratch *slot = scratchSlot(state, 1);
-  if (!slot->ptr) {
-    if (capturing(state)) return nullptr;
+// The block is two halves: of eager calls, which count the tag up, and of captured ones.
+void *taggedScratch(THCState *state, size_t bytes, unsigned *tag) {
+  StreamScratch *slot = scratchSlot(state, kScratchTagged);
+  const bool inGraph = capturing(state);
+  if (slot->bytes < 2 * bytes) {
+    if (inGraph) return nullptr;
+    size_t half = 16384;
+    while (half < bytes) half *= 2;
     // another thread's capture neither forbids this allocation nor is ended by it
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     THC_HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
     void *p = nullptr;
-    const hipError_t e = hipMalloc(&p, bytes);
+    const hipError_t e = hipMalloc(&p, 2 * half);
     THC_HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
     if (e != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;
     }
-    slot->ptr = p, slot->bytes = bytes;
-    clearWords(state->stream, p, bytes);
+    if (slot->ptr) {
+      slot->kind = kScratchOutgrown;
+      slot = scratchSlot(state, kScratchTagged);
+    }
+    slot->ptr = p, slot->bytes = 2 * half, slot->tag = 0;
+    clearWords(state->stream, p, 2 * half);
   }
+  if (inGraph) {
+    void *p = (char *)slot->ptr + slot->bytes / 2;
+    clearWords(state->stream, p, bytes);
+    *tag = 1;
+    return p;
+  }
+  if (++slot->tag == 0) {  // every tag has been used
+    clearWords(state->stream, slot->ptr, slot->bytes / 2);
+    slot->tag = 1;
+  }
+  *tag = slot->tag;
   return slot->ptr;
 }
 

@@ -100,8 +100,8 @@ def test_by_shape_and_over_the_input(shape):
 
 @pytest.mark.parametrize("shape, warm", [((64, 128, 28, 28), False), ((64, 128, 28, 28), True), ((16, 40, 56, 56), True)])
 def test_capture(shape, warm):
-    """A call that has a kernel without scratch is captured on that kernel, also as the first call on its stream: bit for bit
-    what the switch that turns the teams off gives. One that always needed scratch is captured on the teams once they ran."""
+    """A call that has a kernel without scratch takes that one, captured also as the first call on its stream; one that always
+    needed scratch is captured on the teams once they ran. Either gives the bits of an eager call."""
     THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
     lib, st = cunn_amd._lib.load(), cunn_amd.tensor.state()
     hip = ctypes.CDLL("libamdhip64.so")
@@ -123,13 +123,8 @@ def test_capture(shape, warm):
         lib.THCState_synchronize(st)
         return [t.numpy().copy() for t in (gx, gg, gb)]
 
-    teams = C < 96
-    cunn_amd.set_switch("THCUNN_BN_TEAMS", None if teams else "0")
-    try:
-        backward()
-        expected = results()
-    finally:
-        cunn_amd.set_switch("THCUNN_BN_TEAMS", None)
+    backward()
+    expected = results()
     s, graph, run = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
     assert hip.hipStreamCreate(ctypes.byref(s)) == 0
     lib.THCState_setCurrentStream(st, s)
@@ -154,3 +149,63 @@ def test_capture(shape, warm):
         lib.THCState_synchronize(st)
         lib.THCState_setCurrentStream(st, None)
         hip.hipStreamDestroy(s)
+
+
+def test_replays_beside_eager_calls():
+    """A captured graph replayed on another stream while calls of other shapes run on the one it was captured on, and after a larger
+    call has made the scratch grow: neither side finds what the other leaves, then or later."""
+    THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
+    lib, st = cunn_amd._lib.load(), cunn_amd.tensor.state()
+    hip = ctypes.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(6)
+
+    def layer(shape):
+        C = shape[1]
+        f = lambda *s: CT.from_numpy(rng.standard_normal(s).astype(np.float32))
+        z = lambda: CT.from_numpy(np.zeros(C, np.float32))
+        x, gy, w, rm, rv, sm, ss, gg, gb = f(*shape), f(*shape), f(C), z(), CT.from_numpy(np.ones(C, np.float32)), z(), z(), z(), z()
+        y, gx = CT.from_numpy(np.zeros(shape, np.float32)), CT.from_numpy(np.zeros(shape, np.float32))
+        THNN.BatchNormalization_updateOutput(x, y, w, z(), rm, rv, sm, ss, True, 0.1, 1e-5)
+
+        def backward():
+            for t in (gg, gb):
+                lib.THCudaTensor_fill(st, t.handle, 0.0)
+            THNN.BatchNormalization_backward(x, gy, gx, gg, gb, w, rm, rv, sm, ss, True, 1.0, 1e-5)
+        return backward, lambda: [t.numpy().copy() for t in (gx, gg, gb)], gx
+
+    (graphed, graphed_out, graphed_gx), (eager, eager_out, _), (larger, larger_out, _) = (
+        layer(s) for s in ((16, 40, 56, 56), (16, 24, 72, 72), (64, 48, 112, 112)))
+    s, t, graph, run = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(s)) == 0 and hip.hipStreamCreate(ctypes.byref(t)) == 0
+    lib.THCState_setCurrentStream(st, s)
+    try:
+        graphed(), eager()
+        lib.THCState_synchronize(st)
+        want_graphed, want_eager = graphed_out(), eager_out()
+        assert hip.hipStreamBeginCapture(s, 0) == 0
+        graphed()
+        assert hip.hipStreamEndCapture(s, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+        for turn in range(3):
+            print("turn", turn, flush=True)
+            lib.THCudaTensor_fill(st, graphed_gx.handle, -7.0)
+            lib.THCState_synchronize(st)
+            for _ in range(20):
+                assert hip.hipGraphLaunch(run, t) == 0
+                eager()
+            if turn == 1:
+                larger()
+            lib.THCState_synchronize(st)
+            assert hip.hipStreamSynchronize(t) == 0
+            for got, want in ((graphed_out(), want_graphed), (eager_out(), want_eager)):
+                assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        want = larger_out()
+        larger()
+        lib.THCState_synchronize(st)
+        assert all(np.array_equal(a, b) for a, b in zip(larger_out(), want))
+        assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    finally:
+        lib.THCState_synchronize(st)
+        lib.THCState_setCurrentStream(st, None)
+        hip.hipStreamDestroy(s)
+        hip.hipStreamDestroy(t)
