@@ -198,6 +198,24 @@ def test_images_of_both_kinds_in_a_tile(case):
     _forward_and_grad_input(x, gy, w, 1, 1)
 
 
+def test_more_images_than_a_grid_dimension_holds():
+    """70000 images of one position each: 256 of them in a tile, of both kinds; all three passes."""
+    rng = np.random.default_rng(9)
+    N, Ci, Co, k = 70000, 16, 8, 2
+    x, w, gy = (rng.standard_normal(s).astype(np.float32) for s in ((N, Ci, k, k), (Co, Ci, k, k), (N, Co, 1, 1)))
+    x[::1000, :5] *= np.float32(1e-20)
+    x[1::1000, 5:] = 0
+    gy[2::1000, 1:] *= np.float32(1e-20)
+    CT, y, gx = cunn_amd.CudaTensor, cunn_amd.CudaTensor(), cunn_amd.CudaTensor()
+    THNN, tw, a = cunn_amd.THNN, CT.from_numpy(w.reshape(Co, -1)), (k, k, 1, 1, 0, 0)
+    THNN.SpatialConvolutionMM_updateOutput(CT.from_numpy(x), y, tw, None, CT(), CT(), *a)
+    THNN.SpatialConvolutionMM_updateGradInput(CT.from_numpy(x), CT.from_numpy(gy), gx, tw, CT(), CT(), *a)
+    xd, wd, gd = (v.astype(np.float64) for v in (x.reshape(N, -1), w.reshape(Co, -1), gy.reshape(N, Co)))
+    for got, p, q in ((y.numpy().reshape(N, Co), xd, wd.T), (gx.numpy().reshape(N, -1), gd, wd),
+                      (_weight_gradient(x, gy, k, 1, 0), gd.T, xd)):
+        assert (np.abs(got - p @ q) <= p.shape[1] * 2.0 ** -24 * (np.abs(p) @ np.abs(q)) + 2.0 ** -149).all()
+
+
 @pytest.mark.parametrize("relu", [False, True])
 def test_bias_relu_and_buffers(relu):
     """Bias and clamp in the epilogue; a buffer tensor that is too small and cannot grow leaves the call to the other kernels."""
