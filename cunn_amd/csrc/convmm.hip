@@ -2615,44 +2615,42 @@ double termsOf(const FwdPlan &pl, int K) {
 }
 
 // ---- pointwise forward -------------------------------------------------------------------------
-// Launch shape of convPointwiseKernel for an M x K weight matrix: rows per wave, waves along the rows, column
-// tiles per chunk, waves per workgroup.
+// Launch shape of convPointwiseKernel for M rows: blocks of 32 rows per wave, waves along the rows. One workgroup of 8 waves
+// per CU; a chunk of positions is 64 KB of x, two of them in LDS (32 -> 64 at 112 x 112, N = 64, 44.9 us). Outputs of 32 rows or
+// fewer are left to the tiled GEMM, which measured faster.
 struct PwShape {
-  int mr, wr, ct, nw;
+  int mr, wr;
 };
-// K = 32: one workgroup of 8 waves per CU; a chunk of positions is 64 KB of x, two of them in LDS (32 -> 64 at 112 x 112,
-// N = 64, 44.9 us). Outputs of 32 rows or fewer are left to the tiled GEMM, which measured faster.
 bool pwShape(int M, PwShape *sh) {
   if (M >= 256)
-    *sh = {2, 4, 16, 8};  // 256 rows per workgroup
+    *sh = {2, 4};  // 256 rows per workgroup
   else if (M > 64)
-    *sh = {1, 4, 16, 8};  // 128 rows, two waves along the positions
+    *sh = {1, 4};  // 128 rows, two waves along the positions
   else if (M > 32)
-    *sh = {1, 2, 16, 8};  // 64 rows, four waves along the positions
+    *sh = {1, 2};  // 64 rows, four waves along the positions
   else
     return false;
   return true;
 }
 
-template <int K, int MR, int WR, int CT, int NW, bool RELU, bool TRANS>
-void launchPointwiseShape(hipStream_t s, PwArgs p, int device) {
-  constexpr size_t lds = (size_t)pwLdsFloats(K, MR, WR, CT) * sizeof(float);
-  auto kernel = convPointwiseKernel<K, MR, WR, CT, NW, RELU, TRANS>;
-  if (lds > 64 * 1024) {  // once per kernel instance and device: allow more than 64 KB of dynamic LDS
-    static std::atomic<bool> raised[64];
-    if (!raised[device].load()) {
-      THC_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-      raised[device].store(true);
-    }
+template <int MR, int WR>
+void launchPointwise(hipStream_t s, PwArgs p, int device, bool relu, bool transW) {
+  constexpr int lds = kPwLdsFloats * (int)sizeof(float);
+  const int form = transW ? 2 : relu ? 1 : 0;
+  auto kernel = transW ? convPointwiseKernel<MR, WR, false, true>
+                : relu ? convPointwiseKernel<MR, WR, true, false>
+                       : convPointwiseKernel<MR, WR, false, false>;
+  static std::atomic<bool> raised[3][64];  // once per kernel instance and device: allow more than 64 KB of dynamic LDS
+  if (!raised[form][device].load()) {
+    THC_HIP_CHECK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    raised[form][device].store(true);
   }
-  const int rowsPerWg = 32 * MR * WR;
-  const int rowBlocks = launch::ceilDiv(p.M, rowsPerWg);
-  // one workgroup per CU (two of the 4-wave shapes), shared between the row blocks; each streams a run of column tiles
-  int slots = std::max(1, residentSlots(nullptr) / rowBlocks);  // every shape fills a CU with one workgroup
+  const int rowBlocks = launch::ceilDiv(p.M, 32 * MR * WR);
+  // one workgroup per CU, shared between the row blocks; each streams a run of column tiles
+  int slots = std::max(1, residentSlots(nullptr) / rowBlocks);
   if (g_switches.convPointwise > 1) slots = std::min(slots, g_switches.convPointwise);  // tests: long runs of tiles per workgroup
   p.tilesPerWg = launch::ceilDiv(p.nTiles, std::min(slots, p.nTiles));
-  const int gx = launch::ceilDiv(p.nTiles, p.tilesPerWg);
-  kernel<<<dim3(gx, rowBlocks), 64 * NW, lds, s>>>(p);
+  kernel<<<dim3(launch::ceilDiv(p.nTiles, p.tilesPerWg), rowBlocks), 64 * kPwWaves, lds, s>>>(p);
   THC_HIP_CHECK(hipGetLastError());
 }
 
@@ -2735,24 +2733,18 @@ bool convPointwise(THCState *state, const ConvGeom &g, const float *x, const flo
   if (g.K == 64) return split(std::integral_constant<int, 64>{});
   if (g.K == 128) return split(std::integral_constant<int, 128>{});
   if (g.K == 256) return launchPointwiseSplit<256, 2, 2>(s, p, relu, transW), true;
-#define PW_CASE(KK, MRR, WRR, CTT, NWW)                                              \
-  if (g.K == KK && sh.mr == MRR && sh.wr == WRR && sh.ct == CTT && sh.nw == NWW) {   \
-    if (transW)                                                                      \
-      launchPointwiseShape<KK, MRR, WRR, CTT, NWW, false, true>(s, p, device);       \
-    else if (relu)                                                                   \
-      launchPointwiseShape<KK, MRR, WRR, CTT, NWW, true, false>(s, p, device);       \
-    else                                                                             \
-      launchPointwiseShape<KK, MRR, WRR, CTT, NWW, false, false>(s, p, device);      \
-    return true;                                                                     \
-  }
-  PW_CASE(32, 2, 4, 16, 8) PW_CASE(32, 1, 4, 16, 8) PW_CASE(32, 1, 2, 16, 8)
-#undef PW_CASE
-  return false;
+  if (sh.mr == 2)
+    launchPointwise<2, 4>(s, p, device, relu, transW);
+  else if (sh.wr == 4)
+    launchPointwise<1, 4>(s, p, device, relu, transW);
+  else
+    launchPointwise<1, 2>(s, p, device, relu, transW);
+  return true;
 }
 
 // ---- long convolutions on half-precision parts (conv_halves.h) ----------------------------------
 // For the passes with sums long enough that these parts are no less exact than the kernels above and enough work to pay for
-// the two launches that look for the largest element and split the operands.
+// the two launches that take the ranges of the operands and split them.
 struct HalvesGemm {        // one GEMM: output positions nH x nW, its window, and where its elements go
   int nH, nW, dH, dW;
   SplitAxis h, v;
@@ -2800,10 +2792,7 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   // terms, 1.4e-7 at 3000, 1.6e-7 at 24000), that of the other ones with the square root of those that one accumulator
   // gets (1.3e-7 at 560, 1.5e-7 at 720, 2.9e-7 at 2304; K split over workgroups or waves gives each fewer).
   if (force < 0 && (C * maxTaps < 550 || oldTerms() < 550 + C * maxTaps / 36.0)) return false;
-  int group = (int)std::min<long>(N, std::max<long>(1, 0x7fffffffL / 2 / maxL));
-  group = (int)std::min<long>(group, std::max<long>(1, ((1L << 31) - 1 - 4096) / std::max(imgBytes, xImgBytes)));
-  if (group < N && force < 0) return false;
-  group = std::min(group, N);
+  if (N * maxL > 0x7fffffffL / 2 || N * std::max(imgBytes, xImgBytes) > (1L << 31) - 1 - 4096) return false;
 
   // scratch: ranges and forms of images and rows, items, split weights, split images, partial tiles
   long at = 0;
@@ -2820,14 +2809,14 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   // slices of an image that rangesKernel reads, a power of two: enough workgroups to fill the chip, at least 4096 floats each
   const long perImg = (long)C * H * W;
   int nSlots = 1;
-  while (nSlots < kMaxSlots && 2 * nSlots <= perImg / 4096 && nSlots < launch::ceilDiv(2048, group)) nSlots *= 2;
-  const long slots = take((long)group * nSlots * sizeof(uint2)), imgForm = take((long)group * 4), rowRanges = take(M * (long)sizeof(uint2));
+  while (nSlots < kMaxSlots && 2 * nSlots <= perImg / 4096 && nSlots < launch::ceilDiv(2048, N)) nSlots *= 2;
+  const long slots = take((long)N * nSlots * sizeof(uint2)), imgForm = take((long)N * 4), rowRanges = take(M * (long)sizeof(uint2));
   long minL = LONG_MAX;
   for (int i = 0; i < count; ++i) {
     const HalvesGemm &G = gemm[i];
     itemsPad[i] = launch::roundUp(groups * G.h.n * G.v.n, kStageItems);
     pl[i] = FwdPlan{};
-    planTiles(pl[i], M, (long)group * G.nH * G.nW, itemsPad[i] / kStageItems, true, 5.0, false);
+    planTiles(pl[i], M, (long)N * G.nH * G.nW, itemsPad[i] / kStageItems, true, 5.0, false);
     bm = pl[i].bm, bn = pl[i].bn;
     rows = launch::roundUp(M, bm);
     const long splitBytes = (long)rows * itemsPad[i] * 32;
@@ -2838,7 +2827,7 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   }
   const int reach = (int)((bn - 2) / minL) + 1;  // images of a tile lie at most that far from each other
   if ((reach + 1) * (imgBytes / 2 * 3) >= 0x7fffffffL) return false;
-  const long images = take(group * imgBytes), images3 = take(group * (imgBytes / 2 * 3));
+  const long images = take(N * imgBytes), images3 = take(N * (imgBytes / 2 * 3));
   // several GEMMs (phases) in one launch: their tiles fill each other's last rounds, no tile is split
   if (count > 1)
     for (int i = 0; i < count; ++i)
@@ -2849,101 +2838,93 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   Temp tmp;
   char *buf = reinterpret_cast<char *>(scratchFloats(state, scratchBuf, at / 4, tmp, bufName));
   hipStream_t s = state->stream;
-  for (int first = 0; first < N; first += group) {
-    const int cnt = std::min(group, N - first);
-    const float *xg = x + (long)first * perImg;
-    RangeArgs ra{};
-    ra.x = xg, ra.slots = (uint2 *)(buf + slots), ra.perImg = perImg, ra.perSlice = (int)((perImg + nSlots - 1) / nSlots + 3) / 4 * 4;
-    ra.nSlots = nSlots, ra.vec = perImg % 4 == 0 && launch::aligned16(xg);
-    ra.w = w, ra.rows = (uint2 *)(buf + rowRanges), ra.M = M, ra.rs = rs, ra.cs = cs, ra.C = C, ra.taps = std::min(rs, cs);
-    rangesKernel<<<(unsigned)(M + cnt * nSlots), dev::kBlock, 0, s>>>(ra);
-    THC_HIP_CHECK(hipGetLastError());
-    SplitJobs J{};
-    SplitImages &I = J.im;
-    I.x = xg, I.dst = (u32x4 *)(buf + images), I.dst3 = (u32x4 *)(buf + images3), I.slots = (uint2 *)(buf + slots);
-    I.forms = (int *)(buf + imgForm);
-    I.nSlots = nSlots, I.N = cnt, I.C = C, I.H = H, I.W = W, I.top = -lowH, I.left = -lowW, I.Hp = (int)Hp, I.Wp = (int)Wp;
-    I.groups = groups, I.chunks = chunks, I.reach = reach, I.blocks = cnt * groups * chunks, I.magicW = dev::magicOf((int)Wp);
-    J.count = count;
-    long blocks = I.blocks;
-    HalvesBatch<kMaxHalvesJobs> batch{};
-    FwdBatch foldBatch{};
-    int wholeTotal = 0, splitTotal = 0, maxTail = 0;
-    for (int i = 0; i < count; ++i) {
-      const HalvesGemm &G = gemm[i];
-      SplitRows &R = J.rows[i];
-      R.w = w, R.dst = (u32x4 *)(buf + split[i]), R.dst3 = (u32x4 *)(buf + split3[i]);
-      R.ranges = (uint2 *)(buf + rowRanges), R.forms = (int *)(buf + rowForm[i]);
-      R.items = (int *)(buf + items[i]), R.items3 = R.items + itemsPad[i] + 4 * kStageItems;
-      R.rs = rs, R.cs = cs, R.kW = kW, R.M = M, R.rows = rows, R.C = C, R.tileRows = bm, R.itemsPad = itemsPad[i];
-      R.h = G.h, R.v = G.v;
-      blocks += rows + 1;
-      HalvesItem &it = batch.item[i];
-      HalvesArgs &q = it.q;
-      q.a = R.dst, q.b = I.dst, q.a3 = R.dst3, q.b3 = I.dst3, q.items = R.items, q.items3 = R.items3;
-      q.rowForm = R.forms, q.imgForm = I.forms, q.imgBytes = imgBytes, q.planeBytes = (int)(Hp * Wp * 16);
-      q.nItems = groups * G.h.n * G.v.n, q.itemsPad = itemsPad[i];
-      q.w = w, q.x = xg, q.wBytes = (int)(wFloats * 4), q.xBytes = (int)(cnt * xImgBytes);
-      q.rs = rs, q.cs = cs, q.kW = kW, q.C = C, q.H = H, q.W = W, q.h = G.h, q.v = G.v;
-      q.magicT = dev::magicOf(G.h.n * G.v.n), q.magicV = dev::magicOf(G.v.n);
-      ConvGeom &gk = it.g;
-      gk.N = cnt, gk.Cin = C, gk.Cout = M, gk.H = (int)Hp, gk.W = (int)Wp, gk.oH = G.nH, gk.oW = G.nW;
-      gk.kH = G.h.n, gk.kW = G.v.n, gk.dH = G.dH, gk.dW = G.dW, gk.dilH = gk.dilW = 1;
-      gk.K = itemsPad[i] * kHalvesGroup, gk.L = G.nH * G.nW;
-      if (cnt != group) {  // the last, smaller group: the same tile shape, no splits beyond what the scratch holds
-        pl[i].total = pl[i].mTiles * (int)tiles((long)cnt * gk.L, bn);
-        pl[i].full = pl[i].total, pl[i].tail = 0, pl[i].nSplit = 1, pl[i].ktPerSplit = itemsPad[i] / kStageItems;
-      }
-      FwdArgs &a = it.p;
-      a.bias = bias, a.relu = relu ? 1 : 0;
-      a.M = M, a.Ncols = cnt * gk.L;
-      a.out = out + (long)first * outImg + G.outOfs;
-      a.outImg = outImg, a.outRow = outRow, a.outSH = G.outSH, a.outSW = G.outSW;
-      const long spanBytes = ((long)(cnt - 1) * outImg + (long)(M - 1) * outRow + (long)(G.nH - 1) * G.outSH + (long)(G.nW - 1) * G.outSW + 1) * 4;
-      a.outBytes = spanBytes < 0x7fffffffL ? (int)spanBytes : 0;
-      a.magicL = (long)a.Ncols * gk.L < 0xffffffffL ? dev::magicOf(gk.L) : 0;
-      a.magicOW = (long)gk.L * gk.oW < 0xffffffffL ? dev::magicOf(gk.oW) : 0;
-      a.mTiles = pl[i].mTiles, a.bm = bm, a.bn = bn;
-      a.full = pl[i].full, a.tail = pl[i].tail, a.tile0 = pl[i].full;
-      a.nSplit = a.tail > 0 ? pl[i].nSplit : 1;
-      a.ktPerSplit = a.tail > 0 ? pl[i].ktPerSplit : itemsPad[i] / kStageItems;
-      a.partial = (float *)(buf + partial[i]);
-      wholeTotal += a.full, splitTotal += a.tail * a.nSplit;
-      it.wholeEnd = wholeTotal, it.splitEnd = splitTotal;
-      maxTail = std::max(maxTail, a.tail);
-      foldBatch.item[i].p = a, foldBatch.item[i].g = gk;
+  RangeArgs ra{};
+  ra.x = x, ra.slots = (uint2 *)(buf + slots), ra.perImg = perImg, ra.perSlice = (int)((perImg + nSlots - 1) / nSlots + 3) / 4 * 4;
+  ra.nSlots = nSlots, ra.vec = perImg % 4 == 0 && launch::aligned16(x);
+  ra.w = w, ra.rows = (uint2 *)(buf + rowRanges), ra.M = M, ra.rs = rs, ra.cs = cs, ra.C = C, ra.taps = std::min(rs, cs);
+  rangesKernel<<<(unsigned)(M + N * nSlots), dev::kBlock, 0, s>>>(ra);
+  THC_HIP_CHECK(hipGetLastError());
+  SplitJobs J{};
+  SplitImages &I = J.im;
+  I.x = x, I.dst = (u32x4 *)(buf + images), I.dst3 = (u32x4 *)(buf + images3), I.slots = (uint2 *)(buf + slots);
+  I.forms = (int *)(buf + imgForm);
+  I.nSlots = nSlots, I.N = N, I.C = C, I.H = H, I.W = W, I.top = -lowH, I.left = -lowW, I.Hp = (int)Hp, I.Wp = (int)Wp;
+  I.groups = groups, I.chunks = chunks, I.reach = reach, I.blocks = N * groups * chunks, I.magicW = dev::magicOf((int)Wp);
+  J.count = count;
+  long blocks = I.blocks;
+  HalvesBatch<kMaxHalvesJobs> batch{};
+  FwdBatch foldBatch{};
+  int wholeTotal = 0, splitTotal = 0, maxTail = 0;
+  for (int i = 0; i < count; ++i) {
+    const HalvesGemm &G = gemm[i];
+    SplitRows &R = J.rows[i];
+    R.w = w, R.dst = (u32x4 *)(buf + split[i]), R.dst3 = (u32x4 *)(buf + split3[i]);
+    R.ranges = (uint2 *)(buf + rowRanges), R.forms = (int *)(buf + rowForm[i]);
+    R.items = (int *)(buf + items[i]), R.items3 = R.items + itemsPad[i] + 4 * kStageItems;
+    R.rs = rs, R.cs = cs, R.kW = kW, R.M = M, R.rows = rows, R.C = C, R.tileRows = bm, R.itemsPad = itemsPad[i];
+    R.h = G.h, R.v = G.v;
+    blocks += rows + 1;
+    HalvesItem &it = batch.item[i];
+    HalvesArgs &q = it.q;
+    q.a = R.dst, q.b = I.dst, q.a3 = R.dst3, q.b3 = I.dst3, q.items = R.items, q.items3 = R.items3;
+    q.rowForm = R.forms, q.imgForm = I.forms, q.imgBytes = imgBytes, q.planeBytes = (int)(Hp * Wp * 16);
+    q.nItems = groups * G.h.n * G.v.n, q.itemsPad = itemsPad[i];
+    q.w = w, q.x = x, q.wBytes = (int)(wFloats * 4), q.xBytes = (int)(N * xImgBytes);
+    q.rs = rs, q.cs = cs, q.kW = kW, q.C = C, q.H = H, q.W = W, q.h = G.h, q.v = G.v;
+    q.magicT = dev::magicOf(G.h.n * G.v.n), q.magicV = dev::magicOf(G.v.n);
+    ConvGeom &gk = it.g;
+    gk.N = N, gk.Cin = C, gk.Cout = M, gk.H = (int)Hp, gk.W = (int)Wp, gk.oH = G.nH, gk.oW = G.nW;
+    gk.kH = G.h.n, gk.kW = G.v.n, gk.dH = G.dH, gk.dW = G.dW, gk.dilH = gk.dilW = 1;
+    gk.K = itemsPad[i] * kHalvesGroup, gk.L = G.nH * G.nW;
+    FwdArgs &a = it.p;
+    a.bias = bias, a.relu = relu ? 1 : 0;
+    a.M = M, a.Ncols = N * gk.L;
+    a.out = out + G.outOfs;
+    a.outImg = outImg, a.outRow = outRow, a.outSH = G.outSH, a.outSW = G.outSW;
+    const long spanBytes = ((long)(N - 1) * outImg + (long)(M - 1) * outRow + (long)(G.nH - 1) * G.outSH + (long)(G.nW - 1) * G.outSW + 1) * 4;
+    a.outBytes = spanBytes < 0x7fffffffL ? (int)spanBytes : 0;
+    a.magicL = (long)a.Ncols * gk.L < 0xffffffffL ? dev::magicOf(gk.L) : 0;
+    a.magicOW = (long)gk.L * gk.oW < 0xffffffffL ? dev::magicOf(gk.oW) : 0;
+    a.mTiles = pl[i].mTiles, a.bm = bm, a.bn = bn;
+    a.full = pl[i].full, a.tail = pl[i].tail, a.tile0 = pl[i].full;
+    a.nSplit = a.tail > 0 ? pl[i].nSplit : 1;
+    a.ktPerSplit = a.tail > 0 ? pl[i].ktPerSplit : itemsPad[i] / kStageItems;
+    a.partial = (float *)(buf + partial[i]);
+    wholeTotal += a.full, splitTotal += a.tail * a.nSplit;
+    it.wholeEnd = wholeTotal, it.splitEnd = splitTotal;
+    maxTail = std::max(maxTail, a.tail);
+    foldBatch.item[i].p = a, foldBatch.item[i].g = gk;
+  }
+  batch.count = foldBatch.count = count, batch.wholeTotal = wholeTotal;
+  splitOperandsKernel<<<(unsigned)blocks, dev::kBlock, 0, s>>>(J);
+  THC_HIP_CHECK(hipGetLastError());
+  const dim3 grid(wholeTotal + splitTotal);
+  auto launchShape = [&](auto wr, auto wc, auto ti, auto tj) {
+    constexpr int A = decltype(wr)::value, B = decltype(wc)::value, I2 = decltype(ti)::value, J2 = decltype(tj)::value;
+    if (count == 1) {
+      HalvesBatch<1> one{};
+      one.item[0] = batch.item[0], one.count = 1, one.wholeTotal = wholeTotal;
+      convHalvesKernel<1, A, B, I2, J2><<<grid, dev::kBlock, 0, s>>>(one);
+    } else {
+      convHalvesKernel<kMaxHalvesJobs, A, B, I2, J2><<<grid, dev::kBlock, 0, s>>>(batch);
     }
-    batch.count = foldBatch.count = count, batch.wholeTotal = wholeTotal;
-    splitOperandsKernel<<<(unsigned)blocks, dev::kBlock, 0, s>>>(J);
+  };
+  using N1 = std::integral_constant<int, 1>;
+  using N2 = std::integral_constant<int, 2>;
+  using N3 = std::integral_constant<int, 3>;
+  using N4 = std::integral_constant<int, 4>;
+  if (bm == 32)
+    launchShape(N1{}, N4{}, N1{}, N2{});
+  else if (bm == 64)
+    launchShape(N1{}, N4{}, N2{}, N1{});
+  else if (bm == 96)
+    launchShape(N1{}, N4{}, N3{}, N1{});
+  else
+    launchShape(N2{}, N2{}, N2{}, N2{});
+  THC_HIP_CHECK(hipGetLastError());
+  if (maxTail > 0) {
+    fwdTailFixupBatchKernel<<<dim3(maxTail, BM * BN / (4 * dev::kBlock), count), dev::kBlock, 0, s>>>(foldBatch);
     THC_HIP_CHECK(hipGetLastError());
-    const dim3 grid(wholeTotal + splitTotal);
-    auto launchShape = [&](auto wr, auto wc, auto ti, auto tj) {
-      constexpr int A = decltype(wr)::value, B = decltype(wc)::value, I2 = decltype(ti)::value, J2 = decltype(tj)::value;
-      if (count == 1) {
-        HalvesBatch<1> one{};
-        one.item[0] = batch.item[0], one.count = 1, one.wholeTotal = wholeTotal;
-        convHalvesKernel<1, A, B, I2, J2><<<grid, dev::kBlock, 0, s>>>(one);
-      } else {
-        convHalvesKernel<kMaxHalvesJobs, A, B, I2, J2><<<grid, dev::kBlock, 0, s>>>(batch);
-      }
-    };
-    using N1 = std::integral_constant<int, 1>;
-    using N2 = std::integral_constant<int, 2>;
-    using N3 = std::integral_constant<int, 3>;
-    using N4 = std::integral_constant<int, 4>;
-    if (bm == 32)
-      launchShape(N1{}, N4{}, N1{}, N2{});
-    else if (bm == 64)
-      launchShape(N1{}, N4{}, N2{}, N1{});
-    else if (bm == 96)
-      launchShape(N1{}, N4{}, N3{}, N1{});
-    else
-      launchShape(N2{}, N2{}, N2{}, N2{});
-    THC_HIP_CHECK(hipGetLastError());
-    if (maxTail > 0) {
-      fwdTailFixupBatchKernel<<<dim3(maxTail, BM * BN / (4 * dev::kBlock), count), dev::kBlock, 0, s>>>(foldBatch);
-      THC_HIP_CHECK(hipGetLastError());
-    }
   }
   return true;
 }
