@@ -2762,7 +2762,7 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   if (forceGeneric() || force == 0 || count < 1 || count > kMaxHalvesJobs || N < 1 || (force < 0 && C < 16)) return false;
   const int groups = launch::ceilDiv(C, kHalvesGroup);
   int lowH = 0, highH = H - 1, lowW = 0, highW = W - 1;  // rows and columns the windows touch
-  long maxL = 1;
+  long maxL = 1, minPositions = LONG_MAX;  // positions in steps of one
   double products = 0;
   long maxTaps = 0;
   for (int i = 0; i < count; ++i) {
@@ -2779,6 +2779,7 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
     span(G.h, G.nH, G.dH, lowH, highH);
     span(G.v, G.nW, G.dW, lowW, highW);
     maxL = std::max(maxL, (long)G.nH * G.nW);
+    minPositions = std::min(minPositions, (long)G.nH * G.nW * G.dH * G.dW);
     products += (double)N * G.nH * G.nW * M * C * taps;
   }
   const long Hp = (long)highH + 1 - lowH, Wp = (long)highW + 1 - lowW;
@@ -2788,10 +2789,13 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   // N = 6, 528 -> 264 3x3 on 37x37 208 / 108; N = 64, 256 -> 256 3x3 on 28x28 348 / 200; but 1x1 windows use every element
   // once (N = 32, 708 -> 272 on 26x62 163 / 187), and calls of less than half a billion products are two launches.
   if (force < 0 && (groups * kHalvesGroup * 4 > 5 * C || products < 0.5e9 || (count == 1 && maxTaps == 1))) return false;
-  // Precise enough: the error of these kernels hardly grows with the number of terms (1.2e-7 of the result's norm at 500
-  // terms, 1.4e-7 at 3000, 1.6e-7 at 24000), that of the other ones with the square root of those that one accumulator
-  // gets (1.3e-7 at 560, 1.5e-7 at 720, 2.9e-7 at 2304; K split over workgroups or waves gives each fewer).
-  if (force < 0 && (C * maxTaps < 550 || oldTerms() < 550 + C * maxTaps / 36.0)) return false;
+  // Precise enough: the error of these kernels hardly grows with the number of terms (1.2e-7 of the result's norm at 600
+  // terms, 1.3e-7 at 5000, 1.4e-7 at 10000), that of the other ones with the square root of those that one accumulator gets
+  // and that are not zero (K split over workgroups or waves gives each fewer, and so does a border). With both operands half zeros,
+  // as behind a ReLU, it is 1.04e-7 at 600 terms, 1.07e-7 at 700, 1.2e-7 at 850 and 1.4e-7 at 1500 (normal operands 1.3e-7 at
+  // 560, 2.9e-7 at 2304).
+  const double inside = std::min(1.0, (double)H * W / minPositions);  // share of a window's taps on the image, about
+  if (force < 0 && (C * maxTaps * inside < 850 || oldTerms() * inside < 850 + C * maxTaps * inside / 36.0)) return false;
   if (N * maxL > 0x7fffffffL / 2 || N * std::max(imgBytes, xImgBytes) > (1L << 31) - 1 - 4096) return false;
 
   // scratch: ranges and forms of images and rows, items, split weights, split images, partial tiles

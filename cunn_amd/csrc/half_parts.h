@@ -8,10 +8,12 @@
 // 2^-21 of itself at worst. hh' and the two small products are summed in fp32 accumulators of their own. Either split costs 6e-8 of the result's norm, which a fourth
 // product (l l') does not change (8.6e-8 at 48 terms with three and with four), so short sums are left to the six products
 // of bf16 parts (convmm.hip), whose error starts at 4e-8 but grows with the root of the number of terms. The GEMM of
-// conv_halves.h therefore also moves the sum of the large products to a third accumulator every kFoldTerms terms, so
-// that a sum of 2304 terms is rounded some 25 times at its full size and not 144 times, and the weight gradient takes
-// shorter partial sums. Error against 64 bits, normally distributed terms, K = 576 / 1152 / 2304 / 8192: 1.2e-7 / 1.3e-7 /
-// 1.4e-7 / 1.8e-7 in conv_halves.h; six bf16 products 1.4e-7 / 2.0e-7 / 2.9e-7 / 5.7e-7; the fp32 instruction three times that.
+// conv_halves.h therefore also moves the sum of the large products to a third accumulator every kFoldTerms terms, so that a sum
+// of 2304 terms is rounded some 25 times at its full size and not 144 times (a product of fp16 parts has 22 bits, so, unlike
+// one of bf16 parts, it is rounded with every addition), and the weight gradient takes shorter partial sums. Error against 64 bits,
+// normally distributed terms, K = 1152 / 2304 / 8192: 1.2e-7 / 1.3e-7 / 1.4e-7 in conv_halves.h; six bf16 products 2.0e-7 / 2.9e-7 /
+// 5.7e-7; the fp32 instruction three times that. Sums are given to these kernels where their error is no larger than that of the
+// others for operands half of which are zero, too (convmm.hip: convHalves, convGradWeight).
 //
 // The exponent e comes from the largest finite element of what shares one - an image, a weight row, the images of a partial
 // weight gradient - so nothing overflows; and the parts are only used where the smallest non-zero element of it, times 2^e, is
