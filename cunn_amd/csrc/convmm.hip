@@ -2785,10 +2785,15 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   const long Hp = (long)highH + 1 - lowH, Wp = (long)highW + 1 - lowW;
   const long imgBytes = Hp * Wp * groups * kHalvesGroup * 4, xImgBytes = (long)C * H * W * 4;
   if (imgBytes >= (1L << 30) || Hp * Wp * Wp >= 0xffffffffL || wFloats * 4 >= 0x7fffffffL || (long)C * H * W >= 0x7fffffffL) return false;
-  // Fast enough (us, other kernels / these, both passes over the operands included): N = 44, 112 -> 304 3x3 on 25x13 78 / 50;
-  // N = 6, 528 -> 264 3x3 on 37x37 208 / 108; N = 64, 256 -> 256 3x3 on 28x28 348 / 200; but 1x1 windows use every element
-  // once (N = 32, 708 -> 272 on 26x62 163 / 187), and calls of less than half a billion products are two launches.
-  if (force < 0 && (groups * kHalvesGroup * 4 > 5 * C || products < 0.5e9 || (count == 1 && maxTaps == 1))) return false;
+  // Fast enough: the products take about half the time (7.5 us less for 10^9), the ranges and the split read the images twice and
+  // write them once (the bordered copy of the other kernels, where there is a border, does a third of that less), the weights
+  // are read twice and written in both forms by one workgroup a row, and there is a launch more. Over 2000 random layers the ones
+  // taken need 0.57 to 1.06 of the time of the other kernels, the ones left 0.67 to 2.0; e.g. (us, others / these) N = 64, 256 ->
+  // 256 3x3 on 28x28 332 / 199; N = 58, 223 -> 54 3x3 stride 2 on 64x26 59 / 84; N = 9, 361 -> 156 7x7 on 26x9 70 / 76. 1x1 windows
+  // use every element once (N = 32, 708 -> 272 on 26x62 163 / 187). Phases are not split along K: they have to fill the chip
+  // (gradInput, N = 14, 120 -> 311 7x7 stride 2 on 26x42 106 / 142).
+  const double moved = (double)N * C * H * W * (Hp * Wp != (long)H * W ? 4 : 12) + 48.0 * wFloats;
+  if (force < 0 && (groups * kHalvesGroup * 4 > 5 * C || products * 7.5e-9 < 6.0 + moved / 6e6 || (count == 1 && maxTaps == 1))) return false;
   // Precise enough: the error of these kernels hardly grows with the number of terms (1.2e-7 of the result's norm at 600
   // terms, 1.3e-7 at 5000, 1.4e-7 at 10000), that of the other ones with the square root of those that one accumulator gets
   // and that are not zero (K split over workgroups or waves gives each fewer, and so does a border). With both operands half zeros,
@@ -2833,9 +2838,14 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   if ((reach + 1) * (imgBytes / 2 * 3) >= 0x7fffffffL) return false;
   const long images = take(N * imgBytes), images3 = take(N * (imgBytes / 2 * 3));
   // several GEMMs (phases) in one launch: their tiles fill each other's last rounds, no tile is split
-  if (count > 1)
-    for (int i = 0; i < count; ++i)
+  if (count > 1) {
+    int total = 0;
+    for (int i = 0; i < count; ++i) {
       pl[i].tail = 0, pl[i].full = pl[i].total, pl[i].nSplit = 1, pl[i].ktPerSplit = itemsPad[i] / kStageItems;
+      total += pl[i].total;
+    }
+    if (force < 0 && total < residentSlots(nullptr)) return false;
+  }
   for (int i = 0; i < count; ++i) partial[i] = take(partialFloats(pl[i]) * 4);
   if (!roomFor(state, scratchBuf, at / 4)) return false;
 
