@@ -1758,9 +1758,9 @@ convGradWeightSmallKernel(GradWeightArgs p, ConvGeom g) {
 // WM = 2: 128 x 128 tiles of gradWeight (Cout x K), WM = 1: 64 x 256 tiles; a wave multiplies 64 x 64 either way.
 // A block whose sums are not all finite is computed again with the fp32 instruction, straight from memory.
 // HALVES: for long reductions. A split whose images are held by two fp16 parts (half_parts.h), scaled by the largest element
-// of either operand among them, takes these and three products, any other split the three bf16 parts; twice as many splits
-// keep the sums as exact as six products do. Whole pass, ranges (20 / 38 us) and a longer fold (5) included, us: 256 x 2304 over
-// 64 x 28 x 28 positions 339 -> 250 (374 where no split can), 192 x 720 over 32 x 71 x 71 372 -> 320 (419; 382 before).
+// of either operand among them, takes these and three products, any other split the three bf16 parts; five times as many
+// splits keep the sums as exact as six products do (there is no register left to fold them as conv_halves.h does). Whole pass,
+// ranges (20 us) and a longer fold (18) included, us: 256 x 2304 over 64 x 28 x 28 positions 339 -> 272 (395 where no split can).
 // What bounds it: as the forward kernel, two workgroups per CU and a clock that power pulls down. Against the fp32
 // instruction: 256 x 2304 over 64 x 28 x 28 positions (59.2 GFLOP) 519 -> 334 us; 192 x 720 over 32 x 71 x 71 (64 x 256
 // tiles, gathers transposed) 462 -> 342 us; 256 x 2048, stride 2, over 64 x 14 x 14 142 -> 99 us.
@@ -3639,25 +3639,32 @@ void convGradWeight(THCState *state, const ConvGeom &g, const float *x, const fl
   auto slices = [&](long perImg) { return (int)std::max<long>(1, std::min<long>(perImg / 4096, launch::ceilDiv(1024, g.N))); };
   const int gySlots = slices((long)g.Cout * g.L), xSlots = slices((long)g.Cin * g.H * g.W);
   const long rangeFloats = 2L * g.N * (gySlots + xSlots);
-  // Long reductions on half-precision parts, with twice the splits: their sums are then as exact as those of the six products
-  // (3.6e-7 of the norm at 3584 positions a split; on three products 2.9e-7 at 1792) from about 1100 positions a split on.
+  const long count = (long)g.Cout * g.K;
+  const bool fold4 = count % 4 == 0 && launch::aligned16(gW);
+  // Long reductions on half-precision parts, with five times the splits. That keeps their error no larger than that of six products
+  // from about 2800 positions a split of those on, with both operands half zeros, too (as behind a ReLU; a bf16 product adds
+  // without rounding, so six products are the better the fewer of the terms count): 3600 positions 2.0e-7 against 3.0e-7 with
+  // the input half zeros, 1.9e-7 against 2.15e-7 with both; and where the fold does not add all splits one after the other.
+  // Fast enough: the products take 4.5 us less for 10^9 of them (3.4 / 2.2 where the image is gathered element by element, with a
+  // stride), the ranges read both tensors and the splits leave more partials; where no split can take fp16 parts only that is left.
   const int perSplitSix = launch::ceilDiv(totalKt, splits) * BK;
+  const long moreSplits = std::min(totalKt, 5 * splits);
+  const double moved = 4.0 * g.N * ((double)g.Cin * g.H * g.W + (double)g.Cout * g.L) + 8.0 * (moreSplits - splits) * count;
+  const bool pays = fold4 && perSplitSix >= 2800 && (double)g.N * g.L * count * (b4 ? 4.5e-9 : g.dW == 1 ? 3.4e-9 : 2.2e-9) >= 1.5 * (3.0 + moved / 6e6);
   // (They need more scratch: not with a buffer that cannot grow.)
-  if (fast && !tiny && g_switches.convHalves != 0 && (perSplitSix >= 1100 || g_switches.convHalves == 1) &&
-      (!scratchBuf || (growable(scratchBuf) && roomFor(state, scratchBuf, 2 * splits * ((long)g.Cout * g.K + g.Cout) + xpFloats + gypFloats +
+  if (fast && !tiny && g_switches.convHalves != 0 && (pays || g_switches.convHalves == 1) &&
+      (!scratchBuf || (growable(scratchBuf) && roomFor(state, scratchBuf, moreSplits * (count + g.Cout) + xpFloats + gypFloats +
                                                                           rangeFloats + 16)))) {
     halves = true;
     gw = pick();
     kern = gw.fn;
-    splits = std::min(totalKt, 2 * splits);
+    splits = (int)moreSplits;
   }
   const int perSplit = launch::ceilDiv(totalKt, splits);
   splits = launch::ceilDiv(totalKt, perSplit);
-  const long count = (long)g.Cout * g.K;
   // scratch: the splits' partial products, then (second-generation kernel) the images with their zero border
   const long partialFloats = (splits * count + 3) / 4 * 4;
   // the bias gradient rides along when the fold below has the 16-byte form; else it is a pass of its own
-  const bool fold4 = count % 4 == 0 && launch::aligned16(gW);
   const bool fusedBias = gB && fast && fold4 && g.Cout % 4 == 0 && launch::aligned16(gB);
   const long biasFloats = fusedBias ? ((long)splits * g.Cout + 3) / 4 * 4 : 0;
   Temp tmp;

@@ -475,3 +475,37 @@ def test_no_less_exact_than_the_other_kernels(zeros):
             print(case, name, "error %.3g, the other kernels %.3g" % (error, before), flush=True)
             assert error <= 1.02 * before
     assert all(taken.values()), taken
+
+
+@pytest.mark.parametrize("zeros", ["none", "input", "both"])
+def test_weight_gradient_no_less_exact_than_the_other_kernels(zeros):
+    """The same for the weight gradient, around its line and inside; one layer each beyond the line, and without the 16-byte fold."""
+    import torch
+    taken = []
+    for case in ((64, 256, 256, 28, 28, 3, 1, 1), (30, 57, 120, 51, 48, 7, 1, 3), (15, 40, 371, 55, 42, 7, 1, 3), (32, 80, 192, 73, 73, 3, 1, 0),
+                 (16, 256, 256, 28, 28, 3, 1, 1), (55, 105, 221, 72, 25, 3, 1, 0)):
+        N, Ci, Co, H, W, k, st, pad = case
+        oH, oW = (H + 2 * pad - k) // st + 1, (W + 2 * pad - k) // st + 1
+        g = torch.Generator(device="cuda").manual_seed(N)
+        x, gy = (torch.randn(s, device="cuda", generator=g) for s in ((N, Ci, H, W), (N, Co, oH, oW)))
+        if zeros != "none":
+            x = x.clamp_min(0)
+        if zeros == "both":
+            gy = gy * (torch.rand(gy.shape, device="cuda", generator=g) < 0.5)
+        THNN, CT = cunn_amd.THNN, cunn_amd.CudaTensor
+        results = []
+        for switch in (None, "0"):
+            cunn_amd.set_switch("THCUNN_CONV_HALVES", switch)
+            gw = torch.zeros(Co, Ci * k * k, device="cuda")
+            THNN.SpatialConvolutionMM_accGradParameters(CT.from_torch(x), CT.from_torch(gy), CT.from_torch(gw), None, CT(), CT(),
+                                                        k, k, st, st, pad, pad, 1.0)
+            torch.cuda.synchronize()
+            results.append(gw)
+        if torch.equal(*results):
+            continue
+        taken.append(case)
+        ref = sum(gy[n].double().flatten(1) @ torch.nn.functional.unfold(x[n:n + 1].double(), k, padding=pad, stride=st)[0].t() for n in range(N))
+        error, before = (float((v.double() - ref).norm() / ref.norm()) for v in results)
+        print(case, zeros, "error %.3g, the other kernels %.3g" % (error, before), flush=True)
+        assert error <= 1.02 * before
+    assert 1 < len(taken) < 6, taken
