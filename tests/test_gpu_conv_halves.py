@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import cunn_amd
-from test_gpu_conv_split import SIZES, _check_error, _check_non_finite, _check_sizes
+from test_gpu_conv_split import SIZES, _check_error, _check_non_finite, _check_sizes, _passes, _tensors
 
 pytestmark = pytest.mark.gpu
 
@@ -47,6 +47,17 @@ def test_operands_of_all_kinds(case):
         print("case", case, sizes, flush=True)
         _check_sizes(case, *sizes)
     _check_non_finite(case)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_forced_passes_run_these_kernels(case):
+    """Other last bits than with the switch off, in the output and (1x1 windows aside) in gradInput; the weight gradient: LARGE."""
+    x, w, gy = _tensors(case, "normal")
+    here = _passes(case, x, w, gy, gy)
+    cunn_amd.set_switch("THCUNN_CONV_HALVES", "0")
+    other = _passes(case, x, w, gy, gy)
+    assert not np.array_equal(here[0], other[0])
+    assert case[5] == 1 or not np.array_equal(here[1], other[1])
 
 
 def _terms(x, w, dil):
@@ -359,6 +370,39 @@ def test_weight_gradient_of_mixed_rows(case, power, which):
     worst = np.abs(_weight_gradient(x, gy, k, st, pad) - ref) / (N * oH * oW * 2.0 ** -24 * terms + 2.0 ** -149)
     print("worst element at %.3g of its bound" % worst.max(), flush=True)
     assert worst.max() <= 1
+
+
+def test_buffers_of_a_fixed_size():
+    """A buffer tensor that cannot grow and holds just what the other kernels need leaves a call to those, bit for bit; one that holds
+    what these need does not (the weight gradient on half-precision parts asks for one that can grow)."""
+    import torch
+    CT, THNN = cunn_amd.CudaTensor, cunn_amd.THNN
+    rng = np.random.default_rng(11)
+    N, Ci, Co, H, k = 16, 64, 128, 24, 3
+    x, w, gy = (CT.from_numpy(rng.standard_normal(s).astype(np.float32)) for s in ((N, Ci, H, H), (Co, Ci * k * k), (N, Co, H, H)))
+    a = (k, k, 1, 1, 1, 1)
+
+    def call(which, buffer):
+        out = CT.from_numpy(np.zeros(((N, Co, H, H), (N, Ci, H, H), (Co, Ci * k * k))[which], np.float32))
+        if which == 0:
+            THNN.SpatialConvolutionMM_updateOutput(x, out, w, None, buffer, CT(), *a)
+        elif which == 1:
+            THNN.SpatialConvolutionMM_updateGradInput(x, gy, out, w, buffer, CT(), *a)
+        else:
+            THNN.SpatialConvolutionMM_accGradParameters(x, gy, out, None, buffer, CT(), *a, 1.0)
+        return out.numpy()
+
+    for which in range(3):
+        buffers, results = [], []
+        for switch in ("0", "1"):
+            cunn_amd.set_switch("THCUNN_CONV_HALVES", switch)
+            buffers.append(CT())
+            results.append(call(which, buffers[-1]))
+        small, large = (b.numpy().size for b in buffers)
+        print("pass", which, "floats", small, large, flush=True)
+        assert small < large and not np.array_equal(*results)
+        for floats, expected in ((small, results[0]), (large, results[0] if which == 2 else results[1])):
+            assert np.array_equal(call(which, CT.from_torch(torch.zeros(floats, device="cuda"))), expected)
 
 
 def test_captured_calls_do_not_allocate():
