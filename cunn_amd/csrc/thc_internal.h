@@ -140,8 +140,9 @@ void stridedCopy(hipStream_t stream, const Tensor *t, void *contig, size_t elemS
 // on the stream did (then the stream is drained before the smaller block is freed).
 void *streamScratch(THCState *state, size_t bytes);
 // `bytes` of device memory of (state, current stream) in which no 64-bit word has *tag in its upper half, for words that prove
-// themselves by it. A call under capture gets memory of its own, which a kernel in the graph clears before every replay: replays
-// leave nothing behind for eager calls, nor these for them, on whatever stream the graph is replayed. nullptr (the caller takes a path
+// themselves by it. Calls under capture get a half of the block that no eager call uses, which a kernel in the graph clears before every
+// replay: replays leave nothing behind for eager calls, nor these for them, on whatever stream the graph is replayed. Graphs captured
+// on one stream share it: replayed at the same time they can spoil each other's calls, and no later ones. nullptr (the caller takes a path
 // without it) when memory is not to be had, or would have to be allocated while the stream is being captured.
 void *taggedScratch(THCState *state, size_t bytes, unsigned *tag);
 bool capturing(THCState *state);

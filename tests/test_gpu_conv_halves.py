@@ -407,7 +407,7 @@ def test_buffers_of_a_fixed_size():
 
 def test_captured_calls_do_not_allocate():
     """Buffers sized by the other kernels' needs: a captured call takes what fits them (the weight gradient on half-precision
-    parts never does: twice the splits); after an eager call has sized them for these kernels, a captured one is theirs."""
+    parts never does: five times the splits); after an eager call has sized them for these kernels, a captured one is theirs."""
     import ctypes
     lib, st = cunn_amd._lib.load(), cunn_amd.tensor.state()
     hip = ctypes.CDLL("libamdhip64.so")
