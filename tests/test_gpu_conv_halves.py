@@ -9,6 +9,8 @@ import pytest
 import cunn_amd
 from test_gpu_conv_split import SIZES, _check_error, _check_non_finite, _check_sizes, _passes, _tensors
 
+from oracle import oracle as O
+
 pytestmark = pytest.mark.gpu
 
 # N, Cin, Cout, H, W, k, stride, pad
@@ -47,6 +49,35 @@ def test_operands_of_all_kinds(case):
         print("case", case, sizes, flush=True)
         _check_sizes(case, *sizes)
     _check_non_finite(case)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_large_and_non_finite_weights(case):
+    """Blocks that are computed again with weights whose bf16 parts overflow (2^104 and more), infinities, NaNs and subnormal ones: as the
+    oracle gives them (gradInput, where zeros beyond gradOutput meet the weights, without the infinities and NaNs). Bound for an
+    element: two chains of K fp32 additions, ours and the oracle's, each rounded by 2^-24 of what it adds up to at most, and, where sums are
+    subnormal, by 2^-150 (products of the subnormal row are smaller than that)."""
+    N, Ci, Co, H, W, k, st, pad = case
+    x, w, gy = _tensors(case, "normal", 7)
+    x, gy = x * np.float32(1e-4), gy * np.float32(1e-4)
+    w[3, 1], w[4, 2], w[5], w[Co - 1, Ci * k * k - 1] = 3e38, -2.0 ** 104, w[5] * 1e-42, 2.0 ** 110
+    g = (k, k, st, st, pad, pad)
+    for special in (False, True):
+        if special:
+            w[0, 3], w[1, 0], w[2, Ci * k * k - 2], x[0, 1, 2, 3] = np.inf, np.nan, -np.inf, np.inf
+        got = _passes(case, x, w, gy, gy)
+        with np.errstate(all="ignore"):
+            refs = (O.convmm_updateOutput(x, w, None, *g), O.convmm_updateGradInput(x.shape, gy, w, *g))
+            sums = (O.convmm_updateOutput(np.abs(x), np.abs(w), None, *g), O.convmm_updateGradInput(x.shape, np.abs(gy), np.abs(w), *g))
+        for name, here, ref, total, K in list(zip(("output", "gradInput"), got, refs, sums, (Ci * k * k, Co * k * k)))[:1 if special else 2]:
+            print(case, name, special, flush=True)
+            for f in (np.isnan, np.isposinf, np.isneginf):
+                assert np.array_equal(f(here), f(ref)), f.__name__
+            fine = np.isfinite(ref)
+            bound = 2 * K * (2.0 ** -24 * total[fine].astype(np.float64) + 2.0 ** -150)
+            worst = (np.abs(here[fine].astype(np.float64) - ref[fine]) / bound).max()
+            print("worst element at %.3g of its bound" % worst, flush=True)
+            assert worst <= 1
 
 
 @pytest.mark.parametrize("case", CASES)
