@@ -2785,15 +2785,17 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   const long Hp = (long)highH + 1 - lowH, Wp = (long)highW + 1 - lowW;
   const long imgBytes = Hp * Wp * groups * kHalvesGroup * 4, xImgBytes = (long)C * H * W * 4;
   if (imgBytes >= (1L << 30) || Hp * Wp * Wp >= 0xffffffffL || wFloats * 4 >= 0x7fffffffL || (long)C * H * W >= 0x7fffffffL) return false;
-  // Fast enough: the products take about half the time (7.5 us less for 10^9), the ranges and the split read the images twice and
-  // write them once (the bordered copy of the other kernels, where there is a border, does a third of that less), the weights
-  // are read twice and written in both forms by one workgroup a row, and there is a launch more. Over 2000 random layers the ones
-  // taken need 0.57 to 1.06 of the time of the other kernels, the ones left 0.67 to 2.0; e.g. (us, others / these) N = 64, 256 ->
-  // 256 3x3 on 28x28 332 / 199; N = 58, 223 -> 54 3x3 stride 2 on 64x26 59 / 84; N = 9, 361 -> 156 7x7 on 26x9 70 / 76. 1x1 windows
-  // use every element once (N = 32, 708 -> 272 on 26x62 163 / 187). Phases are not split along K: they have to fill the chip
-  // (gradInput, N = 14, 120 -> 311 7x7 stride 2 on 26x42 106 / 142).
+  // Fast enough: the products take about half the time (9 us less for 10^9 of them, on 98 layers of 100 at least 6; least with 2x2
+  // windows and few output planes), the ranges and the split read the images twice and write them once (the bordered copy of the
+  // other kernels, where there is a border, does a third of that less), the weights are read twice and written in both forms by
+  // one workgroup a row, and there is a launch more. Of 12000 random passes the ones taken need 0.4 to 1.07 of the time of the other
+  // kernels, one in a thousand more than all of it; with 7.5 us in the place of 6 the worst needed 1.28 (N = 5, 471 -> 44 2x2
+  // on 75x85: 92 us on the others, 117 on these). E.g. (us, others / these) N = 64, 256 -> 256 3x3 on 28x28 332 / 199; left: N = 58,
+  // 223 -> 54 3x3 stride 2 on 64x26 59 / 84; N = 9, 361 -> 156 7x7 on 26x9 70 / 76. 1x1 windows use every element once
+  // (N = 32, 708 -> 272 on 26x62 163 / 187). Phases are not split along K: they have to fill the chip (gradInput, N = 14, 120 -> 311
+  // 7x7 stride 2 on 26x42 106 / 142).
   const double moved = (double)N * C * H * W * (Hp * Wp != (long)H * W ? 4 : 12) + 48.0 * wFloats;
-  if (force < 0 && (groups * kHalvesGroup * 4 > 5 * C || products * 7.5e-9 < 6.0 + moved / 6e6 || (count == 1 && maxTaps == 1))) return false;
+  if (force < 0 && (groups * kHalvesGroup * 4 > 5 * C || products * 6e-9 < 6.0 + moved / 6e6 || (count == 1 && maxTaps == 1))) return false;
   // Precise enough: the error of these kernels hardly grows with the number of terms (1.2e-7 of the result's norm at 600
   // terms, 1.3e-7 at 5000, 1.4e-7 at 10000), that of the other ones with the square root of those that one accumulator gets
   // and that are not zero (K split over workgroups or waves gives each fewer, and so does a border). With both operands half zeros,
