@@ -2788,7 +2788,7 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   // Fast enough: the products take about half the time (9 us less for 10^9 of them, on 98 layers of 100 at least 6; least with 2x2
   // windows and few output planes), the ranges and the split read the images twice and write them once (the bordered copy of the
   // other kernels, where there is a border, does a third of that less), the weights are read twice and written in both forms by
-  // one workgroup a row, and there is a launch more. Of 12000 random passes the ones taken need 0.4 to 1.07 of the time of the other
+  // one workgroup a row, and there is a launch more. Of 15000 random passes the ones taken need 0.4 to 1.11 of the time of the other
   // kernels, one in a thousand more than all of it; with 7.5 us in the place of 6 the worst needed 1.28 (N = 5, 471 -> 44 2x2
   // on 75x85: 92 us on the others, 117 on these). E.g. (us, others / these) N = 64, 256 -> 256 3x3 on 28x28 332 / 199; left: N = 58,
   // 223 -> 54 3x3 stride 2 on 64x26 59 / 84; N = 9, 361 -> 156 7x7 on 26x9 70 / 76. 1x1 windows use every element once
@@ -2800,9 +2800,10 @@ bool convHalves(THCState *state, int N, int C, int H, int W, int M, const float 
   // terms, 1.3e-7 at 5000, 1.4e-7 at 10000), that of the other ones with the square root of those that one accumulator gets
   // and that are not zero (K split over workgroups or waves gives each fewer, and so does a border). With both operands half zeros,
   // as behind a ReLU, it is 1.04e-7 at 600 terms, 1.07e-7 at 700, 1.2e-7 at 850 and 1.4e-7 at 1500 (normal operands 1.3e-7 at
-  // 560, 2.9e-7 at 2304).
+  // 560, 2.9e-7 at 2304). Over 7000 random passes, ordinary and masked, the error is at most 0.98 times that of the other kernels
+  // (1.03 and 1.015 on two of 13000 with K / 36 in the place of K / 24).
   const double inside = std::min(1.0, (double)H * W / minPositions);  // share of a window's taps on the image, about
-  if (force < 0 && (C * maxTaps * inside < 850 || oldTerms() * inside < 850 + C * maxTaps * inside / 36.0)) return false;
+  if (force < 0 && (C * maxTaps * inside < 850 || oldTerms() * inside < 850 + C * maxTaps * inside / 24.0)) return false;
   if (N * maxL > 0x7fffffffL / 2 || N * std::max(imgBytes, xImgBytes) > (1L << 31) - 1 - 4096) return false;
 
   // scratch: ranges and forms of images and rows, items, split weights, split images, partial tiles
